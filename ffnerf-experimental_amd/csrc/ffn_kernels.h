@@ -237,6 +237,8 @@ hipError_t launch_occ_bitfield(const uint32_t* occ, int G, uint32_t q_min, uint3
 // occupied; *use = 1 when at least half the blocks are empty, else 0
 hipError_t launch_occ_blocks(const uint32_t* bits, int R, uint32_t* blocks, uint32_t* use, hipStream_t st);
 hipError_t launch_march(const MarchArgs& a, bool emit, hipStream_t st);
+// whether launch_march takes the lattice walk (which does not use the block summary) for these arguments
+bool march_takes_lattice(const MarchArgs& a);
 // per-ray slots (ray r's counts[r] samples at slots + r * stride) -> the compacted order (offsets), with ray ids
 // (gate: as MarchArgs::gate)
 hipError_t launch_march_compact(const uint32_t* counts, const uint32_t* offsets, const float4* slots,

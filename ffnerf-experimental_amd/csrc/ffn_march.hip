@@ -13,7 +13,10 @@
 //   * The bitfield holds one bit per cell (x fastest, 32 cells per word):
 //     128^3 cells = 256 KiB, 256^3 = 2 MiB -- resident in each XCD's L2, so the
 //     DDA's bit lookups never reach HBM after the first touch.
-//   * One lane per ray.  Empty cells are skipped in one step: the first lattice
+//   * Two walks give the same samples bit for bit.  The lattice walk (k_march_lattice) gives a ray's lattice
+//     points to the wavefront's lanes and finds each one's cell by itself; the cell walk (k_march) gives a lane
+//     a ray and steps from cell to cell, for lattices much finer than the grid (launch_march).
+//   * The cell walk: one lane per ray.  Empty cells are skipped in one step: the first lattice
 //     index past the cell's exit is computed directly and corrected to the exact
 //     index the one-by-one walk of the specification reaches.
 //   * Empty 8^3 blocks are crossed in one step: a summary (one bit per block,
@@ -35,6 +38,9 @@
 //     scanned slots.  A chunked variant keeps a 16-byte state per
 //     ray so that the render can march, shade and composite a few samples per
 //     ray per round and retire rays whose transmittance fell below T_stop.
+#include <math.h>
+#include <stdlib.h>
+
 #include "ffn_device.h"
 #include "ffn_kernels.h"
 
@@ -394,6 +400,219 @@ __global__ __launch_bounds__(256) void k_march(MarchArgs a) {
   }
 }
 
+// The lattice walk.  The cell walk's state at lattice point k follows from t_k alone: on every axis it has left
+// exactly the cells whose exit time te(c) = (bmin + (c + (d > 0)) cell - o) / d is <= t_k, from the start cell on
+// (it steps while the smallest exit time is <= t_k, and an axis' exit times never decrease along it).  So a
+// lane takes a lattice point and finds its cell without walking: floor of the grid coordinate, which is that
+// cell unless the point lies within the rounding of a face, where the exit times themselves decide.
+//
+// What bounds it: vector instructions (about 45 per point and lane) and the latency of the bit load, which the
+// iterations of a ray overlap.  The cell walk serialises a ray's ~1.5 R cells on one lane: at 40,001 rays of the
+// ball scene (R = 256, dt = sqrt(3)/1024) it left most of the chip idle (1.13 ms a walk; this one 0.05 ms).
+// Both sides measured: march_takes_lattice.
+//
+// A wavefront sets up to 64 consecutive rays up at once, one per lane, and then takes them one at a time with
+// the ray's values in scalar registers.
+struct LatticeRay {
+  float o[3], d[3], t0, t1;
+  float p0[3], slope[3];  // grid coordinate at t0 and its slope per unit of t (the point's cell up to rounding)
+  float eps;              // the largest rounding of a grid coordinate or exit time, in cells (any axis)
+};
+
+// the walk's exit time of cell c on an axis (dir = 1 when the ray ascends it)
+__device__ __forceinline__ float cell_exit(float bmin, float cell, float o, float invd, int c, int dir) {
+  const float bound = bmin + (float)(c + dir) * cell;
+  return (bound - o) * invd;
+}
+
+// the walk's cell on one axis at lattice time tk, from the guess g; R or -1 once the walk has left the grid
+__device__ __forceinline__ int exact_axis_cell(const MarchArgs& a, int i, float o, float d, float t0, float tk, float pf) {
+  const int R = a.res;
+  const float inv = (float)R / (a.bmax[i] - a.bmin[i]), cell = (a.bmax[i] - a.bmin[i]) / (float)R;
+  const float p = o + t0 * d;
+  int c0 = (int)floorf((p - a.bmin[i]) * inv);
+  c0 = c0 < 0 ? 0 : (c0 > R - 1 ? R - 1 : c0);
+  if (d == 0.0f || d != d) return c0;  // the walk never steps along this axis
+  const float invd = 1.0f / d;
+  const int step = d > 0.0f ? 1 : -1, dir = d > 0.0f ? 1 : 0;
+  int g = (int)floorf(pf);
+  g = g < 0 ? 0 : (g > R - 1 ? R - 1 : g);
+  g = step > 0 ? (g > c0 ? g : c0) : (g < c0 ? g : c0);
+  while (g != c0 && !(cell_exit(a.bmin[i], cell, o, invd, g - step, dir) <= tk)) g -= step;
+  while (g >= 0 && g < R && cell_exit(a.bmin[i], cell, o, invd, g, dir) <= tk) g += step;
+  return g;
+}
+
+constexpr int LATTICE_UNROLL = 2;  // 64-point groups whose bit loads are in flight together
+// The most lattice points between a ray's entry and exit that the lattice walk takes; a longer ray (a direction
+// far from unit length, whose steps are tiny) is walked cell by cell by its own lane.
+constexpr float LATTICE_MAX_POINTS = 65536.0f;
+
+template <bool EMIT>
+__global__ __launch_bounds__(256) void k_march_lattice(MarchArgs a, uint32_t rays_per_wave) {
+  if (a.gate && *a.gate == 0u) return;  // the whole launch: every ray has stopped
+  const int lane = threadIdx.x & 63;
+  const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const uint64_t r_begin = wave * rays_per_wave;
+  if (r_begin >= a.num_rays) return;  // the same on every lane of the wavefront
+  const uint32_t n_here = (uint32_t)(a.num_rays - r_begin < rays_per_wave ? a.num_rays - r_begin : rays_per_wave);
+  const int R = a.res;
+
+  // lane j sets up ray r_begin + j
+  const uint32_t r_own = (uint32_t)r_begin + (uint32_t)lane;
+  const bool own = (uint32_t)lane < n_here;
+  LatticeRay L{};
+  MarchState st{0u, 0u, 0u, MARCH_FRESH};
+  bool have = false;
+  if (own) {
+    if (a.state) st = a.state[r_own];
+    if (!(st.flags & MARCH_DONE)) {
+      const float4 ro = a.rays[2 * (size_t)r_own], rd = a.rays[2 * (size_t)r_own + 1];
+      L.o[0] = ro.x; L.o[1] = ro.y; L.o[2] = ro.z;
+      L.d[0] = rd.x; L.d[1] = rd.y; L.d[2] = rd.z;
+      float ta, tb;
+      if (ray_aabb(L.o, L.d, a.bmin, a.bmax, ta, tb)) {
+        L.t0 = fmaxf(ta, a.t_near);
+        L.t1 = fminf(tb, a.t_far);
+        have = L.t1 > L.t0;
+      }
+      if (have) {
+        L.eps = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const float size = a.bmax[i] - a.bmin[i], inv = (float)R / size;
+          const float p = L.o[i] + L.t0 * L.d[i];
+          L.p0[i] = (p - a.bmin[i]) * inv;
+          L.slope[i] = L.d[i] * inv;
+          // With u = 2^-24, A the larger |bound| of the box, D = t1 |d| and s its extent, the coordinate
+          // p0 + tau slope is off by at most u (2 D + A + 9 s) inv cells from the real one at t_k and a face's
+          // exit time by u (3 D + A + 3 s) inv; eps doubles the sum (second-order terms, points a rounding
+          // outside the box).
+          const float A = fmaxf(fabsf(a.bmin[i]), fabsf(a.bmax[i]));
+          const float e = (5.0f * L.t1 * fabsf(L.d[i]) + 2.0f * A + 12.0f * size) * inv * (2.0f / 16777216.0f);
+          L.eps = fmaxf(L.eps, e);
+          if (!(e < 0.5f)) L.eps = 1.0f;  // (NaN included) every point takes the exact path
+        }
+      } else if (EMIT && a.state) {
+        st.flags = (st.flags & ~MARCH_FRESH) | MARCH_DONE;
+        a.state[r_own] = st;
+      }
+    }
+  }
+  if (st.flags & MARCH_FRESH) st.k = st.n = 0;
+  uint32_t emitted = 0;  // of this lane's ray
+  const bool by_cells = have && !(L.t1 - L.t0 <= LATTICE_MAX_POINTS * a.dt);
+  if (by_cells) {
+    float cell[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) cell[i] = (a.bmax[i] - a.bmin[i]) / (float)R;
+    RayWalk<EMIT> w;
+    if (w.start(a, r_own, cell)) {
+      while (!w.advance(a, cell, false)) {
+      }
+      w.finish_state(a, true);
+      emitted = w.emitted;
+    }
+    have = false;
+  }
+  const uint64_t below = (1ull << lane) - 1ull;
+
+  for (uint64_t todo = __ballot(have); todo != 0ull; todo &= todo - 1ull) {
+    const int j = (int)__builtin_ctzll(todo);
+    auto rl = [&](float x) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j)); };
+    const uint32_t r = (uint32_t)r_begin + (uint32_t)j;
+    float o[3], d[3], p0[3], slope[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      o[i] = rl(L.o[i]);
+      d[i] = rl(L.d[i]);
+      p0[i] = rl(L.p0[i]);
+      slope[i] = rl(L.slope[i]);
+    }
+    const float t0 = rl(L.t0), t1 = rl(L.t1), near = 0.5f - rl(L.eps);
+    const uint32_t n_before = (uint32_t)__builtin_amdgcn_readlane((int)st.n, j);
+    uint32_t kb = (uint32_t)__builtin_amdgcn_readlane((int)st.k, j);
+    // the call's samples: at most `chunk`, and max_steps over all calls
+    const uint32_t left = a.max_steps > n_before ? a.max_steps - n_before : 0u;
+    const uint32_t budget = left < a.chunk ? left : a.chunk;
+    uint64_t base = 0;
+    if (EMIT) base = a.slot_stride ? (uint64_t)r * a.slot_stride : (uint64_t)a.offsets[r];
+    uint32_t found = 0;
+    bool over = false;  // a sample past the budget: the ray pauses at it
+    for (;;) {
+      float tk[LATTICE_UNROLL];
+      uint32_t word[LATTICE_UNROLL], bit[LATTICE_UNROLL];
+      bool in[LATTICE_UNROLL];
+#pragma unroll
+      for (int u = 0; u < LATTICE_UNROLL; ++u) {
+        const float tau = ((float)(kb + 64u * u + (uint32_t)lane) + 0.5f) * a.dt;
+        tk[u] = t0 + tau;
+        in[u] = tk[u] < t1;
+        float pf[3];
+        int c[3];
+        bool exact = false;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          pf[i] = fmaf(tau, slope[i], p0[i]);
+          const float fl = floorf(pf[i]);
+          c[i] = (int)fl;
+          exact |= !(fabsf((pf[i] - fl) - 0.5f) < near);
+        }
+        // c outside the grid and not within the rounding of its faces: the walk has left it (or the point
+        // lies before the start cell, which the exact path decides)
+        exact |= (uint32_t)c[0] >= (uint32_t)R || (uint32_t)c[1] >= (uint32_t)R || (uint32_t)c[2] >= (uint32_t)R;
+        if (exact && in[u]) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i) c[i] = exact_axis_cell(a, i, o[i], d[i], t0, tk[u], pf[i]);
+        }
+        const bool inside = (uint32_t)c[0] < (uint32_t)R && (uint32_t)c[1] < (uint32_t)R && (uint32_t)c[2] < (uint32_t)R;
+        const uint32_t bi = (uint32_t)c[0] + (uint32_t)R * ((uint32_t)c[1] + (uint32_t)R * (uint32_t)c[2]);
+        bit[u] = bi & 31u;
+        word[u] = (in[u] && inside) ? a.bits[bi >> 5] : 0u;
+      }
+      bool end = false;
+#pragma unroll
+      for (int u = 0; u < LATTICE_UNROLL; ++u) {
+        const bool occ = (word[u] >> bit[u]) & 1u;
+        const uint64_t m = __ballot(occ);
+        if (m != 0ull && !over) {
+          const uint32_t idx = found + (uint32_t)__popcll(m & below);
+          const uint32_t cnt = (uint32_t)__popcll(m);
+          if (EMIT && occ && idx < budget) {
+            const uint64_t slot = base + idx;
+            if (slot < a.capacity) {
+              a.samples[slot] = make_float4(o[0] + tk[u] * d[0], o[1] + tk[u] * d[1], o[2] + tk[u] * d[2], tk[u]);
+              if (a.ray_ids) a.ray_ids[slot] = r;
+            }
+          }
+          if (found + cnt > budget) {
+            // the first sample past the budget is where the next call starts
+            const uint64_t past = __ballot(occ && idx == budget);
+            kb = kb + 64u * u + (uint32_t)__builtin_ctzll(past);
+            found = budget;
+            over = true;
+          } else {
+            found += cnt;
+          }
+        }
+        end |= __ballot(in[u]) != ~0ull;
+      }
+      if (over || end) break;
+      kb += 64u * LATTICE_UNROLL;
+    }
+    if (lane == j) {
+      emitted = found;
+      if (EMIT && a.state) {
+        st.k = kb;
+        st.n = n_before + found;
+        st.flags = (st.flags & ~MARCH_FRESH) | ((!over || st.n >= a.max_steps) ? MARCH_DONE : 0u);
+        a.state[r_own] = st;
+      }
+    }
+  }
+  if (own && (!EMIT || a.slot_stride)) a.counts[r_own] = emitted;
+}
+
 // One wavefront per ray at a time: the ray's samples from its slots to its compacted range, 64 at a time
 __global__ __launch_bounds__(256) void k_march_compact(const uint32_t* __restrict__ counts,
                                                        const uint32_t* __restrict__ offsets,
@@ -621,8 +840,40 @@ hipError_t launch_occ_blocks(const uint32_t* bits, int R, uint32_t* blocks, uint
   return hipGetLastError();
 }
 
+// The rule between the two walks.  The lattice walk costs rays x lattice points, the cell walk rays x cells, but
+// with few rays its serial walk per lane costs the same however few they are.  ffn_march (count, scan, emit) in
+// us, lattice / cells, K points along the box diagonal, the ball and the shell field:
+//   rays 1000, R 256:    K 1024 63 / 1709, 64 / 1898;      K 4096 166 / 2445, 164 / 3212
+//   rays 40001, R 256:   K 1024 114 / 2118, 117 / 2227;    K 4096 297 / 3069, 297 / 3850
+//   rays 2^18, R 256:    K 1024 480 / 1924, 481 / 2160;    K 4096 1458 / 2795, 1467 / 3609
+//   rays 2^20, R 256:    K 1024 1444 / 2716, 1460 / 3468;  K 4096 4578 / 4245, 4602 / 6175
+//   rays 2^20, R 128:    K 2048 2167 / 2320, 2172 / 3182;  K 4096 3883 / 3459, 3877 / 4988
+// so the line lies at 16 R points for 2^20 rays and moves up in proportion for fewer.  FFN_MARCH_LATTICE=0 keeps
+// the cell walk.
+bool march_takes_lattice(const MarchArgs& a) {
+  const char* env = getenv("FFN_MARCH_LATTICE");
+  if (env && env[0] == '0') return false;
+  double diag2 = 0.0;
+  for (int i = 0; i < 3; ++i) diag2 += ((double)a.bmax[i] - a.bmin[i]) * ((double)a.bmax[i] - a.bmin[i]);
+  const double points = sqrt(diag2) / (double)a.dt;
+  const double fewer = a.num_rays < (1u << 20) ? (double)(1u << 20) / a.num_rays : 1.0;
+  return points <= 16.0 * a.res * fewer;
+}
+
 hipError_t launch_march(const MarchArgs& a, bool emit, hipStream_t st) {
   if (a.num_rays == 0) return hipSuccess;
+  if (march_takes_lattice(a)) {
+    // rays a wavefront sets up at once: as many as leave 8192 wavefronts (8 per SIMD), at least 4
+    uint32_t rpw = 64;
+    while (rpw > 4 && (a.num_rays + rpw - 1) / rpw < 8192u) rpw >>= 1;
+    const uint64_t waves = ((uint64_t)a.num_rays + rpw - 1) / rpw;
+    const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
+    if (emit)
+      hipLaunchKernelGGL(k_march_lattice<true>, grid, block, 0, st, a, rpw);
+    else
+      hipLaunchKernelGGL(k_march_lattice<false>, grid, block, 0, st, a, rpw);
+    return hipGetLastError();
+  }
   const uint64_t waves = (a.num_rays + MARCH_RPW - 1) / MARCH_RPW;
   const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
   if (emit)
