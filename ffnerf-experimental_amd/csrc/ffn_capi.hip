@@ -173,22 +173,23 @@ hipError_t build_dense_levels(Handle* h, const void* table, ffn::DenseLevels* dl
   return ffn::launch_hash_densify(c, table, *dl, st);
 }
 
-// size the bucketed-scatter scratch for n samples and fill the views
-hipError_t ensure_bins(Handle* h, int64_t n, ffn::BinPlan* plan, ffn::BinScratch* s) {
+// size the bucketed-scatter scratch for n samples (n_typical: see plan_bins) and fill the views
+hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* plan, ffn::BinScratch* s) {
   bool from_env = false;
   const size_t budget = bin_budget_bytes(&from_env);
   const size_t pair_bytes = 2 + 4 * (size_t)h->dc.F;
-  *plan = ffn::plan_bins(h->dc, n, budget);
+  *plan = ffn::plan_bins(h->dc, n, n_typical, budget, h->n_cu);
   if (!from_env && !growth_fits_free(h->bin_pairs, pair_bytes * (size_t)plan->max_pairs)) {
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) == hipSuccess) {
       const size_t cap = h->bin_pairs.bytes + fr / 2;
-      *plan = ffn::plan_bins(h->dc, n, cap < ((size_t)64 << 20) ? ((size_t)64 << 20) : cap);
+      *plan = ffn::plan_bins(h->dc, n, n_typical, cap < ((size_t)64 << 20) ? ((size_t)64 << 20) : cap, h->n_cu);
     }
   }
   hipError_t e;
   if ((e = h->bin_meta.ensure(sizeof(uint32_t) * (size_t)plan->meta_elems)) != hipSuccess) return e;
-  if ((e = h->bin_meta_t.ensure(sizeof(uint32_t) * (size_t)plan->meta_elems)) != hipSuccess) return e;
+  if (plan->transpose && (e = h->bin_meta_t.ensure(sizeof(uint32_t) * (size_t)plan->meta_elems)) != hipSuccess)
+    return e;
   if ((e = h->bin_pairs.ensure((2 + 4 * (size_t)h->dc.F) * (size_t)plan->max_pairs)) != hipSuccess) return e;
   if ((e = h->bin_max.ensure(sizeof(float) * (size_t)plan->levels_per_group * plan->nblk)) != hipSuccess) return e;
   s->meta = (uint32_t*)h->bin_meta.p;
@@ -584,7 +585,7 @@ int ffn_hash_encode_bwd(void* handle, const float* x, const float* g, int64_t n,
   UseMark um{h, (hipStream_t)stream};
   ffn::BinPlan plan;
   ffn::BinScratch bs;
-  FFN_HIP(ensure_bins(h, n, &plan, &bs));
+  FFN_HIP(ensure_bins(h, n, n, &plan, &bs));
   // the scatter reads one level per pass: the caller's sample-major rows are transposed to level-major
   // first (the passes would otherwise fetch every row once per level for F floats of it)
   const hipStream_t st = (hipStream_t)stream;
@@ -660,7 +661,7 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   }
   ffn::BinPlan plan{};
   ffn::BinScratch bs{};
-  if (train) FFN_HIP(ensure_bins(h, N, &plan, &bs));
+  if (train) FFN_HIP(ensure_bins(h, N, N, &plan, &bs));
   const ffn::FeatLayout feat = ffn::level_major(N, h->dc.F);
   const ffn::PosSrc src{nullptr, (const float4*)rays, nullptr, log2S};
   float* Ts = (float*)h->Ts.p;
@@ -818,6 +819,9 @@ int check_march(Handle* h, const void* rays, const uint32_t* bits, const ffn_mar
   if (mp->flags & ~FFN_RENDER_NO_WAIT) return fail(-1, "unknown march flags 0x%x", mp->flags);
   return 0;
 }
+
+// samples per ray the marched step's scatter is planned for (the ball scene of the benchmark marches 22)
+constexpr int64_t MARCH_TYPICAL_SAMPLES = 16;
 
 ffn::MarchArgs march_args(Handle* h, const void* rays, uint32_t num_rays, const uint32_t* bits,
                           const ffn_march_params* mp) {
@@ -1123,7 +1127,7 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
     StageTimer tm(h, 3, st);
     ffn::BinPlan plan{};
     ffn::BinScratch bs{};
-    FFN_HIP(ensure_bins(h, n > 0 ? n : 1, &plan, &bs));
+    FFN_HIP(ensure_bins(h, n > 0 ? n : 1, MARCH_TYPICAL_SAMPLES * num_rays, &plan, &bs));
     ffn::BinApply ap{};
     ap.dst = P.table;
     ap.dst_f16 = h->dc.table_f16;

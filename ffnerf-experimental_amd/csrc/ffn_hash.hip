@@ -542,7 +542,8 @@ __global__ __launch_bounds__(emit_nt(F)) void k_bin_emit(DevCfg c, PosSrc src, i
   uint16_t* st_idx = reinterpret_cast<uint16_t*>(st_val + (size_t)grp.np * F);  // [np]
   const int tid = threadIdx.x, lane = tid & 63;
   for (int j = tid; j < nbl; j += NT) lcnt[j] = 0u;
-  const uint32_t be_mask = (1u << grp.log2_be) - 1u;
+  const int log2_be = grp.log2_be[li];
+  const uint32_t be_mask = (1u << log2_be) - 1u;
   if (n_dev) {
     const int64_t nd = (int64_t)*n_dev;
     n = nd < n ? nd : n;
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(emit_nt(F)) void k_bin_emit(DevCfg c, PosSrc src, i
 #pragma unroll
         for (int f = 0; f < F; ++f) bound = fmaxf(bound, fabsf(es.v[cc][f]));
         ent[cc] = corner_entry(lc, cc, l, c.mask[l]);
-        rank[cc] = atomicAdd(&cur[ent[cc] >> grp.log2_be], 1u);
+        rank[cc] = atomicAdd(&cur[ent[cc] >> log2_be], 1u);
       }
     }
     __syncthreads();
@@ -626,7 +627,7 @@ __global__ __launch_bounds__(emit_nt(F)) void k_bin_emit(DevCfg c, PosSrc src, i
     if (es.head) {
 #pragma unroll
       for (int cc = 0; cc < 8; ++cc) {
-        const uint32_t slot = loff[ent[cc] >> grp.log2_be] + rank[cc];
+        const uint32_t slot = loff[ent[cc] >> log2_be] + rank[cc];
         st_idx[slot] = (uint16_t)(ent[cc] & be_mask);
         reinterpret_cast<V*>(st_val)[slot] = FVec<F>::pack(es.v[cc]);
       }
@@ -687,20 +688,38 @@ __global__ __launch_bounds__(256) void k_bin_meta_transpose(const uint32_t* __re
   }
 }
 
+// the update of one table value from its summed gradient
+template <int MODE>
+__device__ __forceinline__ void apply1(const BinApply& ap, float gsum, float& p, float& m, float& v) {
+  if (MODE == BIN_GRAD || MODE == BIN_SGD) {
+    p = p + gsum;
+  } else {
+    m = fmaf(1.0f - ap.beta1, gsum, ap.beta1 * m);
+    v = fmaf(1.0f - ap.beta2, gsum * gsum, ap.beta2 * v);
+    p = p - ap.lr_t * (m / (sqrtf(v) + ap.eps));
+  }
+}
+
 // One block per bucket: sum its pairs in 64-bit fixed point in LDS, then apply the mode's update to the
 // bucket's slice of the table.  The bucket's pairs are one run in each round's slots (its row of the
-// bucket-major run table gives offset and length); a first pass over the row counts them (for the
-// fixed-point scale), the second walks SEG rounds per wavefront at a time with every lane on one block of 8
-// pairs: 16 rounds (a block's run found by selects over the 16 running ends in scalars) or 64 (a binary
-// search over the lanes' running ends).  Zero pairs (the run padding) are skipped.
-template <int F, int MODE, int SEG>
-__global__ __launch_bounds__(1024) void k_bin_reduce(DevCfg c, BinGroup grp, const uint32_t* __restrict__ meta,
-                                                     const uint4* __restrict__ pbuf,
-                                                     const float* __restrict__ cmax, BinApply ap,
-                                                     const uint32_t* __restrict__ n_dev) {
-  extern __shared__ unsigned long long acc[];
-  __shared__ float wmax[16];
-  __shared__ uint32_t wtot[16];
+// run table gives offset and length); a first pass over the row counts them (for the fixed-point scale), the
+// second walks up to 64 rounds per wavefront at a time (`seg`: fewer where the rounds would not reach every
+// wavefront of the block) with every lane on one block of 8 pairs, its run found by a binary search over the
+// lanes' running ends.  Zero pairs (the run padding) are skipped.
+// The update takes four values per lane with 16-byte accesses, two groups in flight (ap.vec4: the buffers are
+// aligned for it).  One value per lane and trip, with a trip's loads waiting for the last trip's stores, made the
+// update the larger part of the kernel where the pairs are few: with the smaller buckets of small batches
+// (plan_bins), 512 rays x 64 samples of the 16 x 2^19 table with Adam 100 -> 76 us (the table and its moments are
+// 403 MB: 5.3 TB/s), 16 x 2^14 entries 47 -> 8.5 us, F = 4 with the reference's SGD 94 -> 33 us, and the 2^22-entry
+// binary16 gradient table with 2^22 points 2391 -> 2229 us (bound there by its pair reads: runs of two pair blocks).
+template <int F, int MODE, int NT>
+__global__ __launch_bounds__(NT) void k_bin_reduce(DevCfg c, BinGroup grp, const uint32_t* __restrict__ meta,
+                                                   const uint4* __restrict__ pbuf, const float* __restrict__ cmax,
+                                                   BinApply ap, const uint32_t* __restrict__ n_dev, int seg) {
+  constexpr int NW = NT / 64;
+  extern __shared__ __align__(16) unsigned long long acc[];
+  __shared__ float wmax[NW];
+  __shared__ uint32_t wtot[NW];
   // bucket, relative to the group, finest levels first: their buckets hold the most pairs, and the lighter
   // coarse-level blocks then fill the last wave of blocks (scatter 7.01 -> 6.91 ms at the benchmark shape)
   const int j = (int)gridDim.x - 1 - (int)blockIdx.x;
@@ -708,21 +727,23 @@ __global__ __launch_bounds__(1024) void k_bin_reduce(DevCfg c, BinGroup grp, con
   while (li + 1 < grp.n_levels && j >= grp.bucket_rel[li + 1]) ++li;
   const int l = grp.level0 + li;
   const int jb = j - grp.bucket_rel[li];
-  const int be = 1 << grp.log2_be;
-  const uint32_t entry_lo = (uint32_t)jb << grp.log2_be;
+  const int be = 1 << grp.log2_be[li];
+  const uint32_t entry_lo = (uint32_t)jb << grp.log2_be[li];
   const uint32_t level_T = c.mask[l] + 1u;
   const int count = (int)((level_T - entry_lo) < (uint32_t)be ? (level_T - entry_lo) : (uint32_t)be);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nr = grp.n_rounds;
   const int nr_use = rounds_used(nr, n_dev, emit_nt(F));  // rounds with samples
   if (nr_use == 0) return;  // no samples: nothing is applied (the same for the whole block)
-  for (int e = tid; e < count * F; e += 1024) acc[e] = 0ull;
-  const uint32_t* mrow = meta + ((int64_t)li * grp.meta_stride + jb) * nr;  // bucket-major: round rr at mrow[rr]
+  for (int e = tid; e < count * F; e += NT) acc[e] = 0ull;
+  // the bucket's row of the run table: round rr at mrow[rr * round_stride]
+  const uint32_t* mrow = meta + (int64_t)li * grp.meta_stride * nr + (int64_t)jb * grp.bucket_stride;
+  const int64_t rs = grp.round_stride;
   // bound on every |value| of the level (the largest of its chunks' bounds) and the bucket's pair count
   float mxl = 0.0f;
-  for (int ch = tid; ch < grp.nblk; ch += 1024) mxl = fmaxf(mxl, cmax[(int64_t)li * grp.nblk + ch]);
+  for (int ch = tid; ch < grp.nblk; ch += NT) mxl = fmaxf(mxl, cmax[(int64_t)li * grp.nblk + ch]);
   uint32_t cnt = 0;
-  for (int rr = tid; rr < nr_use; rr += 1024) cnt += mrow[rr] & 0xFFFFu;
+  for (int rr = tid; rr < nr_use; rr += NT) cnt += mrow[rr * rs] & 0xFFFFu;
   mxl = wave_max_nonneg(mxl);
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) cnt += __shfl_xor(cnt, d);
@@ -734,7 +755,7 @@ __global__ __launch_bounds__(1024) void k_bin_reduce(DevCfg c, BinGroup grp, con
   float mx = 0.0f;
   uint32_t pairs = 0;
 #pragma unroll
-  for (int w = 0; w < 16; ++w) {
+  for (int w = 0; w < NW; ++w) {
     mx = fmaxf(mx, wmax[w]);
     pairs += wtot[w];
   }
@@ -772,61 +793,29 @@ __global__ __launch_bounds__(1024) void k_bin_reduce(DevCfg c, BinGroup grp, con
   if (mx > 0.0f) {
     const int64_t bpr = grp.np / PAD_RUN;  // pair blocks per round
     const int64_t blk_lvl = (int64_t)li * nr * bpr;
-    for (int r0 = wave * SEG; r0 < nr_use; r0 += 16 * SEG) {
-      if constexpr (SEG == 16) {
-        // lanes 0..SEG-1 hold rounds r0 + lane: run offset and block count, then the blocks' running ends
-        uint32_t m = 0;
-        if (lane < SEG && r0 + lane < nr_use) m = mrow[r0 + lane];
-        uint32_t incl = lane < SEG ? (m & 0xFFFFu) / PAD_RUN : 0u;
+    for (int r0 = wave * seg; r0 < nr_use; r0 += NW * seg) {
+      // lane t holds round r0 + t, and the wavefront's blocks are dealt over its lanes in order; block q
+      // belongs to the first round whose running end exceeds q, found by a binary search over the lanes'
+      // running ends.  Every lane runs every search step (the loop count is the same for the whole
+      // wavefront), so the shuffles never read an inactive lane.
+      uint32_t m = 0;
+      if (lane < seg && r0 + lane < nr_use) m = mrow[(r0 + lane) * rs];
+      const uint32_t nb = (m & 0xFFFFu) / PAD_RUN;
+      const uint32_t incl = wave_incl_sum(nb);
+      const uint32_t excl = incl - nb;
+      const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+      for (uint32_t q0 = 0; q0 < total; q0 += 64) {
+        const uint32_t q = q0 + (uint32_t)lane;
+        int t = 0;
 #pragma unroll
-        for (int d = 1; d < SEG; d <<= 1) {
-          const uint32_t o = __shfl_up(incl, d);
-          if (lane >= d) incl += o;
+        for (int step = 32; step >= 1; step >>= 1) {
+          const uint32_t v = (uint32_t)__shfl((int)incl, t + step - 1);
+          if (v <= q) t += step;
         }
-        uint32_t ends[SEG], offs[SEG];
-#pragma unroll
-        for (int t = 0; t < SEG; ++t) {
-          ends[t] = __builtin_amdgcn_readlane(incl, t);
-          offs[t] = __builtin_amdgcn_readlane(m >> 16, t);
-        }
-        for (uint32_t q = (uint32_t)lane; q < ends[SEG - 1]; q += 64) {
-          // the run holding block q: the last round whose running start is <= q
-          uint32_t qb = 0, off = offs[0];
-          int sg = 0;
-#pragma unroll
-          for (int t = 1; t < SEG; ++t) {
-            if (q >= ends[t - 1]) {
-              qb = ends[t - 1];
-              off = offs[t];
-              sg = t;
-            }
-          }
-          add_block(pbuf + (blk_lvl + (int64_t)(r0 + sg) * bpr + off / PAD_RUN + (q - qb)) * pair_block_words(F));
-        }
-      } else {
-        // lane t holds round r0 + t, and the wavefront's blocks are dealt over its lanes in order; block q
-        // belongs to the first round whose running end exceeds q, found by a binary search over the lanes'
-        // running ends.  Every lane runs every search step (the loop count is the same for the whole
-        // wavefront), so the shuffles never read an inactive lane.
-        uint32_t m = 0;
-        if (r0 + lane < nr_use) m = mrow[r0 + lane];
-        const uint32_t nb = (m & 0xFFFFu) / PAD_RUN;
-        const uint32_t incl = wave_incl_sum(nb);
-        const uint32_t excl = incl - nb;
-        const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-        for (uint32_t q0 = 0; q0 < total; q0 += 64) {
-          const uint32_t q = q0 + (uint32_t)lane;
-          int t = 0;
-#pragma unroll
-          for (int step = 32; step >= 1; step >>= 1) {
-            const uint32_t v = (uint32_t)__shfl((int)incl, t + step - 1);
-            if (v <= q) t += step;
-          }
-          const uint32_t qb = (uint32_t)__shfl((int)excl, t);
-          const uint32_t off = (uint32_t)__shfl((int)(m >> 16), t);
-          if (q < total)
-            add_block(pbuf + (blk_lvl + (int64_t)(r0 + t) * bpr + off / PAD_RUN + (q - qb)) * pair_block_words(F));
-        }
+        const uint32_t qb = (uint32_t)__shfl((int)excl, t);
+        const uint32_t off = (uint32_t)__shfl((int)(m >> 16), t);
+        if (q < total)
+          add_block(pbuf + (blk_lvl + (int64_t)(r0 + t) * bpr + off / PAD_RUN + (q - qb)) * pair_block_words(F));
       }
     }
   }
@@ -835,23 +824,75 @@ __global__ __launch_bounds__(1024) void k_bin_reduce(DevCfg c, BinGroup grp, con
   const int64_t base = ((int64_t)c.offset[l] + entry_lo) * F;
   float* dst32 = static_cast<float*>(ap.dst);
   _Float16* dst16 = static_cast<_Float16*>(ap.dst);
-  for (int e = tid; e < count * F; e += 1024) {
+  auto sum = [&](unsigned long long a) { return (float)((double)(long long)a * inv); };
+  if (ap.vec4 && ((base | (int64_t)(count * F)) & 3) == 0) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    typedef unsigned long long u2 __attribute__((ext_vector_type(2)));
+    const int n4 = count * F / 4;
+    f4* d32 = reinterpret_cast<f4*>(dst32 + base);
+    h4* d16 = reinterpret_cast<h4*>(dst16 + base);
+    f4* m4 = MODE == BIN_ADAM ? reinterpret_cast<f4*>(ap.m + base) : nullptr;
+    f4* v4 = MODE == BIN_ADAM ? reinterpret_cast<f4*>(ap.v + base) : nullptr;
+    constexpr int U = 2;
+    for (int e0 = tid; e0 < n4; e0 += U * NT) {
+      f4 p[U], m[U], v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * NT;
+        if (e >= n4) break;
+        if (ap.dst_f16) p[u] = __builtin_convertvector(d16[e], f4);
+        else p[u] = d32[e];
+        if (MODE == BIN_ADAM) {
+          m[u] = m4[e];
+          v[u] = v4[e];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * NT;
+        if (e >= n4) break;
+        const u2 a0 = reinterpret_cast<const u2*>(acc)[2 * e], a1 = reinterpret_cast<const u2*>(acc)[2 * e + 1];
+        const f4 g = {sum(a0[0]), sum(a0[1]), sum(a1[0]), sum(a1[1])};
+        if (MODE == BIN_ADAM && ap.g_tap) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) ap.g_tap[base + 4 * e + q] = g[q];
+        }
+        f4 pp = p[u], mm = m[u], vv = v[u];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float a = pp[q], b = mm[q], cv = vv[q];
+          apply1<MODE>(ap, g[q], a, b, cv);
+          pp[q] = a;
+          mm[q] = b;
+          vv[q] = cv;
+        }
+        if (MODE == BIN_ADAM) {
+          m4[e] = mm;
+          v4[e] = vv;
+        }
+        if (ap.dst_f16) d16[e] = __builtin_convertvector(pp, h4);  // to nearest even, once per entry and step
+        else d32[e] = pp;
+      }
+    }
+    return;
+  }
+  for (int e = tid; e < count * F; e += NT) {
     const int64_t gi = base + e;
-    const float gsum = (float)((double)(long long)acc[e] * inv);
-    float pp = ap.dst_f16 ? (float)dst16[gi] : dst32[gi];
-    if (MODE == BIN_GRAD || MODE == BIN_SGD) {
-      pp = pp + gsum;
-    } else {
+    const float gsum = sum(acc[e]);
+    float pp = ap.dst_f16 ? (float)dst16[gi] : dst32[gi], mm = 0.0f, vv = 0.0f;
+    if (MODE == BIN_ADAM) {
       if (ap.g_tap) ap.g_tap[gi] = gsum;
-      float mm = ap.m[gi], vv = ap.v[gi];
-      float mi = fmaf(1.0f - ap.beta1, gsum, ap.beta1 * mm);
-      float vi = fmaf(1.0f - ap.beta2, gsum * gsum, ap.beta2 * vv);
-      pp = pp - ap.lr_t * (mi / (sqrtf(vi) + ap.eps));
-      ap.m[gi] = mi;
-      ap.v[gi] = vi;
+      mm = ap.m[gi];
+      vv = ap.v[gi];
+    }
+    apply1<MODE>(ap, gsum, pp, mm, vv);
+    if (MODE == BIN_ADAM) {
+      ap.m[gi] = mm;
+      ap.v[gi] = vv;
     }
     if (ap.dst_f16)
-      dst16[gi] = (_Float16)pp;  // round to nearest even, once per entry and step
+      dst16[gi] = (_Float16)pp;
     else
       dst32[gi] = pp;
   }
@@ -1020,32 +1061,60 @@ hipError_t launch_hash_densify(const DevCfg& c, const void* table, const DenseLe
   return launch_densify_t(c, static_cast<const float*>(table), dl, st);
 }
 
-BinPlan plan_bins(const DevCfg& c, int64_t n, size_t pair_budget_bytes) {
+BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_budget_bytes, int n_cu) {
   BinPlan p{};
-  // int64 LDS accumulator of one bucket: 2^log2_be * F * 8 bytes = 64 KiB (two reduce blocks per CU), or
-  // 128 KiB (one) when a level would otherwise have more than 64 buckets.  An emit round's pairs spread
-  // over the buckets, and every run costs its two edge sectors twice (the neighbouring buckets' blocks
-  // read them too) plus its padding: at the benchmark shape 64 buckets per level measured emit 4.95 and
-  // reduce 2.81 ms against 5.12 and 3.19 ms with 128.  Small tables keep the small buckets, so that the
-  // reduction still has blocks for every CU.
-  p.log2_be = c.F == 4 ? 11 : (c.F == 2 ? 12 : 13);
-  {
-    uint32_t max_T = 0;
-    for (int l = 0; l < c.L; ++l) max_T = c.mask[l] + 1 > max_T ? c.mask[l] + 1 : max_T;
-    if ((max_T >> p.log2_be) > 64u) ++p.log2_be;
-  }
   const int rs = emit_nt(c.F);  // samples per emit round
   p.n_rounds = (int)((n + rs - 1) / rs);
-  // rounds per emit block: 32 where a level still has at least 256 blocks (a block's set-up, first load and
-  // last copy-out are paid once per 32 rounds: at the benchmark shape the scatter took 7.15 ms with 8 rounds,
-  // 7.04 with 16 and 7.02 with 32), fewer for small batches so that every CU gets blocks
-  int rpb = 32;
-  while (rpb > 8 && (p.n_rounds + rpb - 1) / rpb < 256) rpb >>= 1;
-  p.chunk = rpb * rs;
+  // Bucket sizes.  A bucket's int64 LDS accumulator is 2^log2_be * F * 8 bytes.
+  // Large batches: at most 64 KiB (two reduce blocks per CU), or 128 KiB (one) when a level would otherwise have
+  // more than 64 buckets.  An emit round's pairs spread over the buckets, and every run costs its two edge
+  // sectors twice (the neighbouring buckets' blocks read them too) plus its padding: at the benchmark shape
+  // 64 buckets per level measured emit 4.95 and reduce 2.81 ms against 5.12 and 3.19 ms with 128.
+  // Small batches (fewer than 512 rounds; at 625 the large buckets measured emit 257 and reduce 204 us against 283
+  // and 227): the table's update, not the pairs, is most of the reduce's work, so
+  // a level gets 64 to 256 buckets, of at most 2048 entries (4096 at F = 1) where that many suffice, and several
+  // blocks share a CU.
+  int max_be = c.F == 4 ? 11 : (c.F == 2 ? 12 : 13);
+  uint32_t max_T = 0;
+  for (int l = 0; l < c.L; ++l) max_T = c.mask[l] + 1 > max_T ? c.mask[l] + 1 : max_T;
+  if ((max_T >> max_be) > 64u) ++max_be;
+  const bool small = (n_typical + rs - 1) / rs < 512;
+  for (int l = 0; l < c.L; ++l) {
+    int lg = max_be;
+    if (small) {
+      lg = c.F == 1 ? 12 : (c.F == 2 ? 11 : 10);  // 32 KiB
+      while (lg > 6 && ((c.mask[l] + 1u) >> lg) < 64u) --lg;
+      while (lg < max_be && ((c.mask[l] + 1u) >> lg) > (c.F == 4 ? 512u : 256u)) ++lg;  // the emit's stage pads every bucket's run
+      lg = lg < max_be ? lg : max_be;
+    }
+    p.log2_be[l] = lg;
+    p.max_log2_be = lg > p.max_log2_be ? lg : p.max_log2_be;
+  }
+  // Rounds per emit block, out of 1, 2, 4 .. 32: the blocks run one per CU (their stage takes more than half a CU's
+  // LDS), so the pass takes ceil(blocks / CUs) turns of a block's rounds and about one round's time of set-up,
+  // first load and last copy-out.  (At the benchmark shape the scatter took 7.15 ms with 8 rounds, 7.04 with 16
+  // and 7.02 with 32; 32 rounds in all over 16 levels 13.5 us with 2 and 31 with 8.)
+  {
+    const int64_t cus = n_cu > 0 ? n_cu : 256;
+    int best = 32;
+    int64_t best_cost = INT64_MAX;
+    for (int rpb = 32; rpb >= 1; rpb >>= 1) {
+      const int64_t blocks = (int64_t)c.L * ((p.n_rounds + rpb - 1) / rpb);
+      const int64_t cost = (blocks + cus - 1) / cus * (rpb + 1);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = rpb;
+      }
+    }
+    p.chunk = best * rs;
+  }
   p.nblk = (int)((n + p.chunk - 1) / p.chunk);
+  // The reduce reads a bucket's row of the run table as a strided column while the rounds are few; from 512 rounds
+  // on, a column's sectors cost more than the transpose's launch.
+  p.transpose = p.n_rounds > 512;
   int max_nbl = 0;
   for (int l = 0; l < c.L; ++l) {
-    const int nbl = (int)(((int64_t)c.mask[l] + 1 + (1 << p.log2_be) - 1) >> p.log2_be);
+    const int nbl = (int)(((int64_t)c.mask[l] + (1 << p.log2_be[l])) >> p.log2_be[l]);
     if (nbl > max_nbl) max_nbl = nbl;
   }
   // every round of a level has its own np pair slots (its pairs and at most PAD_RUN - 1 padding pairs per
@@ -1061,7 +1130,7 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, size_t pair_budget_bytes) {
   for (int g0 = 0; g0 < c.L; g0 += lg) {
     int nb = 0;
     for (int l = g0; l < g0 + lg && l < c.L; ++l)
-      nb += (int)(((int64_t)c.mask[l] + 1 + (1 << p.log2_be) - 1) >> p.log2_be);
+      nb += (int)(((int64_t)c.mask[l] + (1 << p.log2_be[l])) >> p.log2_be[l]);
     if (nb > max_buckets) max_buckets = nb;
   }
   p.max_buckets = max_buckets;
@@ -1072,8 +1141,12 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, size_t pair_budget_bytes) {
 }
 
 bool scatter_supported(const DevCfg& c) {
-  const BinPlan p = plan_bins(c, 1, (size_t)1 << 30);  // the stage size depends on the table, not on n
-  return p.np <= 65535 && emit_lds_bytes(p.max_nbl, c.F) <= 160 * 1024;
+  // the stage size depends on the table and on whether the batch is small
+  for (const int64_t n : {(int64_t)1, (int64_t)1 << 30}) {
+    const BinPlan p = plan_bins(c, 1, n, (size_t)1 << 30, 256);
+    if (p.np > 65535 || emit_lds_bytes(p.max_nbl, c.F) > 160 * 1024) return false;
+  }
+  return true;
 }
 
 hipError_t launch_hash_bwd(const DevCfg& c, const PosSrc& src, int64_t n, const float* g, const FeatLayout& lay,
@@ -1083,12 +1156,13 @@ hipError_t launch_hash_bwd(const DevCfg& c, const PosSrc& src, int64_t n, const 
   // run offsets and lengths are 16-bit, and a round's stage must fit in LDS
   const size_t lds_emit = emit_lds_bytes(plan.max_nbl, c.F);
   if (plan.np > 65535 || lds_emit > 160 * 1024) return hipErrorInvalidConfiguration;  // table too large
-  const size_t lds_acc = sizeof(unsigned long long) * ((size_t)1 << plan.log2_be) * (size_t)c.F;
+  const size_t lds_acc = sizeof(unsigned long long) * ((size_t)1 << plan.max_log2_be) * (size_t)c.F;
+  BinApply apv = ap;
+  apv.vec4 = (((uintptr_t)ap.dst & (ap.dst_f16 ? 7 : 15)) | (((uintptr_t)ap.m | (uintptr_t)ap.v) & 15)) == 0;
   for (int g0 = 0; g0 < c.L; g0 += plan.levels_per_group) {
     BinGroup grp{};
     grp.level0 = g0;
     grp.n_levels = (g0 + plan.levels_per_group <= c.L) ? plan.levels_per_group : c.L - g0;
-    grp.log2_be = plan.log2_be;
     grp.chunk = plan.chunk;
     grp.nblk = plan.nblk;
     grp.n_rounds = plan.n_rounds;
@@ -1097,20 +1171,27 @@ hipError_t launch_hash_bwd(const DevCfg& c, const PosSrc& src, int64_t n, const 
     int rel = 0;
     for (int li = 0; li < grp.n_levels; ++li) {
       const int l = g0 + li;
-      grp.nbl[li] = (int)(((int64_t)c.mask[l] + 1 + (1 << plan.log2_be) - 1) >> plan.log2_be);
+      grp.log2_be[li] = plan.log2_be[l];
+      grp.nbl[li] = (int)(((int64_t)c.mask[l] + (1 << plan.log2_be[l])) >> plan.log2_be[l]);
       grp.bucket_rel[li] = rel;
       rel += grp.nbl[li];
     }
     grp.bucket_rel[grp.n_levels] = rel;
     const int n_buckets = rel;
-    // The reduce walks 64 rounds per wavefront step where a level has many buckets (2^22-entry levels: 512
-    // buckets of 8192 entries, runs of about two pair blocks, which left half the lanes of a 16-round step
-    // idle; cfg3 backward 15.2 -> 14.2 ms uniform, 16.9 -> 16.1 ms shell) or enough rounds to give every
-    // wavefront of a block 64 (the benchmark shape: 16,384 rounds, scatter 6.83 -> 6.74 ms); small batches
-    // keep 16 rounds so that their few rounds spread over the block's wavefronts.  FFN_REDUCE_WALK64=0
-    // keeps the 16-round walk everywhere (the sums are exact, so both give the same table bit for bit).
+    grp.round_stride = plan.transpose ? 1 : grp.meta_stride;
+    grp.bucket_stride = plan.transpose ? grp.n_rounds : 1;
+    const uint32_t* meta = plan.transpose ? s.meta_t : s.meta;
+    // Rounds per wavefront step of the reduce: 64 where that gives every wavefront of a block some (cfg2's
+    // 16,384 rounds: scatter 6.83 -> 6.74 ms against 16; 512 buckets of 2^22-entry levels, whose runs of about two
+    // pair blocks leave most lanes of a 16-round step idle: 15.2 -> 14.2 ms), fewer so that a small batch's rounds
+    // spread over the block's wavefronts.  Blocks of 512 threads where several fit a CU.  FFN_REDUCE_WALK64=0: at
+    // most 16 rounds everywhere (the sums are exact, so the table is the same bit for bit).
+    const bool nt512 = lds_acc <= 32 * 1024;
+    const int n_waves = nt512 ? 8 : 16;
+    int seg = (plan.n_rounds + n_waves - 1) / n_waves;
     const char* w_env = getenv("FFN_REDUCE_WALK64");
-    const bool walk64 = (plan.max_nbl >= 256 || plan.n_rounds >= 16 * 64) && !(w_env && atoi(w_env) == 0);
+    const int seg_max = w_env && atoi(w_env) == 0 ? 16 : 64;
+    seg = seg < 1 ? 1 : (seg > seg_max ? seg_max : seg);
     const dim3 grid_bl((unsigned)plan.nblk, (unsigned)grp.n_levels);
     const dim3 grid_tr((unsigned)((plan.n_rounds + 63) / 64), (unsigned)((plan.max_nbl + 63) / 64),
                        (unsigned)grp.n_levels);
@@ -1118,14 +1199,15 @@ hipError_t launch_hash_bwd(const DevCfg& c, const PosSrc& src, int64_t n, const 
   do {                                                                                                             \
     hipLaunchKernelGGL((k_bin_emit<FV, MV>), grid_bl, dim3(emit_nt(FV)), lds_emit, st, c, src, n, grp, g, lay,   \
                        lr, s.meta, s.cmax, s.pairs, n_dev);                                                        \
-    hipLaunchKernelGGL(k_bin_meta_transpose, grid_tr, dim3(256), 0, st, s.meta, s.meta_t, grp.n_rounds,            \
-                       grp.meta_stride, n_dev, emit_nt(FV));                                                       \
-    if (walk64)                                                                                                    \
-      hipLaunchKernelGGL((k_bin_reduce<FV, MV, 64>), dim3((unsigned)n_buckets), dim3(1024), lds_acc, st, c, grp,   \
-                         s.meta_t, s.pairs, s.cmax, ap, n_dev);                                                    \
+    if (plan.transpose)                                                                                            \
+      hipLaunchKernelGGL(k_bin_meta_transpose, grid_tr, dim3(256), 0, st, s.meta, s.meta_t, grp.n_rounds,          \
+                         grp.meta_stride, n_dev, emit_nt(FV));                                                     \
+    if (nt512)                                                                                                     \
+      hipLaunchKernelGGL((k_bin_reduce<FV, MV, 512>), dim3((unsigned)n_buckets), dim3(512), lds_acc, st, c, grp,   \
+                         meta, s.pairs, s.cmax, apv, n_dev, seg);                                                  \
     else                                                                                                           \
-      hipLaunchKernelGGL((k_bin_reduce<FV, MV, 16>), dim3((unsigned)n_buckets), dim3(1024), lds_acc, st, c, grp,   \
-                         s.meta_t, s.pairs, s.cmax, ap, n_dev);                                                    \
+      hipLaunchKernelGGL((k_bin_reduce<FV, MV, 1024>), dim3((unsigned)n_buckets), dim3(1024), lds_acc, st, c, grp, \
+                         meta, s.pairs, s.cmax, apv, n_dev, seg);                                                  \
   } while (0)
 #define FFN_BIN_F(MV)                     \
   switch (c.F) {                          \

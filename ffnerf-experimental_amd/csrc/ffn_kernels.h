@@ -124,16 +124,22 @@ struct MlpArgs {
 enum { BIN_GRAD = 0, BIN_SGD = 1, BIN_ADAM = 2 };
 
 struct BinGroup {
-  int level0, n_levels, log2_be, chunk, nblk;
+  int level0, n_levels, chunk, nblk;
   int n_rounds;     // emit rounds per level (the samples in runs of the emit round size)
   int np;           // pair slots of one round (the stage size; a multiple of 8)
   int meta_stride;  // entries per round in the run table (the group's largest bucket count)
+  // run-table words between a bucket's rounds and between buckets: 1 and n_rounds once transposed to bucket-major,
+  // else as the emit writes it (meta_stride and 1)
+  int round_stride, bucket_stride;
+  int log2_be[FFN_MAX_LEVELS];         // entries of a bucket of each level of the group
   int nbl[FFN_MAX_LEVELS];             // buckets of each level of the group
   int bucket_rel[FFN_MAX_LEVELS + 1];  // first bucket of each level, relative to the group
 };
 
 struct BinPlan {
-  int log2_be, chunk, nblk, levels_per_group, max_buckets, max_nbl, n_rounds, np;
+  int log2_be[FFN_MAX_LEVELS], max_log2_be;  // entries of a bucket, per level and at most
+  int chunk, nblk, levels_per_group, max_buckets, max_nbl, n_rounds, np;
+  bool transpose;  // the reduce reads a bucket-major run table
   int64_t max_pairs, meta_elems;
 };
 
@@ -147,13 +153,17 @@ struct BinScratch {
 struct BinApply {
   void* dst;   // grad (BIN_GRAD), table (BIN_SGD, BIN_ADAM): float, or binary16 when dst_f16
   int dst_f16;
+  int vec4;    // dst, m and v are aligned for four values per access (set by launch_hash_bwd)
   float* m;
   float* v;
   float* g_tap;  // optional: the summed table gradient (BIN_ADAM)
   float lr_t, beta1, beta2, eps;
 };
 
-BinPlan plan_bins(const DevCfg& c, int64_t n, size_t pair_budget_bytes);
+// n: samples the buffers and launches are made for; n_typical: the samples the bucket sizes are chosen for (they
+// enter the fixed-point scale's pair counts, so a step sized for a capacity passes what the exactly sized step
+// would, and both give the same table bit for bit); n_cu: the GPU's compute units
+BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_budget_bytes, int n_cu);
 // whether the scatter is built for this table shape: a round's stage must fit in a CU's LDS and its run
 // offsets in 16 bits (F = 4 with 2^22-entry levels does not)
 bool scatter_supported(const DevCfg& c);
