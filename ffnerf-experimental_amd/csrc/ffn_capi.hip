@@ -93,7 +93,7 @@ struct Handle {
   Scratch m_blocks;  // the march's summary of the bitfield per 8^3 block, and its use flag
   Scratch m_slots;  // the marched step's per-ray sample slots (one walk instead of count + emit)
   Scratch dense;    // dense vertex copies of the coarse levels (the gather's)
-  Scratch tile_sched;  // the MLP's tile order: busy flags, their scan, scan sums, total, order
+  Scratch tile_sched;  // the MLP's tile order: busy flags (bytes), order, busy count
   uint32_t* host_total = nullptr;  // pinned
 };
 
@@ -127,14 +127,19 @@ bool march_slots_fit(const Scratch& held, size_t need) {
   return need <= ((size_t)mb << 20) && growth_fits_free(held, need);
 }
 
-// The gather's dense vertex copies: every level with 2 <= R and R^3 <= FFN_DENSE_MAX_CELLS (default 2^21:
-// 16 MB at F = 2 in fp32) vertices gets one, filled from `table` on the stream (they follow the table, so
-// they are rebuilt before every gather that follows a table update).  At the benchmark shape the row-major
-// copies of levels 0-6 (res 16-111) took the gather from 5.22 to 4.61 ms (adding level 7, res 154, 4.71;
-// all levels up to res 406 6.24); with levels 5-6 bricked 4.42 (level 7 bricked as well: no change).
-hipError_t build_dense_levels(Handle* h, const void* table, ffn::DenseLevels* dl, hipStream_t st) {
+// The gather's dense vertex copies of the coarse levels, filled from `table` on the stream (they follow the table,
+// so they are rebuilt before every gather that follows a table update).  A level of R^3 vertices gets one where
+// R^3 is at most 2^21 (at the benchmark shape the row-major copies of levels 0-6, res 16-111, took the gather from
+// 5.22 to 4.61 ms; adding level 7, res 154, 4.71; all levels up to res 406 6.24; with levels 5-6 bricked 4.42),
+// at most 16 times its table (a far smaller table is the better working set: 8 x 2^14 entries, 8.4M samples, step
+// 4915 us without copies, 4807 with levels up to 54^3, 4797 up to 122^3), and worth its filling for this gather's
+// n samples: at most 0.6 n vertices while the level's table fits an XCD's 4 MiB L2, 4 n beyond (16 x 2^19 entries,
+// fp16 step: 0.5M samples 640 us without, 629 up to 58^3, 632 up to 111^3; 1M 1137, 1113, 1110; 16 x 2^22 entries,
+// encode: 2^16 points 138 without, 129 up to 58^3, 151 up to 111^3; 2^18 475, 423, 401).  Below 2^16 samples none:
+// the fill's launch costs more (512 rays x 64: step 219 us with all, 201 without).  FFN_DENSE_MAX_CELLS sets the
+// number of vertices alone.
+hipError_t build_dense_levels(Handle* h, const void* table, int64_t n, ffn::DenseLevels* dl, hipStream_t st) {
   const char* env = getenv("FFN_DENSE_MAX_CELLS");
-  const long long max_cells = env ? atoll(env) : (1ll << 21);
   const ffn::DevCfg& c = h->dc;
   const size_t elem = c.table_f16 ? 2 : 4;
   uint64_t total = 0;
@@ -143,7 +148,16 @@ hipError_t build_dense_levels(Handle* h, const void* table, ffn::DenseLevels* dl
   dl->bricked = 0u;
   bool leading = true;
   for (int l = 0; l < c.L; ++l) {
-    const long long R = c.res[l];
+    const long long R = c.res[l], T = (long long)c.mask[l] + 1;
+    long long max_cells = 1ll << 21;
+    if (env) {
+      max_cells = atoll(env);
+    } else {
+      const bool in_l2 = (size_t)T * (size_t)c.F * elem <= ((size_t)4 << 20);
+      const double worth = n < (1 << 16) ? 0.0 : (in_l2 ? 0.6 : 4.0) * (double)n;
+      if (worth < (double)max_cells) max_cells = (long long)worth;
+      if (16 * T < max_cells) max_cells = 16 * T;
+    }
     if (R >= 2 && R * R * R <= max_cells) {
       // copies of at most 2 MiB are row-major and the leading ones share one gather pass
       // (FFN_DENSE_MULTI=0: none); larger copies are bricked (4x4x4 vertices, the grid padded to whole bricks)
@@ -566,7 +580,7 @@ int ffn_hash_encode_fwd(void* handle, const float* x, int64_t n, float* a0, uint
   const ffn::FeatLayout lm = ffn::level_major(n, h->dc.F);
   ffn::PosSrc src{x, nullptr, nullptr, 0};
   ffn::DenseLevels dl;
-  FFN_HIP(build_dense_levels(h, h->params.table, &dl, st));
+  FFN_HIP(build_dense_levels(h, h->params.table, n, &dl, st));
   FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, (float*)h->a0.p, lm, idx_out, &dl, st));
   FFN_HIP(ffn::launch_feat_relayout((const float*)h->a0.p, lm, a0, ffn::sample_major(h->dc.L, h->dc.F), n, h->dc.L,
                                     h->dc.F, st));
@@ -671,10 +685,11 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   float* dLda0 = (float*)h->dLda0.p;
   const ffn_params& P = h->params;
 
-  // the MLP's tile order (below): the sampler writes the tiles' busy flags
-  const size_t nt1 = (size_t)n_tiles + 1, n_sums = ((size_t)n_tiles + 4096) / 4096 + 2;
-  FFN_HIP(h->tile_sched.ensure(sizeof(uint32_t) * (3 * nt1 + n_sums + 4)));
-  uint32_t* tile_flags = (uint32_t*)h->tile_sched.p;
+  // the MLP's tile order (below): the sampler writes the tiles' busy flags (bytes, then the order and the count)
+  const size_t flag_bytes = ((size_t)n_tiles + 15) & ~(size_t)15;
+  FFN_HIP(h->tile_sched.ensure(flag_bytes + sizeof(uint32_t) * ((size_t)n_tiles + 1)));
+  uint8_t* tile_flags = (uint8_t*)h->tile_sched.p;
+  uint32_t* tile_order = (uint32_t*)(tile_flags + flag_bytes);
   {
     StageTimer tm(h, 0, st);
     FFN_HIP(ffn::launch_sample(h->dc, (const float4*)rays, num_rays, (int)spr, sc->rng_seed, P.occ_in,
@@ -685,7 +700,7 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
     ffn::PosSrc s2 = src;
     s2.Ts = Ts;
     ffn::DenseLevels dl;
-    FFN_HIP(build_dense_levels(h, P.table, &dl, st));
+    FFN_HIP(build_dense_levels(h, P.table, N, &dl, st));
     FFN_HIP(ffn::launch_hash_fwd(h->dc, s2, N, P.table, a0, feat, nullptr, &dl, st));
   }
 
@@ -716,9 +731,12 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   a.seed = sc->rng_seed;
   a.do_train = train ? 1 : 0;
   // the MLP's tile order: the busy tiles first, so that every block gets the same share of them (fp32 MLP
-  // 8.41 -> 8.30 ms at the benchmark shape)
-  a.tile_order = tile_flags + 2 * nt1;
-  a.n_busy = tile_flags + nt1 + n_tiles;  // the scan's total (offsets[n_tiles])
+  // 8.41 -> 8.30 ms at the benchmark shape); with a block per tile the flags alone do
+  a.tile_busy = tile_flags;
+  if (n_tiles > n_blocks) {
+    a.tile_order = tile_order;
+    a.n_busy = tile_order + n_tiles;
+  }
   if (taps) {
     a.t_sigma = taps->sigma;
     a.t_rgb = taps->rgb;
@@ -731,8 +749,7 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   }
   {
     StageTimer tm(h, 2, st);
-    FFN_HIP(ffn::launch_tile_order(n_tiles, tile_flags, tile_flags + nt1, tile_flags + 3 * nt1,
-                                   tile_flags + 3 * nt1 + n_sums, const_cast<uint32_t*>(a.tile_order), st));
+    if (a.tile_order) FFN_HIP(ffn::launch_tile_order(n_tiles, tile_flags, tile_order, tile_order + n_tiles, st));
     if (mlp16)
       FFN_HIP(ffn::launch_mlp16(a, LF, h->cfg.nd, h->cfg.nc, n_blocks, st));
     else
@@ -820,7 +837,8 @@ int check_march(Handle* h, const void* rays, const uint32_t* bits, const ffn_mar
   return 0;
 }
 
-// samples per ray the marched step's scatter is planned for (the ball scene of the benchmark marches 22)
+// samples per ray a marched step's or render's scatter and dense copies are planned for (the ball scene of the
+// benchmark marches 22, its shell field 10)
 constexpr int64_t MARCH_TYPICAL_SAMPLES = 16;
 
 ffn::MarchArgs march_args(Handle* h, const void* rays, uint32_t num_rays, const uint32_t* bits,
@@ -884,8 +902,7 @@ int ffn_march(void* handle, const void* rays, uint32_t num_rays, const uint32_t*
   FFN_HIP(h->m_offsets.ensure(sizeof(uint32_t) * n1));
   FFN_HIP(h->m_sums.ensure(sizeof(uint32_t) * ((n1 + 4095) / 4096 + 1)));
   uint32_t* off = (uint32_t*)h->m_offsets.p;
-  FFN_HIP(ffn::launch_scan_u32(counts, num_rays, off, (uint32_t*)h->m_sums.p, total, st));
-  FFN_HIP(hipMemcpyAsync(offsets, off, sizeof(uint32_t) * num_rays, hipMemcpyDeviceToDevice, st));
+  FFN_HIP(ffn::launch_scan_u32(counts, num_rays, off, (uint32_t*)h->m_sums.p, total, st, false, offsets));
   a.offsets = off;
   a.samples = (float4*)samples;
   a.ray_ids = ray_ids;
@@ -915,8 +932,7 @@ int ffn_march_noalloc(void* handle, const void* rays, uint32_t num_rays, const u
   a.counts = counts;
   FFN_HIP(ffn::launch_march(a, false, st));
   // every word the scan reads is written by it first (offsets, tile sums, total): nothing to clear
-  FFN_HIP(ffn::launch_scan_u32(counts, num_rays, off, sums, total, st));
-  FFN_HIP(hipMemcpyAsync(offsets, off, sizeof(uint32_t) * num_rays, hipMemcpyDeviceToDevice, st));
+  FFN_HIP(ffn::launch_scan_u32(counts, num_rays, off, sums, total, st, false, offsets));
   a.offsets = off;
   a.samples = (float4*)samples;
   a.ray_ids = ray_ids;
@@ -1034,7 +1050,7 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
   {
     StageTimer tm(h, 1, st);
     ffn::DenseLevels dl;
-    FFN_HIP(build_dense_levels(h, P.table, &dl, st));
+    FFN_HIP(build_dense_levels(h, P.table, MARCH_TYPICAL_SAMPLES * num_rays, &dl, st));
     FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, P.table, a0, feat, nullptr, &dl, st, n_dev));
   }
   // 3-5. forward MLP, compositing with early termination and the loss, MLP backward.  (With a capacity the
@@ -1244,7 +1260,7 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
   int n_blocks = h->n_cu > 0 ? 2 * h->n_cu : 512;
   const uint32_t rounds = (mp->max_steps + mp->chunk - 1) / mp->chunk;
   ffn::DenseLevels dl;  // the table does not change during the render: one copy serves every round
-  FFN_HIP(build_dense_levels(h, h->params.table, &dl, st));
+  FFN_HIP(build_dense_levels(h, h->params.table, MARCH_TYPICAL_SAMPLES * num_rays, &dl, st));
   // (without waits: the round's count is *total, read on the device; n the capacity)
   const uint32_t* n_dev = no_wait ? total : nullptr;
   for (uint32_t round = 0; round < rounds; ++round) {

@@ -93,9 +93,10 @@ struct MlpArgs {
   // NULL
   const uint32_t* tile_order;
   // with tile_order: the number of busy tiles (a sample with dt > 0), which the order puts first; the
-  // kernels composite the later positions' tiles to the background without the MLP (NULL: every tile takes
-  // the full path)
+  // kernels composite the later positions' tiles to the background without the MLP
   const uint32_t* n_busy;
+  // without tile_order (a block per tile at most): byte t = tile t is busy (NULL: every tile takes the full path)
+  const uint8_t* tile_busy;
   float sh_mult, occ_strength;
   uint32_t seed;
   int do_train;
@@ -168,10 +169,10 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_bud
 // offsets in 16 bits (F = 4 with 2^22-entry levels does not)
 bool scatter_supported(const DevCfg& c);
 
-// tile_busy (may be NULL): word t = 1 when one of samples 64t .. 64t + 63 has dt > 0 (the MLP's busy tiles)
+// tile_busy (may be NULL): byte t = 1 when one of samples 64t .. 64t + 63 has dt > 0 (the MLP's busy tiles)
 hipError_t launch_sample(const DevCfg& c, const float4* rays, uint32_t num_rays, int S, uint32_t seed,
                          const uint32_t* occ_in, int do_train, float* Ts, float* DTs, uint32_t* flags,
-                         hipStream_t st, uint32_t* tile_busy = nullptr);
+                         hipStream_t st, uint8_t* tile_busy = nullptr);
 
 // table: float, or binary16 when c.table_f16 (widened exactly; the sums are the same fp32 operations)
 // Dense copies of the coarse levels' vertex values (the table's element type, F per vertex) from
@@ -268,9 +269,9 @@ hipError_t launch_render_composite(const uint32_t* offsets, const uint32_t* coun
 hipError_t launch_render_finish(const float4* acc, uint32_t num_rays, float4* out_rgb, hipStream_t st);
 // exclusive scan of in[0..n) into out[0..n]; out[n] and *total get the sum.  gated: the kernels do nothing
 // while *total == 0 on entry (a render round after one without samples: in is all zero and out already holds
-// its scan)
+// its scan).  copy (may be NULL): the first n outputs once more
 hipError_t launch_scan_u32(const uint32_t* in, int64_t n, uint32_t* out, uint32_t* sums, uint32_t* total,
-                           hipStream_t st, bool gated = false);
+                           hipStream_t st, bool gated = false, uint32_t* copy = nullptr);
 
 // compositing of a marched training batch (one lane per ray, front to back, stopping after the sample that
 // leaves T < T_stop), the photometric loss gradient and the compositing backward of every sample
@@ -323,11 +324,10 @@ bool mlp_supported(int LF, int nd, int nc);
 int mlp_blocks_per_cu(int LF, int nd, int nc);  // blocks of launch_mlp that fit on one CU
 int mlp16_blocks_per_cu(int LF, int nd, int nc);  // blocks of launch_mlp16 that fit on one CU
 hipError_t launch_mlp(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st);
-// order[n_tiles]: the tiles with a sample of dt > 0 in index order, then the others; scratch: flags and off
-// n_tiles + 1 words each, sums (n_tiles + 4096) / 4096 + 1 words, total 1 word
-// flags: the tiles' busy flags (launch_sample's tile_busy)
-hipError_t launch_tile_order(int64_t n_tiles, const uint32_t* flags, uint32_t* off, uint32_t* sums, uint32_t* total,
-                             uint32_t* order, hipStream_t st);
+// order[n_tiles]: the tiles whose byte in flags (launch_sample's tile_busy; 16-byte aligned) is 1 in index order,
+// then the others; *n_busy: how many are
+hipError_t launch_tile_order(int64_t n_tiles, const uint8_t* flags, uint32_t* order, uint32_t* n_busy,
+                             hipStream_t st);
 // the same kernel's backward over marched samples (a.smp, a.ray_ids, a.in_dLds, a.in_dLdc; a.num_rays = the
 // sample count, log2S = 0): no compositing, no proposals
 hipError_t launch_mlp_marched(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st);

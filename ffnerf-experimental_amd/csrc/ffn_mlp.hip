@@ -508,7 +508,11 @@ __global__ __launch_bounds__(256, (Arch<LF, ND, NC>::blocks_per_cu())) void k_ml
   // and all its gradients are zero, so the later positions only write that (empty_tile).  Taps, which expose
   // per-sample MLP outputs, take the full path for every tile.  (Two loops: an exit from the full path for
   // the empty tiles had the register allocator copy the gradient accumulators on every tile.)
-  const int64_t n_full = (TAPS || MARCHED || !a.n_busy) ? n_tiles : (int64_t)*a.n_busy;
+  int64_t n_full = n_tiles;
+  if constexpr (!TAPS && !MARCHED) {
+    if (a.tile_order) n_full = (int64_t)*a.n_busy;
+    else if (a.tile_busy && blockIdx.x < n_tiles && !a.tile_busy[blockIdx.x]) n_full = 0;
+  }
   int parity = 0;
   int64_t ti = blockIdx.x;
   // Issue priority.  The two blocks a CU holds (blocks b and b + gridDim.x / 2, as the dispatcher deals
@@ -872,26 +876,77 @@ hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, co
 }
 
 // Tile order of a step: the sampler flags each 64-sample tile with a sample of dt > 0 (the tiles the MLP
-// computes; the others composite to the background); the scan of the flags places the busy tiles first, in
-// index order, then the others.  With the busy tiles dealt round-robin the blocks get equal shares of them
-// (with tiles dealt in index order, a quarter of the rays missing the box left the busiest of 512 blocks
-// 8.5 % above the mean).  The order depends on the data alone, so steps stay deterministic.
-__global__ __launch_bounds__(256) void k_tile_place(const uint32_t* __restrict__ flags,
-                                                    const uint32_t* __restrict__ off, int64_t n_tiles,
-                                                    uint32_t* __restrict__ order) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n_tiles) return;
-  const uint32_t o = off[t], n_busy = off[n_tiles];
-  order[flags[t] ? o : n_busy + ((uint32_t)t - o)] = (uint32_t)t;
+// computes; the others composite to the background); the busy tiles are placed first, in index order, then the
+// others.  With the busy tiles dealt round-robin the blocks get equal shares of them (with tiles dealt in index
+// order, a quarter of the rays missing the box left the busiest of 512 blocks 8.5 % above the mean).  The order
+// depends on the data alone, so steps stay deterministic.
+// One launch: a block places 4096 tiles and counts the flags before them, and all of them, itself (bytes, 16 per
+// load; 262,144 tiles: 64 blocks of 256 KiB from the L2).  As a scan of three kernels and a placement the order
+// cost four launches of 4.5 us each.
+constexpr int TO_TILES = 4096;
+__global__ __launch_bounds__(1024) void k_tile_order(const uint8_t* __restrict__ flags, int64_t n_tiles,
+                                                     uint32_t* __restrict__ order, uint32_t* __restrict__ n_busy) {
+  __shared__ uint32_t w_before[16], w_all[16], w_own[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t t0 = (int64_t)blockIdx.x * TO_TILES;
+  uint32_t before = 0, all = 0;  // busy tiles before the block's, and of all
+  for (int64_t i = 16 * (int64_t)tid; i < n_tiles; i += 16 * 1024) {
+    uint4 f = *reinterpret_cast<const uint4*>(flags + i);
+    if (i + 16 > n_tiles) {  // bytes past the last tile are not flags
+      const int keep = (int)(n_tiles - i);
+      auto cut = [keep](uint32_t w, int at) {
+        return keep >= at + 4 ? w : (keep <= at ? 0u : w & ((1u << (8 * (keep - at))) - 1u));
+      };
+      f = make_uint4(cut(f.x, 0), cut(f.y, 4), cut(f.z, 8), cut(f.w, 12));
+    }
+    const uint32_t c = __popc(f.x) + __popc(f.y) + __popc(f.z) + __popc(f.w);
+    all += c;
+    if (i < t0) before += c;  // t0 is a multiple of 16
+  }
+  const int64_t tb = t0 + 4 * (int64_t)tid;
+  uint32_t own[4], s = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    own[q] = tb + q < n_tiles ? flags[tb + q] : 0u;
+    s += own[q];
+  }
+  uint32_t incl = s;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t o = __shfl_up(incl, d);
+    if (lane >= d) incl += o;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    before += __shfl_xor(before, d);
+    all += __shfl_xor(all, d);
+  }
+  if (lane == 63) {
+    w_before[wave] = before;
+    w_all[wave] = all;
+    w_own[wave] = incl;
+  }
+  __syncthreads();
+  uint32_t run = incl - s, total = 0;
+  for (int w = 0; w < 16; ++w) {
+    run += w_before[w] + (w < wave ? w_own[w] : 0u);
+    total += w_all[w];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int64_t t = tb + q;
+    if (t >= n_tiles) break;
+    order[own[q] ? run : total + ((uint32_t)t - run)] = (uint32_t)t;
+    run += own[q];
+  }
+  if (blockIdx.x == 0 && tid == 0) *n_busy = total;
 }
 
-hipError_t launch_tile_order(int64_t n_tiles, const uint32_t* flags, uint32_t* off, uint32_t* sums, uint32_t* total,
-                             uint32_t* order, hipStream_t st) {
+hipError_t launch_tile_order(int64_t n_tiles, const uint8_t* flags, uint32_t* order, uint32_t* n_busy,
+                             hipStream_t st) {
   if (n_tiles <= 0) return hipSuccess;
-  hipError_t e = launch_scan_u32(flags, n_tiles, off, sums, total, st);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_tile_place, dim3((unsigned)((n_tiles + 255) / 256)), dim3(256), 0, st, flags, off, n_tiles,
-                     order);
+  hipLaunchKernelGGL(k_tile_order, dim3((unsigned)((n_tiles + TO_TILES - 1) / TO_TILES)), dim3(1024), 0, st, flags,
+                     n_tiles, order, n_busy);
   return hipGetLastError();
 }
 

@@ -676,7 +676,11 @@ __global__ __launch_bounds__(256, (Arch16<LF, ND, NC>::blocks_per_cu())) void k_
   // and all its gradients are zero, so the later positions only write that (empty_tile).  Taps, which expose
   // per-sample MLP outputs, take the full path for every tile.  (Two loops: an exit from the full path for
   // the empty tiles had the register allocator copy the gradient accumulators on every tile.)
-  const int64_t n_full = (TAPS || MARCHED || !a.n_busy) ? n_tiles : (int64_t)*a.n_busy;
+  int64_t n_full = n_tiles;
+  if constexpr (!TAPS && !MARCHED) {
+    if (a.tile_order) n_full = (int64_t)*a.n_busy;
+    else if (a.tile_busy && blockIdx.x < n_tiles && !a.tile_busy[blockIdx.x]) n_full = 0;
+  }
   int parity = 0;
   int64_t ti = blockIdx.x;
 #pragma unroll 1
