@@ -1063,13 +1063,16 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_bud
   const int rs = emit_nt(c.F);  // samples per emit round
   p.n_rounds = (int)((n + rs - 1) / rs);
   // Bucket sizes.  A bucket's int64 LDS accumulator is 2^log2_be * F * 8 bytes.
+  // Every level gets at least 64 buckets (of at least 64 entries): a level of a small table has as many pairs as
+  // any other, and 4 buckets of 2048 entries kept 4 blocks busy for the whole reduce (the reference's table sizes,
+  // F = 4, 2^20 samples: 1263 -> 322 us).
   // Large batches: at most 64 KiB (two reduce blocks per CU), or 128 KiB (one) when a level would otherwise have
   // more than 64 buckets.  An emit round's pairs spread over the buckets, and every run costs its two edge
   // sectors twice (the neighbouring buckets' blocks read them too) plus its padding: at the benchmark shape
   // 64 buckets per level measured emit 4.95 and reduce 2.81 ms against 5.12 and 3.19 ms with 128.
   // Small batches (fewer than 512 rounds; at 625 the large buckets measured emit 257 and reduce 204 us against 283
   // and 227): the table's update, not the pairs, is most of the reduce's work, so
-  // a level gets 64 to 256 buckets, of at most 2048 entries (4096 at F = 1) where that many suffice, and several
+  // a level gets up to 256 buckets, of at most 2048 entries (4096 at F = 1) where that many suffice, and several
   // blocks share a CU.
   int max_be = c.F == 4 ? 11 : (c.F == 2 ? 12 : 13);
   uint32_t max_T = 0;
@@ -1078,9 +1081,9 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_bud
   const bool small = (n_typical + rs - 1) / rs < 512;
   for (int l = 0; l < c.L; ++l) {
     int lg = max_be;
+    if (small) lg = c.F == 1 ? 12 : (c.F == 2 ? 11 : 10);  // 32 KiB
+    while (lg > 6 && ((c.mask[l] + 1u) >> lg) < 64u) --lg;
     if (small) {
-      lg = c.F == 1 ? 12 : (c.F == 2 ? 11 : 10);  // 32 KiB
-      while (lg > 6 && ((c.mask[l] + 1u) >> lg) < 64u) --lg;
       while (lg < max_be && ((c.mask[l] + 1u) >> lg) > (c.F == 4 ? 512u : 256u)) ++lg;  // the emit's stage pads every bucket's run
       lg = lg < max_be ? lg : max_be;
     }
