@@ -213,6 +213,24 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* pl
   return hipSuccess;
 }
 
+ffn::MlpPtrs mlp_ptrs(const ffn_params& P) {
+  ffn::MlpPtrs w{};
+  uintptr_t bits = 0;
+  for (int k = 0; k < FFN_N_LAYERS; ++k) {
+    w.W[k] = P.W[k];
+    w.b[k] = P.b[k];
+    bits |= (uintptr_t)P.W[k];
+  }
+  w.aligned16 = (bits & 15) == 0;
+  return w;
+}
+
+// CUs times the blocks a kernel runs per CU, at most one per tile of 64 samples
+int grid_blocks(const Handle* h, int per_cu, int64_t n_tiles) {
+  const int64_t b = (int64_t)(h->n_cu > 0 ? h->n_cu : 256) * per_cu;
+  return (int)(b < n_tiles ? b : (n_tiles > 0 ? n_tiles : 1));
+}
+
 bool is_pow2(uint32_t v) { return v && !(v & (v - 1)); }
 
 uint32_t max_level_entries(const ffn::DevCfg& c) {
@@ -661,9 +679,8 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   while ((1u << log2S) < spr) ++log2S;
   const int64_t N = (int64_t)num_rays * spr;
   const int64_t n_tiles = (N + 63) / 64;
-  int n_blocks = (h->n_cu > 0 ? h->n_cu : 256) * (mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc)
-                                                          : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc));
-  if (n_blocks > n_tiles) n_blocks = (int)n_tiles;
+  const int n_blocks = grid_blocks(h, mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, train)
+                                             : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, train), n_tiles);
 
   FFN_HIP(h->Ts.ensure(sizeof(float) * N));
   FFN_HIP(h->DTs.ensure(sizeof(float) * N));
@@ -706,10 +723,7 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
 
   ffn::MlpArgs a{};
   a.c = h->dc;
-  for (int k = 0; k < FFN_N_LAYERS; ++k) {
-    a.w.W[k] = P.W[k];
-    a.w.b[k] = P.b[k];
-  }
+  a.w = mlp_ptrs(P);
   a.rays = (const float4*)rays;
   a.targets = (const float4*)targets;
   a.out_rgb = (float4*)out_rgb;
@@ -1057,23 +1071,20 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
   // blocks are those of the capacity's tiles: a block's tiles and the order of the partials' sum are the same
   // as for the kept count, the further blocks add zero partials.)
   const int64_t n_tiles = (n + 63) / 64;
-  int n_blocks = (h->n_cu > 0 ? h->n_cu : 256) * (mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc)
-                                                         : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc));
-  if (n_blocks > n_tiles) n_blocks = (int)(n_tiles > 0 ? n_tiles : 1);
+  const int n_blocks = grid_blocks(h, mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, true)
+                                             : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, true), n_tiles);
+  const int fwd_blocks = grid_blocks(h, mlp16 ? ffn::mlp16_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc)
+                                               : ffn::mlp_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), n_tiles);
   FFN_HIP(h->partials.ensure(sizeof(float) * (size_t)n_blocks * h->lay.total));
-  ffn::MlpPtrs w{};
-  for (int k = 0; k < FFN_N_LAYERS; ++k) {
-    w.W[k] = P.W[k];
-    w.b[k] = P.b[k];
-  }
+  const ffn::MlpPtrs w = mlp_ptrs(P);
   {
     StageTimer tm(h, 2, st);
     if (mlp16)
       FFN_HIP(ffn::launch_mlp16_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, sc->sh_multiplier, sigma, rgb,
-                                    LF, h->cfg.nd, h->cfg.nc, n_blocks, st, n_dev));
+                                    LF, h->cfg.nd, h->cfg.nc, fwd_blocks, st, n_dev));
     else
       FFN_HIP(ffn::launch_mlp_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, sc->sh_multiplier, sigma, rgb,
-                                  LF, h->cfg.nd, h->cfg.nc, n_blocks, st, n_dev));
+                                  LF, h->cfg.nd, h->cfg.nc, fwd_blocks, st, n_dev));
     ffn::CompMarchArgs ca{};
     ca.offsets = off;
     ca.counts = counts;
@@ -1242,11 +1253,7 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
   a.samples = samples;
   a.ray_ids = ids;
   a.capacity = cap;
-  ffn::MlpPtrs w{};
-  for (int k = 0; k < FFN_N_LAYERS; ++k) {
-    w.W[k] = h->params.W[k];
-    w.b[k] = h->params.b[k];
-  }
+  const ffn::MlpPtrs w = mlp_ptrs(h->params);
   // Each round walks every live ray once into its own chunk of slots (its count and walk state written by the
   // same pass), then packs the slots into the scanned order; without room for the slots (the budget of the
   // marched step) it walks twice, count then emit.  The samples, their order and the walk states agree.
@@ -1257,7 +1264,6 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
   a1.slot_stride = mp->chunk;
   a1.samples = (float4*)h->m_slots.p;
   a1.ray_ids = nullptr;
-  int n_blocks = h->n_cu > 0 ? 2 * h->n_cu : 512;
   const uint32_t rounds = (mp->max_steps + mp->chunk - 1) / mp->chunk;
   ffn::DenseLevels dl;  // the table does not change during the render: one copy serves every round
   FFN_HIP(build_dense_levels(h, h->params.table, MARCH_TYPICAL_SAMPLES * num_rays, &dl, st));
@@ -1283,8 +1289,7 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
     src.x_stride = 4;
     const ffn::FeatLayout feat = ffn::level_major(n, h->dc.F);
     FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, a0, feat, nullptr, &dl, st, n_dev));
-    int nb = (int)((n + 63) / 64);
-    if (nb > n_blocks) nb = n_blocks;
+    const int nb = grid_blocks(h, ffn::mlp_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), (n + 63) / 64);
     FFN_HIP(ffn::launch_mlp_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, mp->sh_multiplier, sigma, rgb, LF,
                                 h->cfg.nd, h->cfg.nc, nb, st, n_dev));
     FFN_HIP(ffn::launch_render_composite(off, counts, num_rays, sigma, rgb, mp->dt, mp->T_stop, state, acc,

@@ -66,6 +66,7 @@ inline FeatLayout level_major(int64_t n, int F) { return FeatLayout{n * F, F}; }
 struct MlpPtrs {
   const float* W[FFN_N_LAYERS];
   const float* b[FFN_N_LAYERS];
+  int aligned16;  // every W is 16-byte aligned
 };
 
 constexpr int RELU_WORDS = 14;  // ReLU-branch tap words per sample: two per hidden layer slot (3 density, 4 colour)
@@ -321,8 +322,12 @@ hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, co
 
 // fused MLP forward + compositing + loss + backward + proposals, per 64-sample tile
 bool mlp_supported(int LF, int nd, int nc);
-int mlp_blocks_per_cu(int LF, int nd, int nc);  // blocks of launch_mlp that fit on one CU
-int mlp16_blocks_per_cu(int LF, int nd, int nc);  // blocks of launch_mlp16 that fit on one CU
+// blocks of launch_mlp / launch_mlp16 that run on one CU (training, or forward-only), and of the forward over
+// indexed samples
+int mlp_blocks_per_cu(int LF, int nd, int nc, bool train);
+int mlp16_blocks_per_cu(int LF, int nd, int nc, bool train);
+int mlp_fwd_blocks_per_cu(int LF, int nd, int nc);
+int mlp16_fwd_blocks_per_cu(int LF, int nd, int nc);
 hipError_t launch_mlp(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st);
 // order[n_tiles]: the tiles whose byte in flags (launch_sample's tile_busy; 16-byte aligned) is 1 in index order,
 // then the others; *n_busy: how many are

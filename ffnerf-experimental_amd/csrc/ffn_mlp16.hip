@@ -66,6 +66,12 @@ __host__ __device__ constexpr int kslot_neuron(int kb, int g, int j) {
 // the same for the position p = 32 kb + 8 g + j of a K-ordered row
 __host__ __device__ constexpr int kpos_neuron(int p) { return kslot_neuron(p >> 5, (p >> 3) & 3, p & 7); }
 
+// the position of neuron n in a K-ordered row (kpos_neuron's inverse); four consecutive neurons from a multiple of
+// four on have consecutive positions
+__host__ __device__ constexpr int neuron_kpos(int n) {
+  return (n & ~31) + 8 * ((n >> 2) & 3) + 4 * ((n >> 4) & 1) + (n & 3);
+}
+
 __device__ __forceinline__ half4 to_half4(const floatx4& v) {
   half4 h;
 #pragma unroll
@@ -176,11 +182,52 @@ struct Arch16 {
   // when training (the stash barriers separate a tile's compositing from the next tile's writes), two
   // alternating slots for a forward-only launch
   static constexpr int comp_floats = 512;
-  static constexpr size_t lds_bytes() {
-    return (size_t)w_halves() * 2 + (size_t)b_floats() * 4 + (size_t)stash_halves() * 2 + comp_floats * 4;
+  // a forward-only launch holds the forward copies alone and has no stash
+  static constexpr int halves(bool train) { return train ? w_halves() : wf_off(FFN_N_LAYERS); }
+  static constexpr size_t lds_bytes(bool train) {
+    return (size_t)halves(train) * 2 + (size_t)b_floats() * 4 + (train ? (size_t)stash_halves() * 2 : 0) +
+           comp_floats * 4;
   }
-  static constexpr int blocks_per_cu() { return lds_bytes() <= 80 * 1024 ? 2 : 1; }
+  static constexpr int blocks_per_cu(bool train) {
+    const int fit = (int)(160 * 1024 / lds_bytes(train)), most = train ? 2 : 4;
+    return fit < 1 ? 1 : (fit < most ? fit : most);
+  }
+  // k_mlp16_fwd holds the forward copies and biases alone
+  static constexpr int fwd_blocks_per_cu() {
+    const int fit = (int)(160 * 1024 / ((size_t)wf_off(FFN_N_LAYERS) * 2 + (size_t)b_floats() * 4));
+    return fit < 1 ? 1 : (fit < 4 ? fit : 4);
+  }
 };
+
+// stage the weights into LDS: fp16 [out_pad][in] and, for the backward (T), [in][out_pad] (K-ordered columns where
+// K blocks are 32 wide, the rows and columns of a padded layer zero), fp32 biases
+template <int LF, int ND, int NC, bool T>
+__device__ __forceinline__ void stage_weights16(_Float16* __restrict__ sWf, float* __restrict__ sB, const MlpPtrs& wp,
+                                                int tid) {
+  using A = Arch16<LF, ND, NC>;
+  read_weights<LF, ND, NC, 256>(
+      wp, tid,
+      [&](auto K, int o, int i, const float4& v) {
+        constexpr int k = K;
+        constexpr bool kf = layer_in(k, LF) % 32 == 0, kt = A::rows_pad(k) % 32 == 0;
+        const half4 h = to_half4(floatx4{v.x, v.y, v.z, v.w});
+        *reinterpret_cast<half4*>(sWf + A::wf_off(k) + o * A::pf(k) + (kf ? neuron_kpos(i) : i)) = h;
+        if constexpr (T) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sWf[A::wt_off(k) + (i + r) * A::pt(k) + (kt ? neuron_kpos(o) : o)] = h[r];
+        }
+      },
+      [&](auto K, int o, float v) { sB[A::b_off(K) + o] = v; });
+  constexpr int k = FFN_WC_OUT;  // rows 3 .. 15
+  constexpr int O = layer_out(k), R = A::rows_pad(k), I = layer_in(k, LF);
+  static_assert(R == 16, "not K-ordered");
+  for (int e = A::pf(k) * O + tid; e < R * A::pf(k); e += 256) sWf[A::wf_off(k) + e] = (_Float16)0.0f;
+  if constexpr (T) {
+    for (int e = tid; e < I * R; e += 256)
+      if (e % R >= O) sWf[A::wt_off(k) + (e / R) * A::pt(k) + e % R] = (_Float16)0.0f;
+  }
+  if (tid >= O && tid < R) sB[A::b_off(k) + tid] = 0.0f;
+}
 
 // forward layer, K = 32 blocks: out tiles = act(W . in + b); W is the K-ordered forward copy
 template <int OT, int KB>
@@ -606,17 +653,16 @@ __device__ __forceinline__ void load_tile_in(const MlpArgs& a, int64_t b, bool v
 // a.in_dLdc, the samples' rays, times and step from the march; no compositing, no proposals.  TRAIN
 // (a.do_train) is a template parameter for the reason given at k_mlp.
 template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC, bool TRAIN>
-__global__ __launch_bounds__(256, (Arch16<LF, ND, NC>::blocks_per_cu())) void k_mlp16(MlpArgs a) {
+__global__ __launch_bounds__(256, (TRAIN ? Arch16<LF, ND, NC>::blocks_per_cu(true) : 4)) void k_mlp16(MlpArgs a) {
   static_assert(TRAIN || !MARCHED, "marched launches train");
   using A = Arch16<LF, ND, NC>;
   constexpr int KB0 = LF / 16;  // D-layout tiles of the encoding
   extern __shared__ __align__(16) unsigned char smem16[];
   _Float16* sWf = reinterpret_cast<_Float16*>(smem16);
   _Float16* sWt = sWf;  // the transposed copies follow the forward weights (offsets in 16-bit units)
-  float* sB = reinterpret_cast<float*>(smem16 + (size_t)A::w_halves() * 2);
-  __bf16* sS = reinterpret_cast<__bf16*>(smem16 + (size_t)A::w_halves() * 2 + (size_t)A::b_floats() * 4);
-  float* sC = reinterpret_cast<float*>(smem16 + (size_t)A::w_halves() * 2 + (size_t)A::b_floats() * 4 +
-                                       (size_t)A::stash_halves() * 2);
+  float* sB = reinterpret_cast<float*>(smem16 + (size_t)A::halves(TRAIN) * 2);
+  __bf16* sS = reinterpret_cast<__bf16*>(sB + A::b_floats());
+  float* sC = reinterpret_cast<float*>(sS + (TRAIN ? A::stash_halves() : 0));
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
   const int col = wave * 16 + s;  // this lane's sample column in a tile
   constexpr bool train = TRAIN;
@@ -630,27 +676,7 @@ __global__ __launch_bounds__(256, (Arch16<LF, ND, NC>::blocks_per_cu())) void k_
     n_tiles = (int64_t)((n_samples + 63) / 64);
   }
 
-  // weights: fp16 [out_pad][in] and [in][out_pad] (K-ordered columns where K blocks are 32 wide, zero
-  // padding), fp32 biases
-#pragma unroll
-  for (int k = 0; k < FFN_N_LAYERS; ++k) {
-    if (!layer_active(k, ND, NC)) continue;
-    const int O = layer_out(k), I = layer_in(k, LF), R = A::rows_pad(k);
-    const int PF = A::pf(k), PT = A::pt(k);
-    const bool kf = I % 32 == 0, kt = R % 32 == 0;
-    const float* gw = a.w.W[k];
-    for (int e = tid; e < R * PF; e += 256) {
-      const int r = e / PF, p = e - r * PF;
-      const int i = p < I ? (kf ? kpos_neuron(p) : p) : I;
-      sWf[A::wf_off(k) + e] = (_Float16)((r < O && i < I) ? gw[r * I + i] : 0.0f);
-    }
-    for (int e = tid; e < I * PT; e += 256) {
-      const int i = e / PT, p = e - i * PT;
-      const int o = p < R ? (kt ? kpos_neuron(p) : p) : R;
-      sWt[A::wt_off(k) + e] = (_Float16)((o < O) ? gw[o * I + i] : 0.0f);
-    }
-    for (int e = tid; e < R; e += 256) sB[A::b_off(k) + e] = e < O ? a.w.b[k][e] : 0.0f;
-  }
+  stage_weights16<LF, ND, NC, TRAIN>(sWf, sB, a.w, tid);
   __syncthreads();
 
   const float Dhalf = half_box_diagonal(c);
@@ -885,7 +911,7 @@ __global__ __launch_bounds__(256, (Arch16<LF, ND, NC>::blocks_per_cu())) void k_
 template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC, bool TRAIN>
 static hipError_t launch16_k(const MlpArgs& a, int n_blocks, hipStream_t st) {
   using A = Arch16<LF, ND, NC>;
-  const size_t lds = A::lds_bytes();
+  const size_t lds = A::lds_bytes(TRAIN);
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)k_mlp16<LF, ND, NC, FEAT, TAPS, MARCHED, SC, TRAIN>,
@@ -943,18 +969,7 @@ __global__ __launch_bounds__(256) void k_mlp16_fwd(MlpPtrs wp, const float* __re
   _Float16* sWf = reinterpret_cast<_Float16*>(smem16f);
   float* sB = reinterpret_cast<float*>(smem16f + (size_t)A::wf_off(FFN_N_LAYERS) * 2);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
-#pragma unroll
-  for (int k = 0; k < FFN_N_LAYERS; ++k) {
-    if (!layer_active(k, ND, NC)) continue;
-    const int O = layer_out(k), I = layer_in(k, LF), R = A::rows_pad(k), PF = A::pf(k);
-    const bool kf = I % 32 == 0;
-    for (int e = tid; e < R * PF; e += 256) {
-      const int r = e / PF, p = e - r * PF;
-      const int i = p < I ? (kf ? kpos_neuron(p) : p) : I;
-      sWf[A::wf_off(k) + e] = (_Float16)((r < O && i < I) ? wp.W[k][r * I + i] : 0.0f);
-    }
-    for (int e = tid; e < R; e += 256) sB[A::b_off(k) + e] = e < O ? wp.b[k][e] : 0.0f;
-  }
+  stage_weights16<LF, ND, NC, false>(sWf, sB, wp, tid);
   __syncthreads();
   for (int64_t grp = (int64_t)blockIdx.x * 4 + wave; grp * 16 < n; grp += (int64_t)gridDim.x * 4) {
     const int64_t b = grp * 16 + s;
@@ -1008,9 +1023,17 @@ static hipError_t launch16_fwd_f(const MlpPtrs& w, const float* a0, const FeatLa
   X(32, 2, 2)                \
   X(64, 2, 2)
 
-int mlp16_blocks_per_cu(int LF, int nd, int nc) {
+int mlp16_blocks_per_cu(int LF, int nd, int nc, bool train) {
 #define X(l, d, n) \
-  if (LF == l && nd == d && nc == n) return Arch16<l, d, n>::blocks_per_cu();
+  if (LF == l && nd == d && nc == n) return Arch16<l, d, n>::blocks_per_cu(train);
+  FFN_MLP16_CONFIGS(X)
+#undef X
+  return 1;
+}
+
+int mlp16_fwd_blocks_per_cu(int LF, int nd, int nc) {
+#define X(l, d, n) \
+  if (LF == l && nd == d && nc == n) return Arch16<l, d, n>::fwd_blocks_per_cu();
   FFN_MLP16_CONFIGS(X)
 #undef X
   return 1;
