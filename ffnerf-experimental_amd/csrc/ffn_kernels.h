@@ -274,7 +274,7 @@ hipError_t launch_render_finish(const float4* acc, uint32_t num_rays, float4* ou
 hipError_t launch_scan_u32(const uint32_t* in, int64_t n, uint32_t* out, uint32_t* sums, uint32_t* total,
                            hipStream_t st, bool gated = false, uint32_t* copy = nullptr);
 
-// compositing of a marched training batch (one lane per ray, front to back, stopping after the sample that
+// compositing of a marched training batch (one wavefront per ray, front to back, stopping after the sample that
 // leaves T < T_stop), the photometric loss gradient and the compositing backward of every sample
 struct CompMarchArgs {
   const uint32_t* offsets;

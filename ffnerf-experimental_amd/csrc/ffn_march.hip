@@ -43,6 +43,7 @@
 
 #include "ffn_device.h"
 #include "ffn_kernels.h"
+#include "ffn_mlp_common.h"
 
 namespace ffn {
 
@@ -703,10 +704,6 @@ __global__ __launch_bounds__(256) void k_render_finish(const float4* __restrict_
   out_rgb[r] = acc[r];  // black background: C + T * 0; w = T_final
 }
 
-// Compositing of marched training rays: one lane per ray walks its samples front to back (the order of the
-// specification, ora_train_step_marched), keeping the transmittance before every sample for the backward
-// sweep, which walks them back to front with dL/dT of the next sample (ffnerf_OG.cl:1593-1634 restated as a
-// sequential recurrence: gT_i = g . (alpha_i c_i) + (1 - alpha_i) gT_(i+1), gT_end = g . bg).
 // (cell, subcell) of the occupancy grid holding the point at time t of ray (o, d), as the proposals compute it;
 // kOutsideGrid for a point outside the grid
 constexpr uint64_t kOutsideGrid = ~(uint64_t)1;
@@ -725,99 +722,170 @@ __device__ __forceinline__ uint64_t occ_run_key(const DevCfg& c, const float (&o
 // The occupancy proposals of marched ray r: its samples, in order, fall into runs of one (cell, subcell) of the
 // occupancy grid, and each run inside the grid proposes as a run of the resampled step does
 // (ffnerf_OG.cl:1640-1821), from the compositing's transmittances (T_end past a termination, so those runs
-// propose nothing).
-__device__ void propose_marched_runs(const CompMarchArgs& a, uint32_t r, uint32_t off, uint32_t cnt, float T_end) {
-  if (cnt == 0) return;
-  const float4 ro = a.rays[2 * r], rdv = a.rays[2 * r + 1];
+// propose nothing).  One wavefront per ray: a lane whose sample starts a run walks to the run's end and proposes.
+__device__ __forceinline__ void propose_marched_runs(const CompMarchArgs& a, uint32_t r, uint32_t off, uint32_t cnt,
+                                                     float T_end, int lane) {
+  const float4 ro = a.rays[2 * (size_t)r], rdv = a.rays[2 * (size_t)r + 1];
   const float o[3] = {ro.x, ro.y, ro.z}, d[3] = {rdv.x, rdv.y, rdv.z};
   const float Dhalf = half_box_diagonal(a.c);
-  uint32_t s = 0;
-  float t_s = a.samples[off].w;
-  uint64_t key_s = occ_run_key(a.c, o, d, t_s);
-  for (uint32_t j = 1; j <= cnt; ++j) {
-    float t_j = 0.0f;
-    uint64_t key_j = ~(uint64_t)0;
-    if (j < cnt) {
+  for (uint32_t s = (uint32_t)lane; s < cnt; s += 64) {
+    const float t_s = a.samples[off + s].w;
+    const uint64_t key = occ_run_key(a.c, o, d, t_s);
+    const uint32_t prev = s > 0 ? s - 1 : 0;
+    const float t_prev = a.samples[off + prev].w;
+    if (key == kOutsideGrid || (s > 0 && occ_run_key(a.c, o, d, t_prev) == key)) continue;
+    uint32_t j = s + 1;  // the run's end
+    float t_last = t_s, t_j = 0.0f;
+    for (; j < cnt; ++j) {
       t_j = a.samples[off + j].w;
-      key_j = occ_run_key(a.c, o, d, t_j);
+      if (occ_run_key(a.c, o, d, t_j) != key) break;
+      t_last = t_j;
     }
-    if (key_j == key_s) continue;
-    if (key_s != kOutsideGrid) {  // the run [s, j) ends here
-      const uint32_t prev = s > 0 ? s - 1 : 0;
-      const bool has_next = j < cnt;
-      occ_propose_run(a.c, o, d, t_s, a.Tr[off + s], a.samples[off + prev].w, a.Tr[off + prev],
-                      a.samples[off + j - 1].w, a.Tr[off + j - 1], has_next, t_j, has_next ? a.Tr[off + j] : 0.0f,
-                      T_end, a.occ_in[key_s >> 3], a.seed, r, s, Dhalf, a.occ_st);
-    }
-    s = j;
-    t_s = t_j;
-    key_s = key_j;
+    const bool has_next = j < cnt;
+    occ_propose_run(a.c, o, d, t_s, a.Tr[off + s], t_prev, a.Tr[off + prev], t_last, a.Tr[off + j - 1], has_next,
+                    has_next ? t_j : 0.0f, has_next ? a.Tr[off + j] : 0.0f, T_end, a.occ_in[key >> 3], a.seed, r, s,
+                    Dhalf, a.occ_st);
   }
 }
 
-__global__ __launch_bounds__(256) void k_composite_marched(CompMarchArgs a) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= a.num_rays) return;
-  const uint32_t cnt = a.counts[r], off = a.offsets[r];
-  float T = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f;
-  uint32_t used = 0;
-  for (uint32_t j = 0; j < cnt; ++j) {
-    const uint32_t b = off + j;
-    const float alpha = 1.0f - fast_exp(fminf(fmaxf(-a.sigma[b] * a.dt, -5.0f), 18.0f));
-    a.Tr[b] = T;
-    const float w = T * alpha;
-    C0 = C0 + w * a.rgb[3 * (size_t)b];
-    C1 = C1 + w * a.rgb[3 * (size_t)b + 1];
-    C2 = C2 + w * a.rgb[3 * (size_t)b + 2];
-    T = T * (1.0f - alpha);
-    ++used;
-    if (T < a.T_stop) break;
+// dL/dT after each lane's sample of a group of 64: the sample's map x -> b + a x (a = 1 - alpha, b = g . (alpha c)),
+// composed over the later lanes and applied to gT, dL/dT after the group; gT becomes the one before it.  Inside a
+// 16-lane row the composition is a suffix scan by DPP row shifts; the four rows follow each other by readlane.
+__device__ __forceinline__ float grad_T_after(float a, float b, int lane, float& gT) {
+  auto step = [&](float ar, float br) {  // self, then the lane to the right
+    b = b + a * br;
+    a = a * ar;
+  };
+  step(dpp_or<0x101>(1.0f, a), dpp_or<0x101>(0.0f, b));  // row_shl:1, 2, 4, 8: the identity past the row's end
+  step(dpp_or<0x102>(1.0f, a), dpp_or<0x102>(0.0f, b));
+  step(dpp_or<0x104>(1.0f, a), dpp_or<0x104>(0.0f, b));
+  step(dpp_or<0x108>(1.0f, a), dpp_or<0x108>(0.0f, b));
+  const float ea = dpp_or<0x101>(1.0f, a), eb = dpp_or<0x101>(0.0f, b);  // the lanes after this one in its row
+  auto rl = [](float x, int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), i)); };
+  const float g3 = gT;  // dL/dT after row 3, 2, 1, 0
+  const float g2 = rl(b, 48) + rl(a, 48) * g3;
+  const float g1 = rl(b, 32) + rl(a, 32) * g2;
+  const float g0 = rl(b, 16) + rl(a, 16) * g1;
+  gT = rl(b, 0) + rl(a, 0) * g0;
+  const int row = lane >> 4;
+  return eb + ea * (row == 3 ? g3 : (row == 2 ? g2 : (row == 1 ? g1 : g0)));
+}
+
+// Compositing of marched training rays and its backward, one wavefront per ray: the specification's recurrences
+// over the ray's samples (ora_train_step_marched; ffnerf_OG.cl:1593-1634 restated: T_(i+1) = T_i (1 - alpha_i);
+// gT_i = g . (alpha_i c_i) + (1 - alpha_i) gT_(i+1), gT_end = g . bg) as scans over 64 samples at a time.
+// What bounds it: latency (a ray's groups follow each other, each a few dependent loads and two scans).  A lane
+// per ray, each walking its own range of the sample arrays, waited for its loads: 40,001 rays with 880,000 samples
+// 217 us, now 28; 2^18 rays 390, now 127.  The recurrences kept sequential over the lanes' values by readlane
+// took 97 and 395 us.
+// (rays_per_wave: consecutive rays of a wavefront)
+__global__ __launch_bounds__(256) void k_composite_marched(CompMarchArgs a, uint32_t rays_per_wave) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t r0 = ((uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * rays_per_wave;
+  auto rl = [](float x, int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), i)); };
+  for (uint64_t rr = r0; rr < r0 + rays_per_wave && rr < a.num_rays; ++rr) {
+    const uint32_t r = (uint32_t)rr;
+    const uint32_t cnt = a.counts[r], off = a.offsets[r];
+    float T = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f;
+    uint32_t used = 0;  // samples up to and including the one that leaves T < T_stop
+    bool stopped = false;
+    for (uint32_t b0 = 0; b0 < cnt && !stopped; b0 += 64) {
+      const int n = (int)(cnt - b0 < 64 ? cnt - b0 : 64);
+      const size_t b = (size_t)off + b0 + lane;
+      float alpha = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
+      if (lane < n) {
+        alpha = 1.0f - fast_exp(fminf(fmaxf(-a.sigma[b] * a.dt, -5.0f), 18.0f));
+        c0 = a.rgb[3 * b];
+        c1 = a.rgb[3 * b + 1];
+        c2 = a.rgb[3 * b + 2];
+      }
+      const float oma = 1.0f - alpha;
+      Seg tot;
+      const Seg pre = comp_seg_prefix(Seg{oma, alpha * c0, alpha * c1, alpha * c2}, lane, 64, &tot);
+      const float Tr = T * pre.a;  // before this lane's sample
+      // the group's samples up to the first that leaves T < T_stop
+      const uint64_t stop = __ballot(lane < n && Tr * oma < a.T_stop);
+      const int m = stop != 0ull ? (int)__builtin_ctzll(stop) + 1 : n;
+      stopped = stop != 0ull;
+      if (stopped) {  // the colours up to sample m - 1
+        const float w = pre.a * alpha;
+        tot = Seg{rl(pre.a * oma, m - 1), rl(pre.v0 + w * c0, m - 1), rl(pre.v1 + w * c1, m - 1),
+                  rl(pre.v2 + w * c2, m - 1)};
+      }
+      C0 = C0 + T * tot.v0;
+      C1 = C1 + T * tot.v1;
+      C2 = C2 + T * tot.v2;
+      T = T * tot.a;
+      if (lane < m) a.Tr[b] = Tr;
+      used += (uint32_t)m;
+    }
+    float bg[3] = {0.0f, 0.0f, 0.0f};
+    if (a.background == FFN_BG_WHITE) {
+      bg[0] = bg[1] = bg[2] = 1.0f;
+    } else if (a.background == FFN_BG_RANDOM) {
+      uint32_t rb = hash_u32(a.seed ^ r * 747796405u ^ 0xA511E9B3u);
+      bg[0] = rand01(rb);
+      bg[1] = rand01(rb);
+      bg[2] = rand01(rb);
+    }
+    const float4 tg = a.targets[r];
+    const float Cf0 = C0 + T * bg[0], Cf1 = C1 + T * bg[1], Cf2 = C2 + T * bg[2];
+    const float gr0 = charbonnier_prime(Cf0 - tg.x), gr1 = charbonnier_prime(Cf1 - tg.y),
+                gr2 = charbonnier_prime(Cf2 - tg.z);
+    if (lane == 0) {
+      a.out_rgb[r] = make_float4(fminf(fmaxf(Cf0, 0.0f), 1.0f), fminf(fmaxf(Cf1, 0.0f), 1.0f),
+                                 fminf(fmaxf(Cf2, 0.0f), 1.0f), 4.0f);
+      if (a.n_used) a.n_used[r] = used;
+      if (a.T_final) a.T_final[r] = T;
+      if (a.color) a.color[r] = make_float4(Cf0, Cf1, Cf2, 0.0f);
+    }
+    // past the termination: no contribution, no gradient
+    for (uint32_t s = used + (uint32_t)lane; s < cnt; s += 64) {
+      const size_t b = (size_t)off + s;
+      a.Tr[b] = T;
+      a.dLds[b] = 0.0f;
+      a.dLdc[3 * b] = a.dLdc[3 * b + 1] = a.dLdc[3 * b + 2] = 0.0f;
+    }
+    float gT = gr0 * bg[0] + gr1 * bg[1] + gr2 * bg[2];
+    for (uint32_t e = used; e > 0;) {  // groups of 64 from the back, aligned as in the forward
+      const uint32_t b0 = (e - 1) & ~63u;
+      const int n = (int)(e - b0);
+      const size_t b = (size_t)off + b0 + lane;
+      float alpha = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f, Ti = 0.0f;
+      if (lane < n) {
+        alpha = 1.0f - fast_exp(fminf(fmaxf(-a.sigma[b] * a.dt, -5.0f), 18.0f));
+        c0 = a.rgb[3 * b];
+        c1 = a.rgb[3 * b + 1];
+        c2 = a.rgb[3 * b + 2];
+        Ti = a.Tr[b];  // written by this lane above
+      }
+      const float oma = 1.0f - alpha;
+      const float gc = gr0 * (alpha * c0) + gr1 * (alpha * c1) + gr2 * (alpha * c2);
+      const float g_next = grad_T_after(oma, gc, lane, gT);  // dL/dT after this lane's sample
+      if (lane < n) {
+        const float gA = gr0 * (Ti * c0) + gr1 * (Ti * c1) + gr2 * (Ti * c2);
+        const float gAlpha = gA - g_next * Ti;
+        a.dLds[b] = gAlpha * (a.dt * oma) + a.regu;
+        const float ws = Ti * alpha;
+        a.dLdc[3 * b] = ws * gr0;
+        a.dLdc[3 * b + 1] = ws * gr1;
+        a.dLdc[3 * b + 2] = ws * gr2;
+      }
+      e = b0;
+    }
+    if (a.occ_st) {
+      __threadfence_block();  // the lanes read each other's Tr
+      propose_marched_runs(a, r, off, cnt, T, lane);
+    }
   }
-  float bg[3] = {0.0f, 0.0f, 0.0f};
-  if (a.background == FFN_BG_WHITE) {
-    bg[0] = bg[1] = bg[2] = 1.0f;
-  } else if (a.background == FFN_BG_RANDOM) {
-    uint32_t rb = hash_u32(a.seed ^ r * 747796405u ^ 0xA511E9B3u);
-    bg[0] = rand01(rb);
-    bg[1] = rand01(rb);
-    bg[2] = rand01(rb);
-  }
-  const float4 tg = a.targets[r];
-  const float Cf0 = C0 + T * bg[0], Cf1 = C1 + T * bg[1], Cf2 = C2 + T * bg[2];
-  const float gr0 = charbonnier_prime(Cf0 - tg.x), gr1 = charbonnier_prime(Cf1 - tg.y),
-              gr2 = charbonnier_prime(Cf2 - tg.z);
-  a.out_rgb[r] = make_float4(fminf(fmaxf(Cf0, 0.0f), 1.0f), fminf(fmaxf(Cf1, 0.0f), 1.0f),
-                             fminf(fmaxf(Cf2, 0.0f), 1.0f), 4.0f);
-  if (a.n_used) a.n_used[r] = used;
-  if (a.T_final) a.T_final[r] = T;
-  if (a.color) a.color[r] = make_float4(Cf0, Cf1, Cf2, 0.0f);
-  float gT = gr0 * bg[0] + gr1 * bg[1] + gr2 * bg[2];
-  for (uint32_t j = used; j-- > 0;) {
-    const uint32_t b = off + j;
-    const float alpha = 1.0f - fast_exp(fminf(fmaxf(-a.sigma[b] * a.dt, -5.0f), 18.0f));
-    const float Ti = a.Tr[b];
-    const float c0 = a.rgb[3 * (size_t)b], c1 = a.rgb[3 * (size_t)b + 1], c2 = a.rgb[3 * (size_t)b + 2];
-    const float gA = gr0 * (Ti * c0) + gr1 * (Ti * c1) + gr2 * (Ti * c2);
-    const float gAlpha = gA - gT * Ti;
-    a.dLds[b] = gAlpha * (a.dt * (1.0f - alpha)) + a.regu;
-    const float ws = Ti * alpha;
-    a.dLdc[3 * (size_t)b] = ws * gr0;
-    a.dLdc[3 * (size_t)b + 1] = ws * gr1;
-    a.dLdc[3 * (size_t)b + 2] = ws * gr2;
-    gT = (gr0 * (alpha * c0) + gr1 * (alpha * c1) + gr2 * (alpha * c2)) + (1.0f - alpha) * gT;
-  }
-  for (uint32_t j = used; j < cnt; ++j) {  // past the termination: no contribution, no gradient
-    const uint32_t b = off + j;
-    a.Tr[b] = T;
-    a.dLds[b] = 0.0f;
-    a.dLdc[3 * (size_t)b] = a.dLdc[3 * (size_t)b + 1] = a.dLdc[3 * (size_t)b + 2] = 0.0f;
-  }
-  if (a.occ_st) propose_marched_runs(a, r, off, cnt, T);
 }
 
 hipError_t launch_composite_marched(const CompMarchArgs& a, hipStream_t st) {
   if (a.num_rays == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_composite_marched, dim3((a.num_rays + 255) / 256), dim3(256), 0, st, a);
+  // one ray per wavefront while the rays are few, so that rays with samples do not queue behind each other
+  const uint32_t rpw = a.num_rays < (1u << 17) ? 1 : 4;
+  const uint64_t waves = ((uint64_t)a.num_rays + rpw - 1) / rpw;
+  hipLaunchKernelGGL(k_composite_marched, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a, rpw);
   return hipGetLastError();
 }
 
