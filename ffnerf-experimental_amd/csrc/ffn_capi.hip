@@ -93,6 +93,7 @@ struct Handle {
   Scratch m_blocks;  // the march's summary of the bitfield per 8^3 block, and its use flag
   Scratch m_slots;  // the marched step's per-ray sample slots (one walk instead of count + emit)
   Scratch dense;    // dense vertex copies of the coarse levels (the gather's)
+  Scratch order_counts, order_pairs, order_perm, order_pts;  // the encode entry points' spatial order
   Scratch tile_sched;  // the MLP's tile order: busy flags (bytes), order, busy count
   uint32_t* host_total = nullptr;  // pinned
 };
@@ -210,6 +211,54 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* pl
   s->meta_t = (uint32_t*)h->bin_meta_t.p;
   s->pairs = (uint4*)h->bin_pairs.p;
   s->cmax = (float*)h->bin_max.p;
+  return hipSuccess;
+}
+
+// Whether ffn_hash_encode_fwd gathers in a spatial order of its points: the sort and the rows written through its
+// permutation cost about 65 us and 0.07 ns a point, and the gather wins the more, the further the tables lie from
+// the L2 and the closer the points.  us, plain / ordered, uniform points; points on a shell:
+//   16 x 2^22 entries (32 MiB a level): 2^18 417 / 457; 375 / 352    2^20 1475 / 1363; 1355 / 907
+//                                       2^22 5711 / 4440; 5208 / 2580  2^24 22020 / 14395; 20858 / 7685
+//   16 x 2^19 entries (4 MiB): 2^20 579 / 597; 552 / 479    2^22 2172 / 1892; 2015 / 1440
+//    8 x 2^14 entries: 2^20 216 / 255; 201 / 206    2^22 794 / 715; 742 / 593
+// The scatter gains nothing reliable (2^22 points, 16 x 2^22: 3837 / 3882; 4187 / 3749; 16 x 2^19 2713 / 2925): the
+// merged pairs leave runs of one or two pairs a bucket, which are padded to eight.  FFN_ORDER=0: never, 1: always.
+bool order_pays(const Handle* h, int64_t n) {
+  if (n >= ((int64_t)1 << 31)) return false;
+  if (const char* e = getenv("FFN_ORDER")) return atoi(e) != 0;
+  uint32_t T = 0;
+  for (int l = 0; l < h->dc.L; ++l) T = h->dc.mask[l] + 1 > T ? h->dc.mask[l] + 1 : T;
+  const bool in_l2 = (size_t)T * (size_t)h->dc.F * (h->dc.table_f16 ? 2 : 4) <= ((size_t)4 << 20);
+  if (n < ((int64_t)1 << (in_l2 ? 22 : 20))) return false;
+  // 36 bytes a point of scratch: the plain order where the device is short of memory
+  const size_t need = (size_t)n * (2 * sizeof(uint2) + sizeof(float4) + sizeof(uint32_t));
+  const bool held = h->order_pairs.bytes >= 2 * sizeof(uint2) * (size_t)n &&
+                    h->order_pts.bytes >= sizeof(float4) * (size_t)n &&
+                    h->order_perm.bytes >= sizeof(uint32_t) * (size_t)n;
+  return held || growth_fits_free(Scratch{}, need);
+}
+
+// the points' Morton order in the handle's scratch: src becomes the ordered points, *perm their indices
+hipError_t order_points(Handle* h, int64_t n, ffn::PosSrc* src, const uint32_t** perm, hipStream_t st) {
+  const size_t words = ffn::order_count_words(n), sums = (words + 4096) / 4096 + 2;
+  hipError_t e;
+  if ((e = h->order_counts.ensure(sizeof(uint32_t) * (2 * words + 1 + sums + 1))) != hipSuccess) return e;
+  if ((e = h->order_pairs.ensure(2 * sizeof(uint2) * (size_t)n)) != hipSuccess) return e;
+  if ((e = h->order_perm.ensure(sizeof(uint32_t) * (size_t)n)) != hipSuccess) return e;
+  if ((e = h->order_pts.ensure(sizeof(float4) * (size_t)n)) != hipSuccess) return e;
+  ffn::OrderScratch s{};
+  s.counts = (uint32_t*)h->order_counts.p;
+  s.offsets = s.counts + words;
+  s.sums = s.offsets + words + 1;
+  s.total = s.sums + sums;
+  s.pairs[0] = (uint2*)h->order_pairs.p;
+  s.pairs[1] = s.pairs[0] + n;
+  e = ffn::launch_order_points(h->dc, src->x, n, s, (uint32_t*)h->order_perm.p, (float4*)h->order_pts.p, st);
+  if (e != hipSuccess) return e;
+  src->x = (const float*)h->order_pts.p;
+  src->x_stride = 4;
+  src->spatial = true;
+  *perm = (const uint32_t*)h->order_perm.p;
   return hipSuccess;
 }
 
@@ -528,7 +577,8 @@ int ffn_destroy(void* handle) {
   h->bin_max.release();
   for (Scratch* sc : {&h->m_state, &h->m_acc, &h->m_counts, &h->m_offsets, &h->m_sums, &h->m_total, &h->m_samples,
                       &h->m_ids, &h->m_a0, &h->m_sigma, &h->m_rgb, &h->m_Tr, &h->m_dLds, &h->m_dLdc, &h->m_bits,
-                      &h->m_blocks, &h->m_slots, &h->dense, &h->tile_sched})
+                      &h->m_blocks, &h->m_slots, &h->dense, &h->tile_sched, &h->order_counts,
+                      &h->order_pairs, &h->order_perm, &h->order_pts})
     sc->release();
   if (h->host_total) (void)hipHostFree(h->host_total);
   delete h;
@@ -597,11 +647,13 @@ int ffn_hash_encode_fwd(void* handle, const float* x, int64_t n, float* a0, uint
   FFN_HIP(h->a0.ensure(sizeof(float) * (size_t)n * h->dc.LF));
   const ffn::FeatLayout lm = ffn::level_major(n, h->dc.F);
   ffn::PosSrc src{x, nullptr, nullptr, 0};
+  const uint32_t* perm = nullptr;  // (corner indices are written in the points' own order)
+  if (!idx_out && order_pays(h, n)) FFN_HIP(order_points(h, n, &src, &perm, st));
   ffn::DenseLevels dl;
   FFN_HIP(build_dense_levels(h, h->params.table, n, &dl, st));
   FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, (float*)h->a0.p, lm, idx_out, &dl, st));
   FFN_HIP(ffn::launch_feat_relayout((const float*)h->a0.p, lm, a0, ffn::sample_major(h->dc.L, h->dc.F), n, h->dc.L,
-                                    h->dc.F, st));
+                                    h->dc.F, st, perm));
   return 0;
 }
 

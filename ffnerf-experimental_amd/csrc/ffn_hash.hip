@@ -280,7 +280,10 @@ __global__ __launch_bounds__(256) void k_hash_fwd(DevCfg c, PosSrc src, int64_t 
                                                   float* __restrict__ a0, FeatLayout lay,
                                                   uint32_t* __restrict__ idx_out, DenseLevels dl,
                                                   const uint32_t* __restrict__ n_dev) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int64_t blk = blockIdx.x;
+  // workgroups are dealt to the eight XCDs in turn (the grid's width is then a multiple of eight)
+  if (src.spatial) blk = (int64_t)(blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int64_t b = blk * blockDim.x + threadIdx.x;
   if constexpr (DEV) {
     const int64_t nd = (int64_t)*n_dev, nn = nd < n ? nd : n;
     for (int64_t bb = b; bb < nn; bb += (int64_t)gridDim.x * blockDim.x)
@@ -995,6 +998,7 @@ static hipError_t launch_hash_fwd_d(const DevCfg& c, const PosSrc& src, int64_t 
   const int rows = dl.n_multi > 0 ? c.L - dl.n_multi + 1 : c.L;
   int64_t bx = (n + 255) / 256;
   if (DEV && bx > HASH_FWD_DEV_BLOCKS) bx = HASH_FWD_DEV_BLOCKS;
+  if (src.spatial) bx = (bx + 7) & ~(int64_t)7;
   const dim3 grid((unsigned)bx, (unsigned)rows), block(256);
 #define FFN_FWD(FV) \
   hipLaunchKernelGGL((k_hash_fwd<FV, TT, DEV>), grid, block, 0, st, c, src, n, table, a0, lay, idx_out, dl, n_dev)
@@ -1238,12 +1242,18 @@ hipError_t launch_hash_bwd(const DevCfg& c, const PosSrc& src, int64_t n, const 
 constexpr int RL_TB = 128;
 template <bool TO_LEVEL_MAJOR>
 __global__ __launch_bounds__(256) void k_feat_relayout(const float* __restrict__ src, float* __restrict__ dst,
-                                                       int64_t n, int L, int F) {
+                                                       int64_t n, int L, int F, const uint32_t* __restrict__ perm) {
   extern __shared__ float tile[];
+  __shared__ uint32_t rows[RL_TB];  // with perm (to sample-major): the tile's rows
   const int LF = L * F, pitch = LF + 1, lgF = F >> 1;  // F is 1, 2 or 4
   const int64_t b0 = (int64_t)blockIdx.x * RL_TB;
   const int nb = (int)(n - b0 < RL_TB ? n - b0 : RL_TB);
   const int tid = threadIdx.x;
+  if (perm) {
+    if (tid < nb) rows[tid] = perm[b0 + tid];
+    __syncthreads();
+  }
+  auto row = [&](int bq) { return perm ? (int64_t)rows[bq] : b0 + bq; };
   // sample-major side: element i of the range is (sample i / LF, feature i % LF); the quotient and
   // remainder advance by a fixed step per iteration
   const int qs = 256 / LF, rs = 256 % LF;
@@ -1269,7 +1279,7 @@ __global__ __launch_bounds__(256) void k_feat_relayout(const float* __restrict__
     __syncthreads();
     int bq = tid / LF, kr = tid % LF;
     for (int i = tid; i < nb * LF; i += 256) {
-      dst[b0 * LF + i] = tile[bq * pitch + kr];
+      dst[row(bq) * LF + kr] = tile[bq * pitch + kr];
       bq += qs;
       kr += rs;
       if (kr >= LF) {
@@ -1281,20 +1291,20 @@ __global__ __launch_bounds__(256) void k_feat_relayout(const float* __restrict__
 }
 
 hipError_t launch_feat_relayout(const float* src, const FeatLayout& ls, float* dst, const FeatLayout& ld, int64_t n,
-                                int L, int F, hipStream_t st) {
+                                int L, int F, hipStream_t st, const uint32_t* perm) {
   if (n <= 0) return hipSuccess;
   const FeatLayout sm = sample_major(L, F), lm = level_major(n, F);
   const bool s_sm = ls.stride_l == sm.stride_l && ls.stride_b == sm.stride_b;
   const bool s_lm = ls.stride_l == lm.stride_l && ls.stride_b == lm.stride_b;
   const bool d_sm = ld.stride_l == sm.stride_l && ld.stride_b == sm.stride_b;
   const bool d_lm = ld.stride_l == lm.stride_l && ld.stride_b == lm.stride_b;
-  if (!((s_sm && d_lm) || (s_lm && d_sm)) || (F != 1 && F != 2 && F != 4)) return hipErrorInvalidValue;
+  if (!((s_sm && d_lm) || (s_lm && d_sm)) || (F != 1 && F != 2 && F != 4) || (perm && s_sm)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((n + RL_TB - 1) / RL_TB));
   const size_t lds = sizeof(float) * (size_t)RL_TB * (size_t)(L * F + 1);
   if (s_sm)
-    hipLaunchKernelGGL(k_feat_relayout<true>, grid, dim3(256), lds, st, src, dst, n, L, F);
+    hipLaunchKernelGGL(k_feat_relayout<true>, grid, dim3(256), lds, st, src, dst, n, L, F, nullptr);
   else
-    hipLaunchKernelGGL(k_feat_relayout<false>, grid, dim3(256), lds, st, src, dst, n, L, F);
+    hipLaunchKernelGGL(k_feat_relayout<false>, grid, dim3(256), lds, st, src, dst, n, L, F, perm);
   return hipGetLastError();
 }
 

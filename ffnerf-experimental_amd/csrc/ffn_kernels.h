@@ -53,7 +53,23 @@ struct PosSrc {
   const float* Ts;
   int log2S;
   int x_stride = 3;
+  // the points are in a spatial order (launch_order_points): the gather gives each XCD a contiguous part of them,
+  // so that the points around a vertex share one L2
+  bool spatial = false;
 };
+
+// Morton order of n points x [n][3] (n < 2^31): perm[i] = the i-th point's index, pts[i] its position; stable, so the
+// order depends on the points alone
+struct OrderScratch {
+  uint32_t* counts;   // order_count_words(n)
+  uint32_t* offsets;  // order_count_words(n) + 1
+  uint32_t* sums;     // launch_scan_u32's
+  uint32_t* total;    // 1
+  uint2* pairs[2];    // n each
+};
+size_t order_count_words(int64_t n);
+hipError_t launch_order_points(const DevCfg& c, const float* x, int64_t n, const OrderScratch& s, uint32_t* perm,
+                               float4* pts, hipStream_t st);
 
 // element (sample b, level l, feature f) of an encoding-shaped array is at
 // l * stride_l + b * stride_b + f: sample-major [N][L*F] or level-major [L][N][F]
@@ -202,8 +218,9 @@ hipError_t launch_hash_fwd(const DevCfg& c, const PosSrc& src, int64_t n, const 
 hipError_t launch_hash_bwd(const DevCfg& c, const PosSrc& src, int64_t n, const float* g, const FeatLayout& lay,
                            int mode, float lr, const BinApply& ap, const BinPlan& plan, const BinScratch& s,
                            hipStream_t st, const uint32_t* n_dev = nullptr);
+// sample-major <-> level-major; perm (to sample-major only; may be NULL): sample b goes to row perm[b]
 hipError_t launch_feat_relayout(const float* src, const FeatLayout& ls, float* dst, const FeatLayout& ld, int64_t n,
-                                int L, int F, hipStream_t st);
+                                int L, int F, hipStream_t st, const uint32_t* perm = nullptr);
 
 hipError_t launch_adam(float* p, float* m, float* v, float* g, int64_t n, float lr_t, float b1, float b2, float eps,
                        int zero_grad, hipStream_t st);

@@ -1,0 +1,61 @@
+"""ffn_hash_encode_fwd in a spatial order of its points (FFN_ORDER=1) gives the encodings of the plain order bit for
+bit: point counts around the sort's blocks and wavefronts, points that coincide, lie outside the box or are not
+finite, every F and table type; and by its own rule beyond 2^20 points."""
+import numpy as np
+import pytest
+
+from common import random_params, spec_cfg0
+
+pytestmark = pytest.mark.gpu
+
+
+def points(n, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.random((n, 3), dtype=np.float32)
+    x[rng.random(n) < 0.2] = np.float32(0.25)
+    out = rng.random(n) < 0.05
+    x[out] = x[out] * 7.0 - 3.0
+    if n > 8:
+        x[1] = np.nan
+        x[3] = [np.inf, 0.5, -np.inf]
+        x[5] = [1.0, 0.0, 1.0]
+    return x
+
+
+@pytest.mark.parametrize("n,F,table", [(1, 2, 0), (63, 1, 0), (4095, 2, 1), (4096, 4, 0), (4097, 2, 0), (70001, 1, 1),
+                                       (262145, 4, 1)])
+def test_order_changes_nothing(monkeypatch, n, F, table):
+    from gpu_helpers import GpuModel
+    L = 4
+    spec = spec_cfg0(n_levels=L, f_per_level=F, log2_T=[9, 14, 16, 18], res=[5.0, 33.0, 130.0, 700.0],
+                     table_dtype=table)
+    m = GpuModel(spec, random_params(spec, seed=3))
+    x = points(n, n)
+    print(f"[encode order] n={n} F={F} table={table}", flush=True)
+    res = []
+    for env in ("0", "1", "1"):
+        monkeypatch.setenv("FFN_ORDER", env)
+        res.append(encode(m, x, L * F))
+    np.testing.assert_array_equal(res[0].view(np.uint32), res[1].view(np.uint32))
+    np.testing.assert_array_equal(res[1].view(np.uint32), res[2].view(np.uint32))
+
+
+def encode(m, x, lf):
+    import ffn_lib as fl
+    import torch
+    x_t = torch.from_numpy(x).cuda()
+    out = torch.full((x.shape[0], lf), 7.0, device="cuda")
+    fl.check(m.lib.ffn_hash_encode_fwd(m.h.h, fl.ptr(x_t), x.shape[0], fl.ptr(out), None, fl.stream_ptr()), "encode")
+    return out.cpu().numpy()
+
+
+def test_order_by_rule(monkeypatch):
+    from gpu_helpers import GpuModel
+    spec = spec_cfg0(n_levels=2, log2_T=[20, 20], res=[150.0, 900.0])
+    m = GpuModel(spec, random_params(spec, seed=4))
+    x = points((1 << 20) + 77, 5)
+    print("[encode order] by rule", flush=True)
+    monkeypatch.delenv("FFN_ORDER", raising=False)
+    by_rule = encode(m, x, 4)
+    monkeypatch.setenv("FFN_ORDER", "0")
+    np.testing.assert_array_equal(by_rule.view(np.uint32), encode(m, x, 4).view(np.uint32))
