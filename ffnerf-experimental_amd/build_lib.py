@@ -18,7 +18,7 @@ ARCH = os.environ.get("FFN_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["ffn_capi.hip", "ffn_sample.hip", "ffn_hash.hip", "ffn_mlp.hip", "ffn_optim.hip", "ffn_march.hip",
-           "ffn_mlp16.hip", "ffn_batch.hip", "ffn_order.hip"]
+           "ffn_mlp16.hip", "ffn_batch.hip", "ffn_order.hip", "ffn_mlp_fwd.hip"]
 
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -731,8 +731,9 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   while ((1u << log2S) < spr) ++log2S;
   const int64_t N = (int64_t)num_rays * spr;
   const int64_t n_tiles = (N + 63) / 64;
-  const int n_blocks = grid_blocks(h, mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, train)
-                                             : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, train), n_tiles);
+  const bool view = !train && !mlp16;  // launch_mlp_view: a tile per wavefront
+  const int n_blocks = grid_blocks(h, view ? 1 : mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, train)
+                                                       : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), n_tiles);
 
   FFN_HIP(h->Ts.ensure(sizeof(float) * N));
   FFN_HIP(h->DTs.ensure(sizeof(float) * N));
@@ -797,9 +798,9 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   a.seed = sc->rng_seed;
   a.do_train = train ? 1 : 0;
   // the MLP's tile order: the busy tiles first, so that every block gets the same share of them (fp32 MLP
-  // 8.41 -> 8.30 ms at the benchmark shape); with a block per tile the flags alone do
+  // 8.41 -> 8.30 ms at the benchmark shape); with a block (or wavefront) per tile the flags alone do
   a.tile_busy = tile_flags;
-  if (n_tiles > n_blocks) {
+  if (n_tiles > (int64_t)n_blocks * (view ? ffn::MLP_VIEW_WAVES : 1)) {
     a.tile_order = tile_order;
     a.n_busy = tile_order + n_tiles;
   }
@@ -818,6 +819,8 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
     if (a.tile_order) FFN_HIP(ffn::launch_tile_order(n_tiles, tile_flags, tile_order, tile_order + n_tiles, st));
     if (mlp16)
       FFN_HIP(ffn::launch_mlp16(a, LF, h->cfg.nd, h->cfg.nc, n_blocks, st));
+    else if (view)
+      FFN_HIP(ffn::launch_mlp_view(a, LF, h->cfg.nd, h->cfg.nc, n_blocks, st));
     else
       FFN_HIP(ffn::launch_mlp(a, LF, h->cfg.nd, h->cfg.nc, n_blocks, st));
   }
@@ -1124,9 +1127,9 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
   // as for the kept count, the further blocks add zero partials.)
   const int64_t n_tiles = (n + 63) / 64;
   const int n_blocks = grid_blocks(h, mlp16 ? ffn::mlp16_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, true)
-                                             : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc, true), n_tiles);
-  const int fwd_blocks = grid_blocks(h, mlp16 ? ffn::mlp16_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc)
-                                               : ffn::mlp_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), n_tiles);
+                                             : ffn::mlp_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), n_tiles);
+  const int fwd_blocks = mlp16 ? grid_blocks(h, ffn::mlp16_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), n_tiles)
+                               : grid_blocks(h, 1, (n + 15) / 16);
   FFN_HIP(h->partials.ensure(sizeof(float) * (size_t)n_blocks * h->lay.total));
   const ffn::MlpPtrs w = mlp_ptrs(P);
   {
@@ -1341,7 +1344,7 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
     src.x_stride = 4;
     const ffn::FeatLayout feat = ffn::level_major(n, h->dc.F);
     FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, a0, feat, nullptr, &dl, st, n_dev));
-    const int nb = grid_blocks(h, ffn::mlp_fwd_blocks_per_cu(LF, h->cfg.nd, h->cfg.nc), (n + 63) / 64);
+    const int nb = grid_blocks(h, 1, (n + 15) / 16);
     FFN_HIP(ffn::launch_mlp_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, mp->sh_multiplier, sigma, rgb, LF,
                                 h->cfg.nd, h->cfg.nc, nb, st, n_dev));
     FFN_HIP(ffn::launch_render_composite(off, counts, num_rays, sigma, rgb, mp->dt, mp->T_stop, state, acc,

@@ -112,7 +112,8 @@ struct MlpArgs {
   // with tile_order: the number of busy tiles (a sample with dt > 0), which the order puts first; the
   // kernels composite the later positions' tiles to the background without the MLP
   const uint32_t* n_busy;
-  // without tile_order (a block per tile at most): byte t = tile t is busy (NULL: every tile takes the full path)
+  // without tile_order (a block, or a wavefront of launch_mlp_view, per tile at most): byte t = tile t is busy
+  // (NULL: every tile takes the full path)
   const uint8_t* tile_busy;
   float sh_mult, occ_strength;
   uint32_t seed;
@@ -339,12 +340,15 @@ hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, co
 
 // fused MLP forward + compositing + loss + backward + proposals, per 64-sample tile
 bool mlp_supported(int LF, int nd, int nc);
-// blocks of launch_mlp / launch_mlp16 that run on one CU (training, or forward-only), and of the forward over
-// indexed samples
-int mlp_blocks_per_cu(int LF, int nd, int nc, bool train);
+// blocks of launch_mlp / launch_mlp16 that run on one CU (launch_mlp16: training, or forward-only), and of its
+// forward over indexed samples
+int mlp_blocks_per_cu(int LF, int nd, int nc);
 int mlp16_blocks_per_cu(int LF, int nd, int nc, bool train);
-int mlp_fwd_blocks_per_cu(int LF, int nd, int nc);
 int mlp16_fwd_blocks_per_cu(int LF, int nd, int nc);
+// launch_mlp for a forward-only step, and launch_mlp_fwd: blocks of MLP_VIEW_WAVES wavefronts, one per CU; a
+// wavefront takes a tile of 64 samples (16 samples) at a time
+constexpr int MLP_VIEW_WAVES = 16;
+hipError_t launch_mlp_view(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st);
 hipError_t launch_mlp(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st);
 // order[n_tiles]: the tiles whose byte in flags (launch_sample's tile_busy; 16-byte aligned) is 1 in index order,
 // then the others; *n_busy: how many are

@@ -70,26 +70,11 @@ struct Arch {
   static constexpr int g_total() { return g_off(FFN_N_LAYERS); }
   static constexpr int PSF = 64 + 4;       // stash pitch: 64 sample columns + 4 pad (conflict-free b128 reads)
   static constexpr int stash_rows = 128;   // one layer's delta rows (<= 64) + input activation rows (<= 64)
-  // sigma[64] + rgb[64][3] of the tile: one slot when training (the stash barriers separate a tile's
-  // compositing from the next tile's writes), two alternating slots for a forward-only launch
-  static constexpr int comp_floats(bool train) { return train ? 256 : 512; }
-  // a forward-only launch has no stash
-  static constexpr int lds_floats(bool train) {
-    return w_total() + (train ? stash_rows * PSF : 0) + comp_floats(train);
-  }
-  // Training: two blocks per CU when the LDS allows it (160 KiB per CU).  Forward-only: as many as its LDS allows
-  // up to four (five wavefronts per SIMD fit its registers): at 64 encoded features and two density layers two
-  // blocks instead of one, a preview of 9216 rays 219 -> 166 us.
-  static constexpr int blocks_per_cu(bool train) {
-    const int fit = 160 * 1024 / (lds_floats(train) * 4);
-    const int most = train ? 2 : 4;
-    return fit < 1 ? 1 : (fit < most ? fit : most);
-  }
-  // k_mlp_fwd holds the weights alone
-  static constexpr int fwd_blocks_per_cu() {
-    const int fit = 160 * 1024 / (w_total() * 4);
-    return fit < 1 ? 1 : (fit < 4 ? fit : 4);
-  }
+  // sigma[64] + rgb[64][3] of the tile (the stash barriers separate a tile's compositing from the next tile's
+  // writes)
+  static constexpr int lds_floats() { return w_total() + stash_rows * PSF + 256; }
+  // two blocks per CU when the LDS allows it (160 KiB per CU)
+  static constexpr int blocks_per_cu() { return lds_floats() * 4 <= 80 * 1024 ? 2 : 1; }
 };
 
 // out tiles (D layout) = act(W . in + b), in given as D-layout tiles.  The
@@ -349,63 +334,6 @@ __device__ __forceinline__ void stage_weights(float* __restrict__ sW, const MlpP
   if (tid >= layer_out(k) && tid < A::rows_pad(k)) sW[A::b_off(k) + tid] = 0.0f;
 }
 
-// a0r[kk] = encoding neuron (LF/4) g + kk (= level n / F, feature n % F) of sample b
-template <int LF, int FEAT>
-__device__ __forceinline__ void load_a0(const float* __restrict__ a0, const FeatLayout& feat, int64_t b, bool valid,
-                                        int g, float (&a0r)[LF / 4]) {
-  constexpr int KA = LF / 4;
-  if (valid) {
-    if constexpr (FEAT >= 2 && KA % 2 == 0) {
-#pragma unroll
-      for (int kk = 0; kk < KA; kk += 2) {
-        const int nn = KA * g + kk;
-        const int l = nn / FEAT, f = nn - l * FEAT;
-        const float2 v = *reinterpret_cast<const float2*>(a0 + l * feat.stride_l + b * feat.stride_b + f);
-        a0r[kk] = v.x;
-        a0r[kk + 1] = v.y;
-      }
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < KA; ++kk) {
-        const int nn = KA * g + kk;
-        const int l = nn / FEAT, f = nn - l * FEAT;
-        a0r[kk] = a0[l * feat.stride_l + b * feat.stride_b + f];
-      }
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < KA; ++q) a0r[q] = 0.0f;
-  }
-}
-
-// The colour output layer's forward (three rows of 64 inputs) on v_mfma_f32_4x4x1f32, whose 16 blocks of
-// four lanes each add a 4x4 outer product (block b: lane 4b + i supplies row i of A, lane 4b + j column j of
-// B, and lane 4b + j receives column j in its four registers; pinned by a probe).  Lane (g, s) is lane j =
-// s % 4 of block 4g + s / 4: it supplies weight row s % 4 (row 3 is the padding's zero row) of input unit
-// 16t + 4g + r and the activation of that unit for its sample, so after the 16 (t, r) steps it holds lane
-// group g's share of its sample's three outputs (and a zero fourth); two row swaps sum the four groups.
-// 16 instructions of 8 cycles where the padded 16-row tile took 16 of 32.  Every lane gets its sample's
-// colours.
-__device__ __forceinline__ void fwd_color_out(const float* __restrict__ W, const float* __restrict__ B, int P,
-                                              const floatx4 (&act)[4], int g, int s, float (&rgb)[3]) {
-  floatx4 part = {0.f, 0.f, 0.f, 0.f};
-  const float* wrow = W + (s & 3) * P + 4 * g;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const floatx4 w4 = *reinterpret_cast<const floatx4*>(wrow + 16 * t);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) part = __builtin_amdgcn_mfma_f32_4x4x1f32(w4[r], act[t][r], part, 0, 0, 0);
-  }
-#pragma unroll
-  for (int o = 0; o < 3; ++o) {
-    const int x = __float_as_int(part[o]);
-    const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);  // {lower half twice, upper half twice}
-    const int y = __float_as_int(__int_as_float((int)h[0]) + __int_as_float((int)h[1]));
-    const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);  // {even rows twice, odd rows twice}
-    rgb[o] = sigmoid_soft((__int_as_float((int)q[0]) + __int_as_float((int)q[1])) + B[o]);
-  }
-}
-
 // forward of the wavefront's 16 samples through both MLPs (ffnerf_OG.cl:1373-1466): hidden activations
 // (kept for the backward), the colour-net input [dout | SH * mult] and the sigmoid colours
 template <int LF, int ND, int NC>
@@ -464,23 +392,21 @@ __device__ __forceinline__ void mlp_fwd_tile(const float* __restrict__ sW, const
 }
 
 // MARCHED: the backward over marched samples -- sample b is a.smp[b] of ray a.ray_ids[b], its loss gradients
-// are read (a.in_dLds, a.in_dLdc), and there is no compositing and no proposal.  TRAIN (a.do_train) is a
-// template parameter: a forward-only tile leaves the loop after its compositing, and that exit, taken at run
-// time, made the register allocator copy the activations and gradient accumulators (90 moves per tile) on
-// the training path too.
-template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC, bool TRAIN>
-__global__ __launch_bounds__(256, (TRAIN ? Arch<LF, ND, NC>::blocks_per_cu(true) : 4)) void k_mlp(MlpArgs a) {
-  static_assert(TRAIN || !MARCHED, "marched launches train");
+// are read (a.in_dLds, a.in_dLdc), and there is no compositing and no proposal.  Training only: a forward-only
+// launch is k_mlp_view (an exit from the tile after its compositing, taken at run time, made the register
+// allocator copy the activations and gradient accumulators, 90 moves per tile, on the training path too).
+template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC>
+__global__ __launch_bounds__(256, (Arch<LF, ND, NC>::blocks_per_cu())) void k_mlp(MlpArgs a) {
   using A = Arch<LF, ND, NC>;
   constexpr int KA = LF / 4;  // a0 values per lane (k-steps of the first layer)
   constexpr int PSF = A::PSF;
   extern __shared__ float smem[];
   float* sW = smem;
   float* sS = smem + A::w_total();            // per-layer stash of deltas and activations
-  float* sC = sS + (TRAIN ? A::stash_rows * A::PSF : 0);  // compositing inputs (double-buffered when forward-only)
+  float* sC = sS + A::stash_rows * A::PSF;    // compositing inputs
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
   const int col = wave * 16 + s;              // this lane's stash column
-  constexpr bool train = TRAIN;
+  constexpr bool train = true;
   const DevCfg& c = a.c;
   const int log2S = a.log2S;
   uint64_t n_samples = (uint64_t)a.num_rays << log2S;
@@ -495,7 +421,6 @@ __global__ __launch_bounds__(256, (TRAIN ? Arch<LF, ND, NC>::blocks_per_cu(true)
   __syncthreads();
 
   const float Dhalf = half_box_diagonal(c);
-  constexpr bool taps = TAPS;
   const bool proposals = train && a.occ_strength > 0.0f;
 
   WaveGrad<1, 4> gc_out;
@@ -540,7 +465,7 @@ __global__ __launch_bounds__(256, (TRAIN ? Arch<LF, ND, NC>::blocks_per_cu(true)
     else __builtin_amdgcn_s_setprio(1);
     __builtin_amdgcn_sched_barrier(0);  // the turn starts here (the scheduler would sink it to the forward's end)
     const int64_t tile = a.tile_order ? (int64_t)a.tile_order[ti] : ti;
-    float* sSig = sC + (train ? 0 : parity * 256);
+    float* sSig = sC;
     float* sRgb = sSig + 64;
     // ------------------------------------------------------------------
     // forward: this lane's sample in the MLP layout
@@ -548,7 +473,7 @@ __global__ __launch_bounds__(256, (TRAIN ? Arch<LF, ND, NC>::blocks_per_cu(true)
     const bool valid = (uint64_t)b < n_samples;
     const int64_t ray = valid ? (MARCHED ? (int64_t)a.ray_ids[b] : (b >> log2S)) : 0;
     float a0r[KA];
-    load_a0<LF, FEAT>(a.a0, a.feat, b, valid, g, a0r);
+    load_enc<LF, FEAT>(a.a0, a.feat, b, valid, g, a0r);
     float dirv[3];
     {
       const float4 rd = a.rays[2 * ray + 1];
@@ -608,17 +533,14 @@ __global__ __launch_bounds__(256, (TRAIN ? Arch<LF, ND, NC>::blocks_per_cu(true)
         float dLds_j, dLdc_j[3];
         __builtin_amdgcn_s_setprio(3);
         composite_tile<TAPS, SC>(a, sSig, sRgb, CL, lane, 0, true, train, proposals, Dhalf, dLds_j, dLdc_j);
-        if (train) {
-          sSig[lane] = dLds_j;
-          sRgb[3 * lane] = dLdc_j[0];
-          sRgb[3 * lane + 1] = dLdc_j[1];
-          sRgb[3 * lane + 2] = dLdc_j[2];
-        }
+        sSig[lane] = dLds_j;
+        sRgb[3 * lane] = dLdc_j[0];
+        sRgb[3 * lane + 1] = dLdc_j[1];
+        sRgb[3 * lane + 2] = dLdc_j[2];
       }
       // the tile's second turn: the block that led the forward yields the backward
       if (gang_hi) __builtin_amdgcn_s_setprio(1);
       else __builtin_amdgcn_s_setprio(2);
-      if (!train) continue;
       __syncthreads();
       dLds = sSig[col];
       dLdc0 = sRgb[3 * col];
@@ -718,46 +640,34 @@ __global__ __launch_bounds__(256, (TRAIN ? Arch<LF, ND, NC>::blocks_per_cu(true)
     }
   }
 
-  if (train) {
-    // every wavefront stores its tiles into the block's partial gradient
-    float* dst = a.partials + (int64_t)blockIdx.x * A::g_total();
-    flush_color_out(dst + A::g_off(FFN_WC_OUT), gc_out, wave, lane);
-    if constexpr (NC >= 2) flush_layer(dst + A::g_off(FFN_WC_01), FFN_M, FFN_M, gc_h[0], wave, g, s);
-    if constexpr (NC >= 3) flush_layer(dst + A::g_off(FFN_WC_12), FFN_M, FFN_M, gc_h[1], wave, g, s);
-    if constexpr (NC >= 4) flush_layer(dst + A::g_off(FFN_WC_23), FFN_M, FFN_M, gc_h[2], wave, g, s);
-    flush_layer(dst + A::g_off(FFN_WC_IN), FFN_M, FFN_C_IN, gc_in, wave, g, s);
-    flush_layer(dst + A::g_off(FFN_WD_OUT), FFN_D_OUT, FFN_M, gd_out, wave, g, s);
-    if constexpr (ND >= 2) flush_layer(dst + A::g_off(FFN_WD_01), FFN_M, FFN_M, gd_h[0], wave, g, s);
-    if constexpr (ND >= 3) flush_layer(dst + A::g_off(FFN_WD_12), FFN_M, FFN_M, gd_h[1], wave, g, s);
-    flush_layer(dst + A::g_off(FFN_WD_IN), FFN_M, LF, gd_in, wave, g, s);
-  }
+  // every wavefront stores its tiles into the block's partial gradient
+  float* dst = a.partials + (int64_t)blockIdx.x * A::g_total();
+  flush_color_out(dst + A::g_off(FFN_WC_OUT), gc_out, wave, lane);
+  if constexpr (NC >= 2) flush_layer(dst + A::g_off(FFN_WC_01), FFN_M, FFN_M, gc_h[0], wave, g, s);
+  if constexpr (NC >= 3) flush_layer(dst + A::g_off(FFN_WC_12), FFN_M, FFN_M, gc_h[1], wave, g, s);
+  if constexpr (NC >= 4) flush_layer(dst + A::g_off(FFN_WC_23), FFN_M, FFN_M, gc_h[2], wave, g, s);
+  flush_layer(dst + A::g_off(FFN_WC_IN), FFN_M, FFN_C_IN, gc_in, wave, g, s);
+  flush_layer(dst + A::g_off(FFN_WD_OUT), FFN_D_OUT, FFN_M, gd_out, wave, g, s);
+  if constexpr (ND >= 2) flush_layer(dst + A::g_off(FFN_WD_01), FFN_M, FFN_M, gd_h[0], wave, g, s);
+  if constexpr (ND >= 3) flush_layer(dst + A::g_off(FFN_WD_12), FFN_M, FFN_M, gd_h[1], wave, g, s);
+  flush_layer(dst + A::g_off(FFN_WD_IN), FFN_M, LF, gd_in, wave, g, s);
 }
 
 // ---------------------------------------------------------------------------
 
-template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC, bool TRAIN>
-static hipError_t launch_k(const MlpArgs& a, int n_blocks, hipStream_t st) {
+template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC>
+static hipError_t launch_f(const MlpArgs& a, int n_blocks, hipStream_t st) {
   using A = Arch<LF, ND, NC>;
-  const size_t lds = sizeof(float) * (size_t)A::lds_floats(TRAIN);
+  const size_t lds = sizeof(float) * (size_t)A::lds_floats();
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)k_mlp<LF, ND, NC, FEAT, TAPS, MARCHED, SC, TRAIN>,
+    hipError_t e = hipFuncSetAttribute((const void*)k_mlp<LF, ND, NC, FEAT, TAPS, MARCHED, SC>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
-  hipLaunchKernelGGL((k_mlp<LF, ND, NC, FEAT, TAPS, MARCHED, SC, TRAIN>), dim3(n_blocks), dim3(256), lds, st, a);
+  hipLaunchKernelGGL((k_mlp<LF, ND, NC, FEAT, TAPS, MARCHED, SC>), dim3(n_blocks), dim3(256), lds, st, a);
   return hipGetLastError();
-}
-
-template <int LF, int ND, int NC, int FEAT, bool TAPS, bool MARCHED, int SC>
-static hipError_t launch_f(const MlpArgs& a, int n_blocks, hipStream_t st) {
-  if constexpr (MARCHED) {
-    return launch_k<LF, ND, NC, FEAT, TAPS, true, SC, true>(a, n_blocks, st);
-  } else {
-    return a.do_train ? launch_k<LF, ND, NC, FEAT, TAPS, false, SC, true>(a, n_blocks, st)
-                      : launch_k<LF, ND, NC, FEAT, TAPS, false, SC, false>(a, n_blocks, st);
-  }
 }
 
 template <int LF, int ND, int NC, bool MARCHED, int SC>
@@ -773,78 +683,6 @@ static hipError_t launch_t(const MlpArgs& a, int n_blocks, hipStream_t st) {
     case 4:
       return taps ? launch_f<LF, ND, NC, 4, true, MARCHED, SC>(a, n_blocks, st)
                   : launch_f<LF, ND, NC, 4, false, MARCHED, SC>(a, n_blocks, st);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-// forward only, over a flat list of samples (the render path): 16 samples per wavefront per step
-template <int LF, int ND, int NC, int FEAT>
-__global__ __launch_bounds__(256) void k_mlp_fwd(MlpPtrs wp, const float* __restrict__ a0, FeatLayout feat,
-                                                 const float4* __restrict__ rays, const uint32_t* __restrict__ ray_ids,
-                                                 int64_t n, float sh_mult, float* __restrict__ sigma,
-                                                 float* __restrict__ rgb, const uint32_t* __restrict__ n_dev) {
-  extern __shared__ float smem[];
-  if (n_dev) {  // the count of a launch sized for a capacity, read on the device
-    const int64_t nd = (int64_t)*n_dev;
-    n = nd < n ? nd : n;
-  }
-  if ((int64_t)blockIdx.x * 64 >= n) return;  // no samples for this block: skip staging the weights
-  float* sW = smem;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
-  stage_weights<LF, ND, NC>(sW, wp, tid);
-  __syncthreads();
-  for (int64_t grp = (int64_t)blockIdx.x * 4 + wave; grp * 16 < n; grp += (int64_t)gridDim.x * 4) {
-    const int64_t b = grp * 16 + s;
-    const bool valid = b < n;
-    float a0r[LF / 4];
-    load_a0<LF, FEAT>(a0, feat, b, valid, g, a0r);
-    float dirv[3] = {0.0f, 0.0f, 1.0f};
-    if (valid) {
-      const float4 rd = rays[2 * (size_t)ray_ids[b] + 1];
-      dirv[0] = rd.x;
-      dirv[1] = rd.y;
-      dirv[2] = rd.z;
-    }
-    floatx4 hd[ND][4];
-    floatx4 acin[2];
-    floatx4 hc[NC][4];
-    float rgb_s[3];
-    mlp_fwd_tile<LF, ND, NC>(sW, a0r, dirv, sh_mult, g, s, hd, acin, hc, rgb_s);
-    if (g == 0 && valid) {
-      sigma[b] = softplus(fminf(fmaxf(acin[0][0], -10.0f), 10.0f));
-      rgb[3 * b] = rgb_s[0];
-      rgb[3 * b + 1] = rgb_s[1];
-      rgb[3 * b + 2] = rgb_s[2];
-    }
-  }
-}
-
-template <int LF, int ND, int NC, int FEAT>
-static hipError_t launch_fwd_f(const MlpPtrs& w, const float* a0, const FeatLayout& feat, const float4* rays,
-                               const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma, float* rgb,
-                               int n_blocks, hipStream_t st, const uint32_t* n_dev) {
-  using A = Arch<LF, ND, NC>;
-  const size_t lds = sizeof(float) * (size_t)A::w_total();
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_fwd<LF, ND, NC, FEAT>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
-  hipLaunchKernelGGL((k_mlp_fwd<LF, ND, NC, FEAT>), dim3(n_blocks), dim3(256), lds, st, w, a0, feat, rays, ray_ids, n,
-                     sh_mult, sigma, rgb, n_dev);
-  return hipGetLastError();
-}
-
-template <int LF, int ND, int NC>
-static hipError_t launch_fwd_t(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
-                               const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
-                               float* rgb, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
-  switch (c.F) {
-    case 1: return launch_fwd_f<LF, ND, NC, 1>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
-    case 2: return launch_fwd_f<LF, ND, NC, 2>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
-    case 4: return launch_fwd_f<LF, ND, NC, 4>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
     default: return hipErrorInvalidValue;
   }
 }
@@ -865,32 +703,12 @@ bool mlp_supported(int LF, int nd, int nc) {
   return false;
 }
 
-int mlp_blocks_per_cu(int LF, int nd, int nc, bool train) {
+int mlp_blocks_per_cu(int LF, int nd, int nc) {
 #define X(l, d, n) \
-  if (LF == l && nd == d && nc == n) return Arch<l, d, n>::blocks_per_cu(train);
+  if (LF == l && nd == d && nc == n) return Arch<l, d, n>::blocks_per_cu();
   FFN_MLP_CONFIGS(X)
 #undef X
   return 1;
-}
-
-int mlp_fwd_blocks_per_cu(int LF, int nd, int nc) {
-#define X(l, d, n) \
-  if (LF == l && nd == d && nc == n) return Arch<l, d, n>::fwd_blocks_per_cu();
-  FFN_MLP_CONFIGS(X)
-#undef X
-  return 1;
-}
-
-hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
-                          const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
-                          float* rgb, int LF, int nd, int nc, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
-  if (n <= 0) return hipSuccess;
-#define X(l, d, nn)                   \
-  if (LF == l && nd == d && nc == nn) \
-    return launch_fwd_t<l, d, nn>(c, w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
-  FFN_MLP_CONFIGS(X)
-#undef X
-  return hipErrorInvalidValue;
 }
 
 // Tile order of a step: the sampler flags each 64-sample tile with a sample of dt > 0 (the tiles the MLP
@@ -969,6 +787,7 @@ hipError_t launch_tile_order(int64_t n_tiles, const uint8_t* flags, uint32_t* or
 }
 
 hipError_t launch_mlp(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st) {
+  if (!a.do_train) return hipErrorInvalidValue;  // launch_mlp_view
 #define X(l, d, n) \
   if (LF == l && nd == d && nc == n)                                                         \
     return a.S == 64 ? launch_t<l, d, n, false, 64>(a, n_blocks, st) : launch_t<l, d, n, false, 0>(a, n_blocks, st);

@@ -74,6 +74,63 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// a0r[kk] = encoding neuron (LF/4) g + kk (= level n / F, feature n % F) of sample b
+template <int LF, int FEAT>
+__device__ __forceinline__ void load_enc(const float* __restrict__ a0, const FeatLayout& feat, int64_t b, bool valid,
+                                        int g, float (&a0r)[LF / 4]) {
+  constexpr int KA = LF / 4;
+  if (valid) {
+    if constexpr (FEAT >= 2 && KA % 2 == 0) {
+#pragma unroll
+      for (int kk = 0; kk < KA; kk += 2) {
+        const int nn = KA * g + kk;
+        const int l = nn / FEAT, f = nn - l * FEAT;
+        const float2 v = *reinterpret_cast<const float2*>(a0 + l * feat.stride_l + b * feat.stride_b + f);
+        a0r[kk] = v.x;
+        a0r[kk + 1] = v.y;
+      }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < KA; ++kk) {
+        const int nn = KA * g + kk;
+        const int l = nn / FEAT, f = nn - l * FEAT;
+        a0r[kk] = a0[l * feat.stride_l + b * feat.stride_b + f];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < KA; ++q) a0r[q] = 0.0f;
+  }
+}
+
+// The colour output layer's forward (three rows of 64 inputs) on v_mfma_f32_4x4x1f32, whose 16 blocks of
+// four lanes each add a 4x4 outer product (block b: lane 4b + i supplies row i of A, lane 4b + j column j of
+// B, and lane 4b + j receives column j in its four registers; pinned by a probe).  Lane (g, s) is lane j =
+// s % 4 of block 4g + s / 4: it supplies weight row s % 4 (row 3 is the padding's zero row) of input unit
+// 16t + 4g + r and the activation of that unit for its sample, so after the 16 (t, r) steps it holds lane
+// group g's share of its sample's three outputs (and a zero fourth); two row swaps sum the four groups.
+// 16 instructions of 8 cycles where the padded 16-row tile took 16 of 32.  Every lane gets its sample's
+// colours.
+__device__ __forceinline__ void fwd_color_out(const float* __restrict__ W, const float* __restrict__ B, int P,
+                                              const floatx4 (&act)[4], int g, int s, float (&rgb)[3]) {
+  floatx4 part = {0.f, 0.f, 0.f, 0.f};
+  const float* wrow = W + (s & 3) * P + 4 * g;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const floatx4 w4 = *reinterpret_cast<const floatx4*>(wrow + 16 * t);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part = __builtin_amdgcn_mfma_f32_4x4x1f32(w4[r], act[t][r], part, 0, 0, 0);
+  }
+#pragma unroll
+  for (int o = 0; o < 3; ++o) {
+    const int x = __float_as_int(part[o]);
+    const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);  // {lower half twice, upper half twice}
+    const int y = __float_as_int(__int_as_float((int)h[0]) + __int_as_float((int)h[1]));
+    const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);  // {even rows twice, odd rows twice}
+    rgb[o] = sigmoid_soft((__int_as_float((int)q[0]) + __int_as_float((int)q[1])) + B[o]);
+  }
+}
+
 // the background colour of ray rj (black, white, or the seeded random colour while training;
 // ffnerf_OG.cl:1534-1541)
 __device__ __forceinline__ void background(const MlpArgs& a, int64_t rj, bool train, float (&bg)[3]) {

@@ -1,0 +1,516 @@
+// ffn_mlp_fwd.hip -- the fp32 networks' forward: forward-only steps (previews, snapshots) and the forward over
+// indexed samples (the marched render and the marched step's compositing input).
+//
+// Reference: ffnerf_OG.cl:1373-1466 (MLP fwd), 1505-1591 (compositing).
+//
+// MI355X design
+//   * Every fp32 value x of a product is the exact sum of three bfloat16 values: h = x's top 16 bits, m = the top
+//     16 bits of x - h, l = x - h - m (8 + 8 + 8 significand bits; the differences are exact).  A product a b is the
+//     six terms a_h b_h + a_h b_m + a_m b_h + a_m b_m + a_h b_l + a_l b_h, each exact on
+//     v_mfma_f32_16x16x32_bf16, which adds 32 products to its fp32 accumulator with one rounding; the three terms
+//     left out are below 2^-23 of a b together.  Against 64-bit sums of 32 random products: relative error 4.2e-8
+//     (fp32 MFMAs, eight of K = 4 in a chain, 1.04e-7); on outputs that pass a ReLU 4.4e-8 (7.7e-8).  Six K = 32
+//     instructions of 16 cycles do the work of eight fp32 ones of 32, and unlike those they run beside vector
+//     instructions.
+//   * A block of 16 wavefronts, one per CU, shares the weights in LDS (three bfloat16 planes, K-ordered rows); a
+//     wavefront works alone (no barrier after the staging): 16 samples through all layers, activations in registers
+//     in the D layout of one layer = the B operand of the next (K slot j of lane group g in block kb is neuron
+//     32 kb + 16 (j / 4) + 4 g + j % 4).  A forward-only step's wavefront takes a tile of 64 samples as four such
+//     groups and composites it on its 64 lanes.
+//   * What bounds it: matrix instructions and the vector instructions of the splits (5.5 per value) about alike.
+//     Measured against the fp32-MFMA forward (three blocks of four wavefronts per CU, 16-byte weight staging):
+//     880,000 marched samples of the 32-feature model 167 -> 108 us, a frame's first round of 3.0M samples 542 ->
+//     347; a preview of 590,000 samples of the 64-feature model with two density layers 166 -> 97 us.
+//   * An infinite value's m is not a number, so its split products are none either where the value's own products
+//     would be infinities.  The wavefront sees that in its sums (every sum of a sample with such a value is not a
+//     number) or, for a weight, when it is staged, and redoes those samples with plain fp32 products.
+#include "ffn_device.h"
+#include "ffn_kernels.h"
+#include "ffn_mlp_common.h"
+
+namespace ffn {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int VIEW_NT = 64 * MLP_VIEW_WAVES;
+
+template <int LF_, int ND_, int NC_>
+struct ArchF {
+  static constexpr int LF = LF_, ND = ND_, NC = NC_;
+  // layers on the split products (the colour output layer's three rows stay on fp32 4x4x1 MFMAs)
+  static constexpr bool split(int k) { return layer_active(k, ND, NC) && k != FFN_WC_OUT; }
+  static constexpr int cols(int k) { return layer_in(k, LF) < 32 ? 32 : layer_in(k, LF); }
+  // row pitch in halves: the 8-half pad keeps the 16-byte reads aligned and spreads a tile's rows over the banks
+  static constexpr int pitch(int k) { return cols(k) + 8; }
+  static constexpr int sz(int k) { return split(k) ? layer_out(k) * pitch(k) : 0; }
+  static constexpr int w_off(int k) {  // of plane 0, in halves; plane p follows at p * plane()
+    int o = 0;
+    for (int j = 0; j < k; ++j) o += sz(j);
+    return o;
+  }
+  static constexpr int plane() { return w_off(FFN_N_LAYERS); }
+  static constexpr int OUT_P = FFN_M + 4;  // the colour output layer: four fp32 rows (the last one zero)
+  static constexpr int out_off() { return 3 * plane() / 2; }  // in floats
+  static constexpr int b_off(int k) {
+    int o = out_off() + 4 * OUT_P;
+    for (int j = 0; j < k; ++j) o += layer_active(j, ND, NC) ? (j == FFN_WC_OUT ? 4 : layer_out(j)) : 0;
+    return o;
+  }
+  static constexpr int w_floats() { return b_off(FFN_N_LAYERS); }
+  static_assert(plane() % 8 == 0, "16-byte aligned planes");
+};
+
+// position of input neuron n in a layer's K-ordered row: for the first layer lane group g holds neurons (LF / 4) g
+// + kk as slots kk of its K blocks (LF = 16: slots 0 .. 3 of one block), for the others see the file comment
+template <int LF, int K>
+__device__ __forceinline__ constexpr int row_pos(int n) {
+  if constexpr (K == FFN_WD_IN) {
+    constexpr int KA = LF / 4;
+    const int g = n / KA, kk = n % KA;
+    return 32 * (kk / 8) + 8 * g + kk % 8;
+  } else {
+    return (n & ~31) + 8 * ((n >> 2) & 3) + 4 * ((n >> 4) & 1) + (n & 3);
+  }
+}
+
+__device__ __forceinline__ float top16(float x) { return __int_as_float(__float_as_int(x) & (int)0xFFFF0000); }
+// {x1's upper half, x0's upper half}
+__device__ __forceinline__ uint32_t upper_halves(float x1, float x0) {
+  return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+}
+
+// eight values of a K block, as three bfloat16 operands
+struct Split8 {
+  bf16x8 h, m, l;
+};
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float x0 = x[2 * q], x1 = x[2 * q + 1];
+    const float r0 = x0 - top16(x0), r1 = x1 - top16(x1);
+    const float l0 = r0 - top16(r0), l1 = r1 - top16(r1);
+    h[q] = upper_halves(x1, x0);
+    m[q] = upper_halves(r1, r0);
+    l[q] = upper_halves(l1, l0);
+  }
+  Split8 s;
+  s.h = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
+  s.m = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
+  s.l = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+  return s;
+}
+// the K blocks of D-layout tiles
+template <int IT>
+__device__ __forceinline__ void split_tiles(const floatx4 (&t)[IT], Split8 (&o)[IT / 2]) {
+#pragma unroll
+  for (int kb = 0; kb < IT / 2; ++kb) {
+    const float x[8] = {t[2 * kb][0],     t[2 * kb][1],     t[2 * kb][2],     t[2 * kb][3],
+                        t[2 * kb + 1][0], t[2 * kb + 1][1], t[2 * kb + 1][2], t[2 * kb + 1][3]};
+    o[kb] = split8(x);
+  }
+}
+
+// out tiles (D layout) = act(W . in + b), two output tiles at a time so that consecutive MFMAs are independent;
+// bad becomes not a number where the sample's sums are infinite or not numbers
+template <int OT, int KB>
+__device__ __forceinline__ void fwd_split(const __bf16* __restrict__ W, int plane, int P, const float* __restrict__ B,
+                                          const Split8 (&in)[KB], floatx4 (&out)[OT], int g, int s, bool relu,
+                                          float& bad) {
+  const __bf16* wrow = W + s * P + 8 * g;
+  constexpr int G = OT < 2 ? OT : 2;
+#pragma unroll
+  for (int t0 = 0; t0 < OT; t0 += G) {
+    floatx4 acc[G];
+#pragma unroll
+    for (int t = 0; t < G; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[t][r] = B[16 * (t0 + t) + 4 * g + r];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      bf16x8 wh[G], wm[G], wl[G];
+#pragma unroll
+      for (int t = 0; t < G; ++t) {
+        const __bf16* w = wrow + 16 * (t0 + t) * P + 32 * kb;
+        wh[t] = *reinterpret_cast<const bf16x8*>(w);
+        wm[t] = *reinterpret_cast<const bf16x8*>(w + plane);
+        wl[t] = *reinterpret_cast<const bf16x8*>(w + 2 * plane);
+      }
+      auto term = [&](const bf16x8 (&w)[G], const bf16x8& x) {
+#pragma unroll
+        for (int t = 0; t < G; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], x, acc[t], 0, 0, 0);
+      };
+      term(wl, in[kb].h);
+      term(wh, in[kb].l);
+      term(wm, in[kb].m);
+      term(wm, in[kb].h);
+      term(wh, in[kb].m);
+      term(wh, in[kb].h);
+    }
+    if (t0 == 0) bad = fmaf(acc[0][0], 0.0f, bad);
+#pragma unroll
+    for (int t = 0; t < G; ++t) {
+      if (relu) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[t][r] = relu_f(acc[t][r]);
+      }
+      out[t0 + t] = acc[t];
+    }
+  }
+}
+
+// stage the weights into LDS (split into planes) and the biases; returns whether this thread's weights are all finite
+template <int LF, int ND, int NC>
+__device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtrs& wp, int tid) {
+  using A = ArchF<LF, ND, NC>;
+  __bf16* sW = reinterpret_cast<__bf16*>(sm);
+  float bad = 0.0f;
+  read_weights<LF, ND, NC, VIEW_NT>(
+      wp, tid,
+      [&](auto K, int o, int i, const float4& v) {
+        constexpr int k = K;
+        if constexpr (k == FFN_WC_OUT) {
+          *reinterpret_cast<float4*>(sm + A::out_off() + o * A::OUT_P + i) = v;
+        } else {
+          const float x[4] = {v.x, v.y, v.z, v.w};
+          float r[4], l[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            r[q] = x[q] - top16(x[q]);
+            l[q] = r[q] - top16(r[q]);
+            bad = fmaf(x[q], 0.0f, bad);
+          }
+          __bf16* w = sW + A::w_off(k) + o * A::pitch(k) + row_pos<LF, k>(i);  // four consecutive positions
+          *reinterpret_cast<uint2*>(w) = make_uint2(upper_halves(x[1], x[0]), upper_halves(x[3], x[2]));
+          *reinterpret_cast<uint2*>(w + A::plane()) = make_uint2(upper_halves(r[1], r[0]), upper_halves(r[3], r[2]));
+          *reinterpret_cast<uint2*>(w + 2 * A::plane()) =
+              make_uint2(upper_halves(l[1], l[0]), upper_halves(l[3], l[2]));
+        }
+      },
+      [&](auto K, int o, float v) { sm[A::b_off(K) + o] = v; });
+  if (tid < A::OUT_P) sm[A::out_off() + 3 * A::OUT_P + tid] = 0.0f;
+  if constexpr (LF == 16) {  // the first layer's rows have 16 neurons in 32 positions
+    constexpr int P = A::pitch(FFN_WD_IN);
+    for (int e = tid; e < 3 * FFN_M * 4; e += VIEW_NT) {
+      const int p = e / (FFN_M * 4), o = (e >> 2) % FFN_M, g = e & 3;
+      *reinterpret_cast<uint2*>(sW + p * A::plane() + A::w_off(FFN_WD_IN) + o * P + 8 * g + 4) = make_uint2(0u, 0u);
+    }
+  }
+  return bad == 0.0f;
+}
+
+// The forward of the wavefront's samples in todo (bit i: sample b0 + i) with plain fp32 products, a lane per neuron
+// of a layer: for samples that met an infinity or a weight that is not finite.
+template <int LF, int ND, int NC, int FEAT>
+__device__ __forceinline__ void redo_samples(const MlpPtrs& wp, const float* __restrict__ a0, const FeatLayout& feat,
+                                             int64_t b0, int64_t n, const float (&dirv)[3], float sh_mult, int lane,
+                                             uint32_t todo, floatx4 (&hd)[ND][4], floatx4 (&hc)[NC][4], float& dout0,
+                                             float (&rgb)[3]) {
+  const int g = lane >> 4, s = lane & 15;
+#pragma unroll 1
+  for (; todo; todo &= todo - 1) {
+    const int i = __builtin_ctz(todo);
+    const float d[3] = {__shfl(dirv[0], i), __shfl(dirv[1], i), __shfl(dirv[2], i)};
+    const int lv = lane / FEAT;
+    float x = lane < LF && b0 + i < n ? a0[lv * feat.stride_l + (b0 + i) * feat.stride_b + (lane - lv * FEAT)] : 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < FFN_N_LAYERS; ++k) {
+      if (!layer_active(k, ND, NC)) continue;
+      const int K = layer_in(k, LF), o = lane < layer_out(k) ? lane : 0;
+      const float* __restrict__ W = wp.W[k] + o * K;
+      float acc = wp.b[k][o];
+#pragma unroll 1
+      for (int j = 0; j < K; ++j) acc = fmaf(W[j], __shfl(x, j), acc);
+      if (k == FFN_WD_OUT) {
+        x = acc;
+        const float d0 = __shfl(x, 0);
+        if (s == i) dout0 = d0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+          if (lane == 16 + q) x = sh_component(d, q) * sh_mult;
+      } else if (k == FFN_WC_OUT) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const float v = sigmoid_soft(__shfl(acc, q));
+          if (s == i) rgb[q] = v;
+        }
+      } else {
+        x = relu_f(acc);
+        auto keep = [&](floatx4 (&h)[4]) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float v = __shfl(x, 16 * t + 4 * g + r);
+              if (s == i) h[t][r] = v;
+            }
+        };
+        if (k == FFN_WD_IN) keep(hd[0]);
+        if (k == FFN_WC_IN) keep(hc[0]);
+        if constexpr (ND >= 2) {
+          if (k == FFN_WD_01) keep(hd[1]);
+        }
+        if constexpr (NC >= 2) {
+          if (k == FFN_WC_01) keep(hc[1]);
+        }
+      }
+    }
+  }
+}
+
+// forward of the wavefront's 16 samples through both networks; hd, hc: the hidden activations (for the ReLU tap).
+// Returns the samples (bit per sample) that redo_samples has to do again.
+template <int LF, int ND, int NC>
+__device__ __forceinline__ uint32_t fwd_samples(const float* __restrict__ sm, const float (&a0r)[LF / 4],
+                                            const float (&dirv)[3], float sh_mult, int g, int s, floatx4 (&hd)[ND][4],
+                                            floatx4 (&hc)[NC][4], float& dout0, float (&rgb)[3]) {
+  static_assert(ND <= 2 && NC == 2, "the layers redo_samples keeps");
+  using A = ArchF<LF, ND, NC>;
+  constexpr int PL = A::plane(), KB0 = A::cols(FFN_WD_IN) / 32;
+  // an offset of zero that the compiler cannot see through: it would read the weights before the caller's loop and
+  // spill them (200 to 900 bytes a lane)
+  int zero = 0;
+  __asm__ volatile("" : "+s"(zero));
+  sm += zero;
+  const __bf16* sW = reinterpret_cast<const __bf16*>(sm);
+  float bad = 0.0f;
+  Split8 x0[KB0];
+#pragma unroll
+  for (int kb = 0; kb < KB0; ++kb) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = 8 * kb + j < LF / 4 ? a0r[8 * kb + j] : 0.0f;
+    x0[kb] = split8(v);
+  }
+  fwd_split<4, KB0>(sW + A::w_off(FFN_WD_IN), PL, A::pitch(FFN_WD_IN), sm + A::b_off(FFN_WD_IN), x0, hd[0], g, s, true, bad);
+  Split8 x[2];
+#pragma unroll
+  for (int i = 1; i < ND; ++i) {
+    const int k = i == 1 ? FFN_WD_01 : FFN_WD_12;
+    split_tiles(hd[i - 1], x);
+    fwd_split<4, 2>(sW + A::w_off(k), PL, A::pitch(k), sm + A::b_off(k), x, hd[i], g, s, true, bad);
+  }
+  split_tiles(hd[ND - 1], x);
+  floatx4 o1[1];
+  fwd_split<1, 2>(sW + A::w_off(FFN_WD_OUT), PL, A::pitch(FFN_WD_OUT), sm + A::b_off(FFN_WD_OUT), x, o1, g, s, false,
+                   bad);
+  dout0 = o1[0][0];
+  floatx4 cin[2];
+  cin[0] = o1[0];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) cin[1][r] = sh_component(dirv, 4 * g + r) * sh_mult;
+  Split8 xc[1];
+  split_tiles(cin, xc);
+  fwd_split<4, 1>(sW + A::w_off(FFN_WC_IN), PL, A::pitch(FFN_WC_IN), sm + A::b_off(FFN_WC_IN), xc, hc[0], g, s, true, bad);
+#pragma unroll
+  for (int i = 1; i < NC; ++i) {
+    const int k = i == 1 ? FFN_WC_01 : (i == 2 ? FFN_WC_12 : FFN_WC_23);
+    split_tiles(hc[i - 1], x);
+    fwd_split<4, 2>(sW + A::w_off(k), PL, A::pitch(k), sm + A::b_off(k), x, hc[i], g, s, true, bad);
+  }
+  fwd_color_out(sm + A::out_off(), sm + A::b_off(FFN_WC_OUT), A::OUT_P, hc[NC - 1], g, s, rgb);
+  return (uint32_t)__ballot(bad != 0.0f) & 0xFFFFu;  // not a number in all four lanes of a sample alike
+}
+
+template <int LF, int ND, int NC, int FEAT>
+__global__ __launch_bounds__(VIEW_NT) void k_mlp_fwd(MlpPtrs wp, const float* __restrict__ a0, FeatLayout feat,
+                                                     const float4* __restrict__ rays,
+                                                     const uint32_t* __restrict__ ray_ids, int64_t n, float sh_mult,
+                                                     float* __restrict__ sigma, float* __restrict__ rgb,
+                                                     const uint32_t* __restrict__ n_dev) {
+  extern __shared__ __align__(16) float smv[];
+  if (n_dev) {  // the count of a launch sized for a capacity, read on the device
+    const int64_t nd = (int64_t)*n_dev;
+    n = nd < n ? nd : n;
+  }
+  if ((int64_t)blockIdx.x * 16 >= n) return;  // no samples for this block: skip staging the weights
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
+  const uint32_t always = __syncthreads_and(stage_split<LF, ND, NC>(smv, wp, tid)) ? 0u : 0xFFFFu;
+  // groups of 16 samples: a block's first, then its second ..., so that few groups spread over the blocks
+  for (int64_t grp = (int64_t)blockIdx.x + (int64_t)gridDim.x * wave; grp * 16 < n;
+       grp += (int64_t)gridDim.x * MLP_VIEW_WAVES) {
+    const int64_t b = grp * 16 + s;
+    const bool valid = b < n;
+    float a0r[LF / 4];
+    load_enc<LF, FEAT>(a0, feat, b, valid, g, a0r);
+    float dirv[3] = {0.0f, 0.0f, 1.0f};
+    if (valid) {
+      const float4 rd = rays[2 * (size_t)ray_ids[b] + 1];
+      dirv[0] = rd.x;
+      dirv[1] = rd.y;
+      dirv[2] = rd.z;
+    }
+    floatx4 hd[ND][4], hc[NC][4];
+    float dout0, c[3];
+    const uint32_t redo = always | fwd_samples<LF, ND, NC>(smv, a0r, dirv, sh_mult, g, s, hd, hc, dout0, c);
+    if (redo) redo_samples<LF, ND, NC, FEAT>(wp, a0, feat, 16 * grp, n, dirv, sh_mult, lane, redo, hd, hc, dout0, c);
+    if (g == 0 && valid) {
+      sigma[b] = softplus(fminf(fmaxf(dout0, -10.0f), 10.0f));
+      rgb[3 * b] = c[0];
+      rgb[3 * b + 1] = c[1];
+      rgb[3 * b + 2] = c[2];
+    }
+  }
+}
+
+// A forward-only step: tiles of 64 samples, one per wavefront at a time (a.tile_order puts the busy ones first).
+template <int LF, int ND, int NC, int FEAT, bool TAPS, int SC>
+__global__ __launch_bounds__(VIEW_NT) void k_mlp_view(MlpArgs a) {
+  using A = ArchF<LF, ND, NC>;
+  extern __shared__ __align__(16) float smv[];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
+  const int log2S = a.log2S;
+  const uint64_t n_samples = (uint64_t)a.num_rays << log2S;
+  const uint32_t always = __syncthreads_and(stage_split<LF, ND, NC>(smv, a.w, tid)) ? 0u : 0xFFFFu;
+  float* sSig = smv + A::w_floats() + 256 * wave;  // sigma[64], rgb[64][3] of the wavefront's tile
+  float* sRgb = sSig + 64;
+  const float Dhalf = half_box_diagonal(a.c);
+  const int64_t first = (int64_t)blockIdx.x + (int64_t)gridDim.x * wave, step = (int64_t)gridDim.x * MLP_VIEW_WAVES;
+  int64_t n_full = a.n_tiles;
+  if constexpr (!TAPS) {
+    if (a.tile_order) n_full = (int64_t)*a.n_busy;
+    else if (a.tile_busy && first < a.n_tiles && !a.tile_busy[first]) n_full = 0;
+  }
+  int64_t ti = first;
+#pragma unroll 1
+  for (; ti < n_full; ti += step) {
+    const int64_t tile = a.tile_order ? (int64_t)a.tile_order[ti] : ti;
+    const CompLane CL = load_comp_lane<SC>(a, tile, lane, true, n_samples, log2S, false);
+#pragma unroll 1
+    for (int cb = 0; cb < 4; ++cb) {
+      const int col = 16 * cb + s;
+      const int64_t b = tile * 64 + col;
+      const bool valid = (uint64_t)b < n_samples;
+      float a0r[LF / 4];
+      load_enc<LF, FEAT>(a.a0, a.feat, b, valid, g, a0r);
+      const float4 rd = a.rays[2 * (valid ? (b >> log2S) : 0) + 1];
+      const float dirv[3] = {rd.x, rd.y, rd.z};
+      const float dt_b = valid ? a.DTs[b] : 0.0f;
+      floatx4 hd[ND][4], hc[NC][4];
+      float dout0, c[3];
+      const uint32_t redo = always | fwd_samples<LF, ND, NC>(smv, a0r, dirv, a.sh_mult, g, s, hd, hc, dout0, c);
+      if (redo)
+        redo_samples<LF, ND, NC, FEAT>(a.w, a.a0, a.feat, tile * 64 + 16 * cb, (int64_t)n_samples, dirv, a.sh_mult,
+                                       lane, redo, hd, hc, dout0, c);
+      if constexpr (TAPS) {
+        if (a.t_relu) {
+          uint32_t* rec = valid ? a.t_relu + (int64_t)RELU_WORDS * b : nullptr;
+#pragma unroll
+          for (int i = 0; i < ND; ++i) tap_relu(rec, i, hd[i], g);
+#pragma unroll
+          for (int i = 0; i < NC; ++i) tap_relu(rec, 3 + i, hc[i], g);
+        }
+      }
+      if (g == 0) {
+        const float sig = softplus(fminf(fmaxf(dout0, -10.0f), 10.0f));
+        sSig[col] = dt_b <= 0.0f ? 0.0f : sig;
+        sRgb[3 * col] = c[0];
+        sRgb[3 * col + 1] = c[1];
+        sRgb[3 * col + 2] = c[2];
+      }
+    }
+    wave_lds_sync();
+    float dLds, dLdc[3];
+    composite_tile<TAPS, SC>(a, sSig, sRgb, CL, lane, 0, true, false, false, Dhalf, dLds, dLdc);
+    wave_lds_sync();
+  }
+#pragma unroll 1
+  for (; ti < a.n_tiles; ti += step) {
+    const int64_t tile = a.tile_order ? (int64_t)a.tile_order[ti] : ti;
+    const CompLane CL = load_comp_lane<SC>(a, tile, lane, false, n_samples, log2S, false);
+    empty_tile<LF, FEAT, SC>(a, CL, lane, 0, 0, false, false, g);
+  }
+}
+
+// ---------------------------------------------------------------------------
+
+template <int LF, int ND, int NC, int FEAT>
+static hipError_t launch_fwd_f(const MlpPtrs& w, const float* a0, const FeatLayout& feat, const float4* rays,
+                               const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma, float* rgb,
+                               int n_blocks, hipStream_t st, const uint32_t* n_dev) {
+  const size_t lds = sizeof(float) * (size_t)ArchF<LF, ND, NC>::w_floats();
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_fwd<LF, ND, NC, FEAT>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((k_mlp_fwd<LF, ND, NC, FEAT>), dim3(n_blocks), dim3(VIEW_NT), lds, st, w, a0, feat, rays, ray_ids,
+                     n, sh_mult, sigma, rgb, n_dev);
+  return hipGetLastError();
+}
+
+template <int LF, int ND, int NC>
+static hipError_t launch_fwd_t(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
+                               const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
+                               float* rgb, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
+  switch (c.F) {
+    case 1: return launch_fwd_f<LF, ND, NC, 1>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
+    case 2: return launch_fwd_f<LF, ND, NC, 2>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
+    case 4: return launch_fwd_f<LF, ND, NC, 4>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int LF, int ND, int NC, int FEAT, bool TAPS, int SC>
+static hipError_t launch_view_f(const MlpArgs& a, int n_blocks, hipStream_t st) {
+  const size_t lds = sizeof(float) * ((size_t)ArchF<LF, ND, NC>::w_floats() + 256 * MLP_VIEW_WAVES);
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_view<LF, ND, NC, FEAT, TAPS, SC>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((k_mlp_view<LF, ND, NC, FEAT, TAPS, SC>), dim3(n_blocks), dim3(VIEW_NT), lds, st, a);
+  return hipGetLastError();
+}
+
+template <int LF, int ND, int NC, int SC>
+static hipError_t launch_view_t(const MlpArgs& a, int n_blocks, hipStream_t st) {
+  const bool taps = taps_requested(a);
+  switch (a.c.F) {
+    case 1:
+      return taps ? launch_view_f<LF, ND, NC, 1, true, SC>(a, n_blocks, st)
+                  : launch_view_f<LF, ND, NC, 1, false, SC>(a, n_blocks, st);
+    case 2:
+      return taps ? launch_view_f<LF, ND, NC, 2, true, SC>(a, n_blocks, st)
+                  : launch_view_f<LF, ND, NC, 2, false, SC>(a, n_blocks, st);
+    case 4:
+      return taps ? launch_view_f<LF, ND, NC, 4, true, SC>(a, n_blocks, st)
+                  : launch_view_f<LF, ND, NC, 4, false, SC>(a, n_blocks, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+#define FFN_MLP_FWD_CONFIGS(X) \
+  X(16, 1, 2)                  \
+  X(32, 1, 2)                  \
+  X(64, 1, 2)                  \
+  X(16, 2, 2)                  \
+  X(32, 2, 2)                  \
+  X(64, 2, 2)
+
+hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
+                          const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
+                          float* rgb, int LF, int nd, int nc, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
+  if (n <= 0) return hipSuccess;
+#define X(l, d, nn)                   \
+  if (LF == l && nd == d && nc == nn) \
+    return launch_fwd_t<l, d, nn>(c, w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
+  FFN_MLP_FWD_CONFIGS(X)
+#undef X
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_mlp_view(const MlpArgs& a, int LF, int nd, int nc, int n_blocks, hipStream_t st) {
+#define X(l, d, n)                   \
+  if (LF == l && nd == d && nc == n) \
+    return a.S == 64 ? launch_view_t<l, d, n, 64>(a, n_blocks, st) : launch_view_t<l, d, n, 0>(a, n_blocks, st);
+  FFN_MLP_FWD_CONFIGS(X)
+#undef X
+  return hipErrorInvalidValue;
+}
+
+}  // namespace ffn
