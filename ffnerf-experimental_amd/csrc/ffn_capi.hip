@@ -34,11 +34,20 @@ int fail(int code, const char* fmt, ...) {
     if (e_ != hipSuccess) return fail(-3, "%s: %s", #call, hipGetErrorString(e_));        \
   } while (0)
 
+// A buffer that grows with its calls.  Its size is not a function of the call's size alone (the bucket sizes and the
+// dense copies follow the samples a call is planned for), so a smaller call may grow it: once a call of the handle
+// has been captured into a graph, outgrown buffers are kept for the graph's launches until ffn_destroy.
 struct Scratch {
   void* p = nullptr;
   size_t bytes = 0;
+  std::vector<void*>* outgrown = nullptr;  // set by the handle's first captured call
   hipError_t ensure(size_t need) {
     if (need <= bytes) return hipSuccess;
+    if (p && outgrown) {
+      outgrown->push_back(p);
+      p = nullptr;
+      bytes = 0;
+    }
     if (p) {
       hipError_t e = hipFree(p);
       if (e != hipSuccess) return e;
@@ -96,6 +105,16 @@ struct Handle {
   Scratch order_counts, order_pairs, order_perm, order_pts;  // the encode entry points' spatial order
   Scratch tile_sched;  // the MLP's tile order: busy flags (bytes), order, busy count
   uint32_t* host_total = nullptr;  // pinned
+  std::vector<void*> outgrown;     // buffers that captured calls may use, replaced by larger ones since
+
+  template <class Fn>
+  void each_scratch(Fn&& fn) {
+    for (Scratch* sc : {&Ts, &DTs, &flags, &a0, &dLda0, &partials, &bin_meta, &bin_meta_t, &bin_pairs, &bin_max,
+                        &m_state, &m_acc, &m_counts, &m_offsets, &m_sums, &m_total, &m_samples, &m_ids, &m_a0,
+                        &m_sigma, &m_rgb, &m_Tr, &m_dLds, &m_dLdc, &m_bits, &m_blocks, &m_slots, &dense,
+                        &order_counts, &order_pairs, &order_perm, &order_pts, &tile_sched})
+      fn(*sc);
+  }
 };
 
 // A scratch buffer may grow to `need` bytes when it is no larger than what it already holds plus half of the
@@ -214,6 +233,11 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* pl
   return hipSuccess;
 }
 
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
 // Whether ffn_hash_encode_fwd gathers in a spatial order of its points: the sort and the rows written through its
 // permutation cost about 65 us and 0.07 ns a point, and the gather wins the more, the further the tables lie from
 // the L2 and the closer the points.  us, plain / ordered, uniform points; points on a shell:
@@ -223,7 +247,7 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* pl
 //    8 x 2^14 entries: 2^20 216 / 255; 201 / 206    2^22 794 / 715; 742 / 593
 // The scatter gains nothing reliable (2^22 points, 16 x 2^22: 3837 / 3882; 4187 / 3749; 16 x 2^19 2713 / 2925): the
 // merged pairs leave runs of one or two pairs a bucket, which are padded to eight.  FFN_ORDER=0: never, 1: always.
-bool order_pays(const Handle* h, int64_t n) {
+bool order_pays(const Handle* h, int64_t n, hipStream_t st) {
   if (n >= ((int64_t)1 << 31)) return false;
   if (const char* e = getenv("FFN_ORDER")) return atoi(e) != 0;
   uint32_t T = 0;
@@ -235,7 +259,8 @@ bool order_pays(const Handle* h, int64_t n) {
   const bool held = h->order_pairs.bytes >= 2 * sizeof(uint2) * (size_t)n &&
                     h->order_pts.bytes >= sizeof(float4) * (size_t)n &&
                     h->order_perm.bytes >= sizeof(uint32_t) * (size_t)n;
-  return held || growth_fits_free(Scratch{}, need);
+  // (a captured call cannot allocate it either)
+  return held || (!capturing(st) && growth_fits_free(Scratch{}, need));
 }
 
 // the points' Morton order in the handle's scratch: src becomes the ordered points, *perm their indices
@@ -480,8 +505,10 @@ struct StageTimer {
 void note_use(Handle* h, hipStream_t st) {
   // a call captured into a graph runs when the graph is launched, not here: the caller orders those launches
   // before ffn_destroy (no event is recorded into the capture)
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return;
+  if (capturing(st)) {
+    h->each_scratch([&](Scratch& sc) { sc.outgrown = &h->outgrown; });
+    return;
+  }
   for (StreamUse& u : h->uses) {
     if (u.st == st) {
       if (hipEventRecord(u.ev, st) != hipSuccess) h->uses_lost = true;
@@ -565,21 +592,8 @@ int ffn_destroy(void* handle) {
   }
   h->uses.clear();
   destroy_events(h);
-  h->Ts.release();
-  h->DTs.release();
-  h->flags.release();
-  h->a0.release();
-  h->dLda0.release();
-  h->partials.release();
-  h->bin_meta.release();
-  h->bin_meta_t.release();
-  h->bin_pairs.release();
-  h->bin_max.release();
-  for (Scratch* sc : {&h->m_state, &h->m_acc, &h->m_counts, &h->m_offsets, &h->m_sums, &h->m_total, &h->m_samples,
-                      &h->m_ids, &h->m_a0, &h->m_sigma, &h->m_rgb, &h->m_Tr, &h->m_dLds, &h->m_dLdc, &h->m_bits,
-                      &h->m_blocks, &h->m_slots, &h->dense, &h->tile_sched, &h->order_counts,
-                      &h->order_pairs, &h->order_perm, &h->order_pts})
-    sc->release();
+  h->each_scratch([](Scratch& sc) { sc.release(); });
+  for (void* p : h->outgrown) (void)hipFree(p);
   if (h->host_total) (void)hipHostFree(h->host_total);
   delete h;
   return 0;
@@ -648,7 +662,7 @@ int ffn_hash_encode_fwd(void* handle, const float* x, int64_t n, float* a0, uint
   const ffn::FeatLayout lm = ffn::level_major(n, h->dc.F);
   ffn::PosSrc src{x, nullptr, nullptr, 0};
   const uint32_t* perm = nullptr;  // (corner indices are written in the points' own order)
-  if (!idx_out && order_pays(h, n)) FFN_HIP(order_points(h, n, &src, &perm, st));
+  if (!idx_out && order_pays(h, n, st)) FFN_HIP(order_points(h, n, &src, &perm, st));
   ffn::DenseLevels dl;
   FFN_HIP(build_dense_levels(h, h->params.table, n, &dl, st));
   FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, (float*)h->a0.p, lm, idx_out, &dl, st));

@@ -1,9 +1,9 @@
-// ffn_order.hip -- a spatial order of query points for the encode entry points.
+// ffn_order.hip -- a spatial order of query points for the encode entry point.
 //
 // Points in no order touch a table vertex from wavefronts all over the GPU at different times: every corner of a
 // table beyond the L2 is a cache line from further away (2^24 uniform points, 16 x 2^22 entries: 7.3 times the
 // algorithmic bytes).  In Morton order the points around a vertex are neighbours, so its line is fetched about
-// once, and points of one cell follow each other, which the scatter's merge turns into one pair per corner.
+// once.
 //
 // The order is a stable least-significant-digit radix sort of (key, index) pairs: three passes over 8 bits of a
 // 24-bit Morton key (256 cells per axis).  A pass counts digits per block of 4096 pairs, scans the counts

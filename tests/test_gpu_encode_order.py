@@ -59,3 +59,36 @@ def test_order_by_rule(monkeypatch):
     by_rule = encode(m, x, 4)
     monkeypatch.setenv("FFN_ORDER", "0")
     np.testing.assert_array_equal(by_rule.view(np.uint32), encode(m, x, 4).view(np.uint32))
+
+
+def test_graph_outlives_larger_calls(monkeypatch):
+    """An encode captured into a graph keeps its buffers when later eager calls outgrow them: its replays give the
+    encodings of the points that the input holds then."""
+    import ffn_lib as fl
+    import torch
+    from gpu_helpers import GpuModel
+    spec = spec_cfg0(n_levels=2, log2_T=[16, 18], res=[40.0, 300.0])
+    m = GpuModel(spec, random_params(spec, seed=6))
+    monkeypatch.setenv("FFN_ORDER", "1")
+    n = 70001
+    x_t = torch.from_numpy(points(n, 7)).cuda()
+    out = torch.zeros((n, 4), device="cuda")
+    s = torch.cuda.Stream()
+
+    def call():
+        fl.check(m.lib.ffn_hash_encode_fwd(m.h.h, fl.ptr(x_t), n, fl.ptr(out), None, fl.stream_ptr()), "encode")
+
+    print("[encode order] graph", flush=True)
+    with torch.cuda.stream(s):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call()
+    for rep in range(3):
+        encode(m, points(4 * n * (rep + 1), 8 + rep), 4)
+        x = points(n, 20 + rep)
+        x_t.copy_(torch.from_numpy(x))
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), encode(m, x, 4).view(np.uint32))
