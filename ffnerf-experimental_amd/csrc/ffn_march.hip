@@ -660,7 +660,10 @@ __global__ __launch_bounds__(256) void k_march_init(MarchState* __restrict__ sta
 }
 
 // front-to-back compositing of this round's samples of each ray (alpha as ffnerf_OG.cl:1505-1520);
-// a ray whose transmittance drops below T_stop is retired
+// a ray whose transmittance drops below T_stop is retired.
+// What bounds it: the latency of a lane's loads, so a lane loads RENDER_AHEAD samples before it composites them in
+// order (past the ray's end the last one again).  450x800 frame, three rounds: one at a time 81 us, four 61, eight 50.
+constexpr uint32_t RENDER_AHEAD = 8;
 __global__ __launch_bounds__(256) void k_render_composite(const uint32_t* __restrict__ offsets,
                                                           const uint32_t* __restrict__ counts, uint32_t num_rays,
                                                           const float* __restrict__ sigma,
@@ -679,20 +682,30 @@ __global__ __launch_bounds__(256) void k_render_composite(const uint32_t* __rest
   if (!(T >= T_stop)) return;  // retired in an earlier round
   float C0 = cv.x, C1 = cv.y, C2 = cv.z;
   uint32_t used = 0;
-  for (uint32_t j = 0; j < cnt; ++j) {
-    const uint32_t b = off + j;
-    const float alpha = 1.0f - fast_exp(fminf(fmaxf(-sigma[b] * dt, -5.0f), 18.0f));
-    const float w = T * alpha;
-    C0 = C0 + w * rgb[3 * (size_t)b];
-    C1 = C1 + w * rgb[3 * (size_t)b + 1];
-    C2 = C2 + w * rgb[3 * (size_t)b + 2];
-    T = T * (1.0f - alpha);
-    ++used;
-    if (T < T_stop) {
-      state[r].flags |= MARCH_DONE;
-      break;
+  bool stopped = false;
+  for (uint32_t j = 0; j < cnt && !stopped; j += RENDER_AHEAD) {
+    float sg[RENDER_AHEAD], c[RENDER_AHEAD][3];
+#pragma unroll
+    for (uint32_t u = 0; u < RENDER_AHEAD; ++u) {
+      const size_t b = (size_t)off + (j + u < cnt ? j + u : cnt - 1);
+      sg[u] = sigma[b];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) c[u][i] = rgb[3 * b + i];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < RENDER_AHEAD; ++u) {
+      if (j + u >= cnt || stopped) continue;
+      const float alpha = 1.0f - fast_exp(fminf(fmaxf(-sg[u] * dt, -5.0f), 18.0f));
+      const float w = T * alpha;
+      C0 = C0 + w * c[u][0];
+      C1 = C1 + w * c[u][1];
+      C2 = C2 + w * c[u][2];
+      T = T * (1.0f - alpha);
+      ++used;
+      stopped = T < T_stop;
     }
   }
+  if (stopped) state[r].flags |= MARCH_DONE;
   acc[r] = make_float4(C0, C1, C2, T);
   if (n_used) n_used[r] += used;
 }
