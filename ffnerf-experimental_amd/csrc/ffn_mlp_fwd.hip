@@ -4,14 +4,9 @@
 // Reference: ffnerf_OG.cl:1373-1466 (MLP fwd), 1505-1591 (compositing).
 //
 // MI355X design
-//   * Every fp32 value x of a product is the exact sum of three bfloat16 values: h = x's top 16 bits, m = the top
-//     16 bits of x - h, l = x - h - m (8 + 8 + 8 significand bits; the differences are exact).  A product a b is the
-//     six terms a_h b_h + a_h b_m + a_m b_h + a_m b_m + a_h b_l + a_l b_h, each exact on
-//     v_mfma_f32_16x16x32_bf16, which adds 32 products to its fp32 accumulator with one rounding; the three terms
-//     left out are below 2^-23 of a b together.  Against 64-bit sums of 32 random products: relative error 4.2e-8
-//     (fp32 MFMAs, eight of K = 4 in a chain, 1.04e-7); on outputs that pass a ReLU 4.4e-8 (7.7e-8).  Six K = 32
-//     instructions of 16 cycles do the work of eight fp32 ones of 32, and unlike those they run beside vector
-//     instructions.
+//   * The layers' products are fp32 products on bfloat16 matrix instructions, three planes a value and eight terms a
+//     product (ffn_mlp_split.h): half the matrix cycles of the fp32 instruction, beside vector instructions, and sums
+//     no further from 64 bits.
 //   * A block of 16 wavefronts, one per CU, shares the weights in LDS (three bfloat16 planes, K-ordered rows); a
 //     wavefront works alone (no barrier after the staging): 16 samples through all layers, activations in registers
 //     in the D layout of one layer = the B operand of the next (K slot j of lane group g in block kb is neuron
@@ -27,10 +22,9 @@
 #include "ffn_device.h"
 #include "ffn_kernels.h"
 #include "ffn_mlp_common.h"
+#include "ffn_mlp_split.h"
 
 namespace ffn {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int VIEW_NT = 64 * MLP_VIEW_WAVES;
 
@@ -73,92 +67,6 @@ __device__ __forceinline__ constexpr int row_pos(int n) {
   }
 }
 
-__device__ __forceinline__ float top16(float x) { return __int_as_float(__float_as_int(x) & (int)0xFFFF0000); }
-// {x1's upper half, x0's upper half}
-__device__ __forceinline__ uint32_t upper_halves(float x1, float x0) {
-  return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
-}
-
-// eight values of a K block, as three bfloat16 operands
-struct Split8 {
-  bf16x8 h, m, l;
-};
-__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
-  uint32_t h[4], m[4], l[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float x0 = x[2 * q], x1 = x[2 * q + 1];
-    const float r0 = x0 - top16(x0), r1 = x1 - top16(x1);
-    const float l0 = r0 - top16(r0), l1 = r1 - top16(r1);
-    h[q] = upper_halves(x1, x0);
-    m[q] = upper_halves(r1, r0);
-    l[q] = upper_halves(l1, l0);
-  }
-  Split8 s;
-  s.h = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
-  s.m = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
-  s.l = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
-  return s;
-}
-// the K blocks of D-layout tiles
-template <int IT>
-__device__ __forceinline__ void split_tiles(const floatx4 (&t)[IT], Split8 (&o)[IT / 2]) {
-#pragma unroll
-  for (int kb = 0; kb < IT / 2; ++kb) {
-    const float x[8] = {t[2 * kb][0],     t[2 * kb][1],     t[2 * kb][2],     t[2 * kb][3],
-                        t[2 * kb + 1][0], t[2 * kb + 1][1], t[2 * kb + 1][2], t[2 * kb + 1][3]};
-    o[kb] = split8(x);
-  }
-}
-
-// out tiles (D layout) = act(W . in + b), two output tiles at a time so that consecutive MFMAs are independent;
-// bad becomes not a number where the sample's sums are infinite or not numbers
-template <int OT, int KB>
-__device__ __forceinline__ void fwd_split(const __bf16* __restrict__ W, int plane, int P, const float* __restrict__ B,
-                                          const Split8 (&in)[KB], floatx4 (&out)[OT], int g, int s, bool relu,
-                                          float& bad) {
-  const __bf16* wrow = W + s * P + 8 * g;
-  constexpr int G = OT < 2 ? OT : 2;
-#pragma unroll
-  for (int t0 = 0; t0 < OT; t0 += G) {
-    floatx4 acc[G];
-#pragma unroll
-    for (int t = 0; t < G; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[t][r] = B[16 * (t0 + t) + 4 * g + r];
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      bf16x8 wh[G], wm[G], wl[G];
-#pragma unroll
-      for (int t = 0; t < G; ++t) {
-        const __bf16* w = wrow + 16 * (t0 + t) * P + 32 * kb;
-        wh[t] = *reinterpret_cast<const bf16x8*>(w);
-        wm[t] = *reinterpret_cast<const bf16x8*>(w + plane);
-        wl[t] = *reinterpret_cast<const bf16x8*>(w + 2 * plane);
-      }
-      auto term = [&](const bf16x8 (&w)[G], const bf16x8& x) {
-#pragma unroll
-        for (int t = 0; t < G; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], x, acc[t], 0, 0, 0);
-      };
-      term(wl, in[kb].h);
-      term(wh, in[kb].l);
-      term(wm, in[kb].m);
-      term(wm, in[kb].h);
-      term(wh, in[kb].m);
-      term(wh, in[kb].h);
-    }
-    if (t0 == 0) bad = fmaf(acc[0][0], 0.0f, bad);
-#pragma unroll
-    for (int t = 0; t < G; ++t) {
-      if (relu) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[t][r] = relu_f(acc[t][r]);
-      }
-      out[t0 + t] = acc[t];
-    }
-  }
-}
-
 // stage the weights into LDS (split into planes) and the biases; returns whether this thread's weights are all finite
 template <int LF, int ND, int NC>
 __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtrs& wp, int tid) {
@@ -173,18 +81,9 @@ __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtr
           *reinterpret_cast<float4*>(sm + A::out_off() + o * A::OUT_P + i) = v;
         } else {
           const float x[4] = {v.x, v.y, v.z, v.w};
-          float r[4], l[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            r[q] = x[q] - top16(x[q]);
-            l[q] = r[q] - top16(r[q]);
-            bad = fmaf(x[q], 0.0f, bad);
-          }
-          __bf16* w = sW + A::w_off(k) + o * A::pitch(k) + row_pos<LF, k>(i);  // four consecutive positions
-          *reinterpret_cast<uint2*>(w) = make_uint2(upper_halves(x[1], x[0]), upper_halves(x[3], x[2]));
-          *reinterpret_cast<uint2*>(w + A::plane()) = make_uint2(upper_halves(r[1], r[0]), upper_halves(r[3], r[2]));
-          *reinterpret_cast<uint2*>(w + 2 * A::plane()) =
-              make_uint2(upper_halves(l[1], l[0]), upper_halves(l[3], l[2]));
+          for (int q = 0; q < 4; ++q) bad = fmaf(x[q], 0.0f, bad);
+          put_split4(sW + A::w_off(k) + o * A::pitch(k) + row_pos<LF, k>(i), A::plane(), x);  // consecutive positions
         }
       },
       [&](auto K, int o, float v) { sm[A::b_off(K) + o] = v; });
