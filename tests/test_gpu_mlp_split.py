@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from test_gpu_math import _load
+from test_gpu_mlp_view import planes
 
 N = 4096
 FULL = np.uint32(0x3F80FFFF).view(np.float32)  # h = 1, m and l one unit below their bounds 2^-7 and 2^-15
@@ -46,6 +47,18 @@ def layer(split, x, W, B):
     return out.cpu().numpy().astype(np.float64)
 
 
+MAX_TOL = 1.5 * 2.0 ** -24
+
+
+# which products the layer test would miss: none of the eight
+@pytest.mark.parametrize("term", [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0), (1, 2), (2, 1)])
+def test_a_lost_term_shows(term):
+    x, W, _ = operands("full one", 64)
+    lost = np.abs(planes(x)[term[0]] @ planes(W)[term[1]].T)
+    size = np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T
+    assert (lost / size).max() > 2 * MAX_TOL
+
+
 # The split sums may be no further from float64 than the fp32 instruction's (2-norm: of 262,144 sums, so steady to a
 # per cent), nor, for their largest error, than that or one and a half roundings of the sum's terms.  With six of the
 # eight terms a single product is off by up to 4.7e-7 and by 7e-8 in the 2-norm; the fp32 instruction by 6.0e-8 and 2.5e-8.
@@ -64,4 +77,4 @@ def test_no_further_than_fp32(kind, K):
         err[split] = np.linalg.norm(e) / np.linalg.norm(ref), np.max(np.abs(e) / size)
     print(f"[split layer] {kind} K={K}: split {err[1][0]:.2e} {err[1][1]:.2e}, fp32 {err[0][0]:.2e} {err[0][1]:.2e}")
     assert err[1][0] <= 1.02 * err[0][0]
-    assert err[1][1] <= max(err[0][1], 1.5 * 2.0 ** -24)
+    assert err[1][1] <= max(err[0][1], MAX_TOL)

@@ -9,19 +9,38 @@ from oracle import oracle as ora
 pytestmark = pytest.mark.gpu
 
 
-def forward64(spec, p, a0, dirs, sh_mult):
+def planes(x):
+    """The three bfloat16 planes of float32 values (ffn_mlp_split.h), as float64."""
+    out, r = [], np.asarray(x, np.float32)
+    for _ in range(3):
+        h = (r.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+        out.append(h.astype(np.float64))
+        r = (r - h).astype(np.float32)
+    return out
+
+
+def forward64(spec, p, a0, dirs, sh_mult, drop=None):
+    """The networks in float64; drop = (plane of the weight, plane of the input): without that term of the split
+    layers' products."""
     f = {k: np.asarray(v, np.float64) for k, v in p.items() if k[:2] in ("Wd", "Wc", "bd", "bc")}
+
+    def layer(x, name, bias):
+        y = x @ f[name].T + f[bias]
+        if drop and name != "Wc_out":
+            y = y - planes(x)[drop[1]] @ planes(p[name])[drop[0]].T
+        return y
+
     x = a0.astype(np.float64)
     dens = ["in"] + (["01"] if spec["nd"] >= 2 else []) + ["out"]
     for i, n in enumerate(dens):
-        x = x @ f["Wd_" + n].T + f["bd_" + ("out" if n == "out" else str(i))]
+        x = layer(x, "Wd_" + n, "bd_" + ("out" if n == "out" else str(i)))
         if n != "out":
             x = np.maximum(x, 0.0)
     d0 = np.clip(x[:, 0], -10, 10)
     sh = np.stack([ora_sh(d) for d in dirs]) * sh_mult
     x = np.concatenate([x, sh], 1)
     for i, n in enumerate(["in", "01", "out"]):
-        x = x @ f["Wc_" + n].T + f["bc_" + ("out" if n == "out" else str(i))]
+        x = layer(x, "Wc_" + n, "bc_" + ("out" if n == "out" else str(i)))
         if n != "out":
             x = np.maximum(x, 0.0)
     return np.log1p(np.exp(d0)), 1.0 / (1.0 + np.exp(-np.clip(0.5 * x, -18, 18)))
@@ -35,9 +54,16 @@ def ora_sh(d):
     return out.astype(np.float64)
 
 
-# Rounding of a layer: the split terms left out (2^-23) and one fp32 rounding per 32 products, of at most 64 products
-# and a bias of a few units each, through five layers whose gains are near one; the activations add 1e-6 (their
-# own test).  1e-5 of the largest output covers their sum; a wrong lane, plane or K order misses it by far.
+# Two sums of 64 products a layer and its activation: the GPU's error is 0.6 to 1.8e-7 over these shapes; a plane or term
+# of the products that is lost shows as at least ten times this limit (asserted from the same inputs), but for the two
+# smallest terms, which test_gpu_mlp_split.py pins.
+VIEW_TOL = 5e-7
+
+
+def view_error(sig, rgb, sig64, rgb64, on):
+    return np.abs(sig - sig64)[on].max() / max(1.0, sig64.max()), np.abs(rgb - rgb64).max()
+
+
 @pytest.mark.parametrize("L,F,nd,n_rays,S", [(8, 2, 1, 33, 64), (16, 2, 1, 700, 16), (16, 4, 2, 129, 64),
                                              (16, 1, 1, 5, 4), (8, 4, 2, 65, 32), (16, 1, 2, 130, 64),
                                              (16, 4, 1, 40, 64), (32, 2, 2, 9, 64)])
@@ -52,11 +78,15 @@ def test_view_forward(L, F, nd, n_rays, S):
     print(f"[view] LF={L * F} F={F} nd={nd} rays={n_rays} S={S}", flush=True)
     _, t = GpuModel(spec, p).train_step(rays, np.zeros((n_rays, 4), np.float32), S, sc, taps=True)
     dirs = np.repeat(rays[:, 4:7], S, axis=0)
-    sig, rgb = forward64(spec, p, t["a0"].reshape(-1, L * F), dirs, sc["sh_multiplier"])
+    nets = spec, p, t["a0"].reshape(-1, L * F), dirs, sc["sh_multiplier"]
+    ref = forward64(*nets)
     on = t["DTs"].reshape(-1) > 0
+    err = view_error(t["sigma"].reshape(-1), t["rgb"].reshape(-1, 3), *ref, on)
+    lost = {d: max(view_error(*forward64(*nets, drop=d), *ref, on)) for d in [(2, 0), (0, 2), (1, 1), (1, 0), (0, 1)]}
+    print(f"[view] sigma {err[0]:.2e} rgb {err[1]:.2e}; a lost term {min(lost.values()):.1e}", flush=True)
+    assert min(lost.values()) > 10 * VIEW_TOL
     assert np.all(t["sigma"].reshape(-1)[~on] == 0)
-    assert np.abs(t["sigma"].reshape(-1) - sig)[on].max() <= 1e-5 * max(1.0, sig.max())
-    assert np.abs(t["rgb"].reshape(-1, 3) - rgb).max() <= 1e-5
+    assert max(err) <= VIEW_TOL
 
 
 def positive_params(spec, seed):
