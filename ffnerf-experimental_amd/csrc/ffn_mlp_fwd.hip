@@ -16,9 +16,12 @@
 //     Measured against the fp32-MFMA forward (three blocks of four wavefronts per CU, 16-byte weight staging):
 //     880,000 marched samples of the 32-feature model 167 -> 108 us, a frame's first round of 3.0M samples 542 ->
 //     347; a preview of 590,000 samples of the 64-feature model with two density layers 166 -> 97 us.
-//   * An infinite value's m is not a number, so its split products are none either where the value's own products
-//     would be infinities.  The wavefront sees that in its sums (every sum of a sample with such a value is not a
-//     number) or, for a weight, when it is staged, and redoes those samples with plain fp32 products.
+//   * The split does not hold infinities (their m is not a number), and loses the lower planes of operands near the
+//     smallest numbers.  A wavefront sees infinities in its sums (every sum of a sample with such a value is not a
+//     number) and does those samples again on the fp32 instruction, with the weights from memory; a block whose staged
+//     weights are not all in the split's range takes the fp32 instruction alone
+//     (a preview of 2^20 samples of a diverged model: 0.58 ms, in the split's range 0.32; a sample and a lane per neuron
+//     at a time it took 15.8).
 #include "ffn_device.h"
 #include "ffn_kernels.h"
 #include "ffn_mlp_common.h"
@@ -67,12 +70,20 @@ __device__ __forceinline__ constexpr int row_pos(int n) {
   }
 }
 
-// stage the weights into LDS (split into planes) and the biases; returns whether this thread's weights are all finite
+// Whether the split holds a weight: zero, or its exponent at most 64 from 1's.  Beyond, infinities and "not a number"
+// apart, the instruction's flush of operands below 2^-126 could take more of a product than its rounding does: a
+// weight's lower planes below 2^-110, an input's at weights so large that the lost 2^-125 counts.
+__device__ __forceinline__ bool split_holds(float w) {
+  const uint32_t e = (__float_as_uint(w) >> 23) & 255u;
+  return w == 0.0f || (e >= 127u - 64u && e <= 127u + 64u);
+}
+
+// stage the weights into LDS (split into planes) and the biases; returns whether the split holds this thread's weights
 template <int LF, int ND, int NC>
 __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtrs& wp, int tid) {
   using A = ArchF<LF, ND, NC>;
   __bf16* sW = reinterpret_cast<__bf16*>(sm);
-  float bad = 0.0f;
+  bool holds = true;
   read_weights<LF, ND, NC, VIEW_NT>(
       wp, tid,
       [&](auto K, int o, int i, const float4& v) {
@@ -82,7 +93,7 @@ __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtr
         } else {
           const float x[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-          for (int q = 0; q < 4; ++q) bad = fmaf(x[q], 0.0f, bad);
+          for (int q = 0; q < 4; ++q) holds = holds && split_holds(x[q]);
           put_split4(sW + A::w_off(k) + o * A::pitch(k) + row_pos<LF, k>(i), A::plane(), x);  // consecutive positions
         }
       },
@@ -95,75 +106,92 @@ __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtr
       *reinterpret_cast<uint2*>(sW + p * A::plane() + A::w_off(FFN_WD_IN) + o * P + 8 * g + 4) = make_uint2(0u, 0u);
     }
   }
-  return bad == 0.0f;
+  return holds;
 }
 
-// The forward of the wavefront's samples in todo (bit i: sample b0 + i) with plain fp32 products, a lane per neuron
-// of a layer: for samples that met an infinity or a weight that is not finite.
-template <int LF, int ND, int NC, int FEAT>
-__device__ __forceinline__ void redo_samples(const MlpPtrs& wp, const float* __restrict__ a0, const FeatLayout& feat,
-                                             int64_t b0, int64_t n, const float (&dirv)[3], float sh_mult, int lane,
-                                             uint32_t todo, floatx4 (&hd)[ND][4], floatx4 (&hc)[NC][4], float& dout0,
-                                             float (&rgb)[3]) {
-  const int g = lane >> 4, s = lane & 15;
-#pragma unroll 1
-  for (; todo; todo &= todo - 1) {
-    const int i = __builtin_ctz(todo);
-    const float d[3] = {__shfl(dirv[0], i), __shfl(dirv[1], i), __shfl(dirv[2], i)};
-    const int lv = lane / FEAT;
-    float x = lane < LF && b0 + i < n ? a0[lv * feat.stride_l + (b0 + i) * feat.stride_b + (lane - lv * FEAT)] : 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < FFN_N_LAYERS; ++k) {
-      if (!layer_active(k, ND, NC)) continue;
-      const int K = layer_in(k, LF), o = lane < layer_out(k) ? lane : 0;
-      const float* __restrict__ W = wp.W[k] + o * K;
-      float acc = wp.b[k][o];
-#pragma unroll 1
-      for (int j = 0; j < K; ++j) acc = fmaf(W[j], __shfl(x, j), acc);
-      if (k == FFN_WD_OUT) {
-        x = acc;
-        const float d0 = __shfl(x, 0);
-        if (s == i) dout0 = d0;
+// out tiles (D layout) = act(W . in + b) on the fp32 instruction, with the sums' order of the training kernels; W: the
+// layer's rows of P floats, the weight of k-step kk of input tile tp at col(tp) + kk
+template <int OT, int IT, class Col>
+__device__ __forceinline__ void fwd_fp32(const float* __restrict__ W, bool aligned16, int P, const float* __restrict__ B,
+                                         const floatx4 (&in)[4], floatx4 (&out)[4], int g, int s, bool relu, Col col) {
 #pragma unroll
-        for (int q = 0; q < 16; ++q)
-          if (lane == 16 + q) x = sh_component(d, q) * sh_mult;
-      } else if (k == FFN_WC_OUT) {
+  for (int t = 0; t < OT; ++t) {
+    floatx4 acc;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          const float v = sigmoid_soft(__shfl(acc, q));
-          if (s == i) rgb[q] = v;
-        }
-      } else {
-        x = relu_f(acc);
-        auto keep = [&](floatx4 (&h)[4]) {
+    for (int r = 0; r < 4; ++r) acc[r] = B[16 * t + 4 * g + r];
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
+    for (int tp = 0; tp < IT; ++tp) {
+      const float* w = W + (16 * t + s) * P + col(tp);
+      floatx4 w4;
+      if (aligned16) w4 = *reinterpret_cast<const floatx4*>(w);
+      else w4 = floatx4{w[0], w[1], w[2], w[3]};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float v = __shfl(x, 16 * t + 4 * g + r);
-              if (s == i) h[t][r] = v;
-            }
-        };
-        if (k == FFN_WD_IN) keep(hd[0]);
-        if (k == FFN_WC_IN) keep(hc[0]);
-        if constexpr (ND >= 2) {
-          if (k == FFN_WD_01) keep(hd[1]);
-        }
-        if constexpr (NC >= 2) {
-          if (k == FFN_WC_01) keep(hc[1]);
-        }
-      }
+      for (int rp = 0; rp < 4; ++rp) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w4[rp], in[tp][rp], acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);  // (all weights' loads at once would spill)
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[t][r] = relu ? relu_f(acc[r]) : acc[r];
   }
 }
 
-// forward of the wavefront's 16 samples through both networks; hd, hc: the hidden activations (for the ReLU tap).
-// Returns the samples (bit per sample) that redo_samples has to do again.
+// The forward of the wavefront's 16 samples with fp32 products, for samples and weights that the split cannot hold: the
+// weights straight from memory (the caches hold them), the biases and the colour output layer from LDS.  Not inlined:
+// its registers would be spilled on the split's path.  b: the lane's sample (< 0: none); relu: its record of the
+// ReLU tap (NULL: not written).  Returns the colours and the density network's first output.
+template <int LF, int ND, int NC, int FEAT, bool TAPS>
+__device__ __noinline__ float4 fwd_samples_fp32(const MlpPtrs* __restrict__ wp, const float* __restrict__ sm,
+                                                const float* __restrict__ a0, const FeatLayout* __restrict__ feat,
+                                                int64_t b, float dx, float dy, float dz, float sh_mult,
+                                                uint32_t* __restrict__ relu) {
+  using A = ArchF<LF, ND, NC>;
+  const int lane = threadIdx.x & 63, g = lane >> 4, s = lane & 15;
+  const bool al = wp->aligned16;
+  auto d_col = [&](int tp) { return 16 * tp + 4 * g; };
+  float a0r[LF / 4];
+  load_enc<LF, FEAT>(a0, *feat, b, b >= 0, g, a0r);
+  floatx4 x[4], h[4];
+#pragma unroll
+  for (int q = 0; q < LF / 16; ++q) x[q] = floatx4{a0r[4 * q], a0r[4 * q + 1], a0r[4 * q + 2], a0r[4 * q + 3]};
+  auto tap = [&](int layer, const floatx4 (&v)[4]) {
+    if constexpr (TAPS) tap_relu(relu, layer, v, g);
+  };
+  fwd_fp32<4, LF / 16>(wp->W[FFN_WD_IN], al, LF, sm + A::b_off(FFN_WD_IN), x, h, g, s, true,
+                       [&](int q) { return LF / 4 * g + 4 * q; });
+  tap(0, h);
+#pragma unroll
+  for (int i = 1; i < ND; ++i) {
+    const int k = i == 1 ? FFN_WD_01 : FFN_WD_12;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = h[t];
+    fwd_fp32<4, 4>(wp->W[k], al, FFN_M, sm + A::b_off(k), x, h, g, s, true, d_col);
+    tap(i, h);
+  }
+  floatx4 o1[4];
+  fwd_fp32<1, 4>(wp->W[FFN_WD_OUT], al, FFN_M, sm + A::b_off(FFN_WD_OUT), h, o1, g, s, false, d_col);
+  const float dir[3] = {dx, dy, dz};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o1[1][r] = sh_component(dir, 4 * g + r) * sh_mult;
+  fwd_fp32<4, 2>(wp->W[FFN_WC_IN], al, FFN_C_IN, sm + A::b_off(FFN_WC_IN), o1, h, g, s, true, d_col);
+  tap(3, h);
+#pragma unroll
+  for (int i = 1; i < NC; ++i) {
+    const int k = i == 1 ? FFN_WC_01 : (i == 2 ? FFN_WC_12 : FFN_WC_23);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = h[t];
+    fwd_fp32<4, 4>(wp->W[k], al, FFN_M, sm + A::b_off(k), x, h, g, s, true, d_col);
+    tap(3 + i, h);
+  }
+  float rgb[3];
+  fwd_color_out(sm + A::out_off(), sm + A::b_off(FFN_WC_OUT), A::OUT_P, h, g, s, rgb);
+  return make_float4(rgb[0], rgb[1], rgb[2], o1[0][0]);
+}
+
+// forward of the wavefront's 16 samples through both networks on the split products; hd, hc: the hidden activations (for
+// the ReLU tap).  Returns the samples (bit per sample) whose sums are not finite, to be done again by fwd_samples_fp32.
 template <int LF, int ND, int NC>
-__device__ __forceinline__ uint32_t fwd_samples(const float* __restrict__ sm, const float (&a0r)[LF / 4],
+__device__ __forceinline__ uint32_t fwd_samples_split(const float* __restrict__ sm, const float (&a0r)[LF / 4],
                                             const float (&dirv)[3], float sh_mult, int g, int s, floatx4 (&hd)[ND][4],
                                             floatx4 (&hc)[NC][4], float& dout0, float (&rgb)[3]) {
-  static_assert(ND <= 2 && NC == 2, "the layers redo_samples keeps");
   using A = ArchF<LF, ND, NC>;
   constexpr int PL = A::plane(), KB0 = A::cols(FFN_WD_IN) / 32;
   // an offset of zero that the compiler cannot see through: it would read the weights before the caller's loop and
@@ -224,14 +252,12 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_fwd(MlpPtrs wp, const float* __
   }
   if ((int64_t)blockIdx.x * 16 >= n) return;  // no samples for this block: skip staging the weights
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
-  const uint32_t always = __syncthreads_and(stage_split<LF, ND, NC>(smv, wp, tid)) ? 0u : 0xFFFFu;
+  const bool split_ok = __syncthreads_and(stage_split<LF, ND, NC>(smv, wp, tid));
   // groups of 16 samples: a block's first, then its second ..., so that few groups spread over the blocks
   for (int64_t grp = (int64_t)blockIdx.x + (int64_t)gridDim.x * wave; grp * 16 < n;
        grp += (int64_t)gridDim.x * MLP_VIEW_WAVES) {
     const int64_t b = grp * 16 + s;
     const bool valid = b < n;
-    float a0r[LF / 4];
-    load_enc<LF, FEAT>(a0, feat, b, valid, g, a0r);
     float dirv[3] = {0.0f, 0.0f, 1.0f};
     if (valid) {
       const float4 rd = rays[2 * (size_t)ray_ids[b] + 1];
@@ -239,10 +265,26 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_fwd(MlpPtrs wp, const float* __
       dirv[1] = rd.y;
       dirv[2] = rd.z;
     }
-    floatx4 hd[ND][4], hc[NC][4];
     float dout0, c[3];
-    const uint32_t redo = always | fwd_samples<LF, ND, NC>(smv, a0r, dirv, sh_mult, g, s, hd, hc, dout0, c);
-    if (redo) redo_samples<LF, ND, NC, FEAT>(wp, a0, feat, 16 * grp, n, dirv, sh_mult, lane, redo, hd, hc, dout0, c);
+    uint32_t redo = 0xFFFFu;
+    if (split_ok) {
+      float a0r[LF / 4];
+      load_enc<LF, FEAT>(a0, feat, b, valid, g, a0r);
+      floatx4 hd[ND][4], hc[NC][4];
+      redo = fwd_samples_split<LF, ND, NC>(smv, a0r, dirv, sh_mult, g, s, hd, hc, dout0, c);
+    }
+    if (redo) {  // the other samples keep their results, which so do not depend on their neighbours
+      const MlpPtrs w = wp;  // (a copy of its own: a kernel argument whose address is taken is read from memory everywhere)
+      const FeatLayout lay = feat;
+      const float4 f = fwd_samples_fp32<LF, ND, NC, FEAT, false>(&w, smv, a0, &lay, valid ? b : -1, dirv[0],
+                                                                 dirv[1], dirv[2], sh_mult, nullptr);
+      if ((redo >> s) & 1u) {
+        c[0] = f.x;
+        c[1] = f.y;
+        c[2] = f.z;
+        dout0 = f.w;
+      }
+    }
     if (g == 0 && valid) {
       sigma[b] = softplus(fminf(fmaxf(dout0, -10.0f), 10.0f));
       rgb[3 * b] = c[0];
@@ -260,7 +302,7 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_view(MlpArgs a) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
   const int log2S = a.log2S;
   const uint64_t n_samples = (uint64_t)a.num_rays << log2S;
-  const uint32_t always = __syncthreads_and(stage_split<LF, ND, NC>(smv, a.w, tid)) ? 0u : 0xFFFFu;
+  const bool split_ok = __syncthreads_and(stage_split<LF, ND, NC>(smv, a.w, tid));
   float* sSig = smv + A::w_floats() + 256 * wave;  // sigma[64], rgb[64][3] of the wavefront's tile
   float* sRgb = sSig + 64;
   const float Dhalf = half_box_diagonal(a.c);
@@ -274,33 +316,45 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_view(MlpArgs a) {
 #pragma unroll 1
   for (; ti < n_full; ti += step) {
     const int64_t tile = a.tile_order ? (int64_t)a.tile_order[ti] : ti;
-    const CompLane CL = load_comp_lane<SC>(a, tile, lane, true, n_samples, log2S, false);
 #pragma unroll 1
     for (int cb = 0; cb < 4; ++cb) {
       const int col = 16 * cb + s;
       const int64_t b = tile * 64 + col;
       const bool valid = (uint64_t)b < n_samples;
-      float a0r[LF / 4];
-      load_enc<LF, FEAT>(a.a0, a.feat, b, valid, g, a0r);
       const float4 rd = a.rays[2 * (valid ? (b >> log2S) : 0) + 1];
       const float dirv[3] = {rd.x, rd.y, rd.z};
-      const float dt_b = valid ? a.DTs[b] : 0.0f;
-      floatx4 hd[ND][4], hc[NC][4];
       float dout0, c[3];
-      const uint32_t redo = always | fwd_samples<LF, ND, NC>(smv, a0r, dirv, a.sh_mult, g, s, hd, hc, dout0, c);
-      if (redo)
-        redo_samples<LF, ND, NC, FEAT>(a.w, a.a0, a.feat, tile * 64 + 16 * cb, (int64_t)n_samples, dirv, a.sh_mult,
-                                       lane, redo, hd, hc, dout0, c);
-      if constexpr (TAPS) {
-        if (a.t_relu) {
-          uint32_t* rec = valid ? a.t_relu + (int64_t)RELU_WORDS * b : nullptr;
+      uint32_t* rec = TAPS && a.t_relu && valid ? a.t_relu + (int64_t)RELU_WORDS * b : nullptr;
+      uint32_t redo = 0xFFFFu;
+      if (split_ok) {
+        float a0r[LF / 4];
+        load_enc<LF, FEAT>(a.a0, a.feat, b, valid, g, a0r);
+        floatx4 hd[ND][4], hc[NC][4];
+        redo = fwd_samples_split<LF, ND, NC>(smv, a0r, dirv, a.sh_mult, g, s, hd, hc, dout0, c);
+        if constexpr (TAPS) {
+          if (a.t_relu) {
 #pragma unroll
-          for (int i = 0; i < ND; ++i) tap_relu(rec, i, hd[i], g);
+            for (int i = 0; i < ND; ++i) tap_relu(rec, i, hd[i], g);
 #pragma unroll
-          for (int i = 0; i < NC; ++i) tap_relu(rec, 3 + i, hc[i], g);
+            for (int i = 0; i < NC; ++i) tap_relu(rec, 3 + i, hc[i], g);
+          }
+        }
+      }
+      if (redo) {
+        const bool mine = (redo >> s) & 1u;
+        const MlpPtrs w = a.w;  // (as in k_mlp_fwd)
+        const FeatLayout lay = a.feat;
+        const float4 f = fwd_samples_fp32<LF, ND, NC, FEAT, TAPS>(&w, smv, a.a0, &lay, valid ? b : -1, rd.x, rd.y,
+                                                                  rd.z, a.sh_mult, mine ? rec : nullptr);
+        if (mine) {
+          c[0] = f.x;
+          c[1] = f.y;
+          c[2] = f.z;
+          dout0 = f.w;
         }
       }
       if (g == 0) {
+        const float dt_b = valid ? a.DTs[b] : 0.0f;
         const float sig = softplus(fminf(fmaxf(dout0, -10.0f), 10.0f));
         sSig[col] = dt_b <= 0.0f ? 0.0f : sig;
         sRgb[3 * col] = c[0];
@@ -308,6 +362,7 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_view(MlpArgs a) {
         sRgb[3 * col + 2] = c[2];
       }
     }
+    const CompLane CL = load_comp_lane<SC>(a, tile, lane, true, n_samples, log2S, false);
     wave_lds_sync();
     float dLds, dLdc[3];
     composite_tile<TAPS, SC>(a, sSig, sRgb, CL, lane, 0, true, false, false, Dhalf, dLds, dLdc);

@@ -132,3 +132,82 @@ def test_infinities(what):
     assert np.mean(used == used_ref) > 0.99  # as test_render_matches_oracle
     same = used == used_ref
     np.testing.assert_allclose(out[same], ref[same], rtol=1e-3, atol=2e-5)
+
+
+# Weights outside the split's range, which the fp32 instruction takes: a layer scaled down so far that its weights' and
+# outputs' lower bfloat16 planes are below the smallest normal number, and the next one up again; one weight alone.
+@pytest.mark.parametrize("what", ["scaled", "one small", "one large"])
+@pytest.mark.parametrize("L,F,nd", [(8, 2, 1), (8, 4, 2), (16, 4, 2)])
+def test_weights_outside_the_split(what, L, F, nd):
+    from gpu_helpers import GpuModel
+    spec = spec_cfg0(n_levels=L, f_per_level=F, log2_T=[10] * L, res=[4.0 + 3 * i for i in range(L)], nd=nd)
+    p = random_params(spec, seed=F + nd)
+    if what == "scaled":
+        up = "Wd_01" if nd > 1 else "Wd_out"
+        p["Wd_in"] *= np.float32(2.0 ** -118)
+        p["bd_0"] *= np.float32(2.0 ** -118)
+        p[up] *= np.float32(2.0 ** 118)
+    elif what == "one small":
+        p["Wc_in"][3, 5] = np.float32(1e-38)
+    else:  # its input is zero: neuron 9 of the density layer never fires
+        p["Wd_in"][9], p["bd_0"][9] = 0.0, -1.0
+        p["Wd_01" if nd > 1 else "Wd_out"][4, 9] = np.float32(1e38)
+    n, S = 67, 32
+    rays = look_at_rays(n, spec, seed=5, miss_frac=0.1)
+    sc = default_scalars(do_train=0, occ_strength=0.0)
+    print(f"[view range] {what} LF={L * F} nd={nd}", flush=True)
+    _, t = GpuModel(spec, p).train_step(rays, np.zeros((n, 4), np.float32), S, sc, taps=True)
+    ref = forward64(spec, p, t["a0"].reshape(-1, L * F), np.repeat(rays[:, 4:7], S, axis=0), sc["sh_multiplier"])
+    on = t["DTs"].reshape(-1) > 0
+    err = view_error(t["sigma"].reshape(-1), t["rgb"].reshape(-1, 3), *ref, on)
+    # two fp32 sums a layer of at most 64 products on K = 4 instructions: twice the split sums' error (VIEW_TOL)
+    assert max(err) <= 2 * VIEW_TOL
+    # the ReLU tap comes from the pass that counts: a hidden unit above zero by more than its rounding is on
+    h = t["a0"].reshape(-1, L * F).astype(np.float64) @ p["Wd_in"].astype(np.float64).T + p["bd_0"]
+    word = t["relu"].reshape(-1, t["relu"].shape[-1])[:, 0]
+    sure = np.abs(h[:, :32]) > 1e-5 * np.abs(h).max()
+    bits = (word[:, None] >> np.arange(32, dtype=np.uint32)) & 1
+    np.testing.assert_array_equal((bits == 1)[sure & on[:, None]], (h[:, :32] > 0)[sure & on[:, None]])
+
+
+# A diverged model ("not a number" in a weight): its outputs say so, and its previews take about as long as the fp32
+# instruction makes them: 64 rays' samples a wavefront at twice the matrix cycles, not a sample at a time.
+def test_diverged_model():
+    import torch
+    from gpu_helpers import GpuModel
+    import ffn_lib as fl
+    import ctypes as C
+    spec = spec_cfg0()
+    ms = {}
+    n, S = 16384, 64
+    rays = look_at_rays(n, spec, seed=2, miss_frac=0.0)
+    rays_t, out = torch.from_numpy(rays).cuda(), torch.zeros((n, 4), device="cuda")
+    sc = fl.FfnStepScalars()
+    sc.sh_multiplier, sc.rng_seed, sc.do_train = 1.0, 5, 0
+    for what in ("finite", "nan"):
+        p = random_params(spec, seed=3)
+        p["occ_in"][:] = 0xFFFFFFFF
+        if what == "nan":
+            p["Wc_in"][7, 3] = np.nan
+        m = GpuModel(spec, p)
+        print(f"[view diverged] {what}", flush=True)
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = 1e9
+        for _ in range(5):
+            ev[0].record()
+            fl.check(m.lib.ffn_train_step(m.h.h, fl.ptr(rays_t), fl.ptr(out), fl.ptr(out), n, S, C.byref(sc), None,
+                                          fl.stream_ptr()), "view")
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]))
+        ms[what] = best
+        if what == "nan":
+            _, t = m.train_step(rays[:65], np.zeros((65, 4), np.float32), 32, default_scalars(do_train=0), taps=True)
+            f = GpuModel(spec, {**p, "Wc_in": np.nan_to_num(p["Wc_in"])})
+            _, tf = f.train_step(rays[:65], np.zeros((65, 4), np.float32), 32, default_scalars(do_train=0), taps=True)
+            # the density network is not touched: same sums but for the instruction they are taken on
+            on = t["DTs"].reshape(-1) > 0
+            np.testing.assert_allclose(t["sigma"].reshape(-1)[on], tf["sigma"].reshape(-1)[on], rtol=1e-5, atol=1e-6)
+            assert not np.allclose(t["rgb"].reshape(-1, 3)[on], tf["rgb"].reshape(-1, 3)[on], equal_nan=True)
+    print(f"[view diverged] {ms['finite']:.3f} ms finite, {ms['nan']:.3f} ms not", flush=True)
+    assert ms["nan"] < 5 * ms["finite"]
