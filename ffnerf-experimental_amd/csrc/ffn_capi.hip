@@ -1153,7 +1153,7 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
                                     LF, h->cfg.nd, h->cfg.nc, fwd_blocks, st, n_dev));
     else
       FFN_HIP(ffn::launch_mlp_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, sc->sh_multiplier, sigma, rgb,
-                                  LF, h->cfg.nd, h->cfg.nc, fwd_blocks, st, n_dev));
+                                  true, LF, h->cfg.nd, h->cfg.nc, fwd_blocks, st, n_dev));
     ffn::CompMarchArgs ca{};
     ca.offsets = off;
     ca.counts = counts;
@@ -1359,8 +1359,8 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
     const ffn::FeatLayout feat = ffn::level_major(n, h->dc.F);
     FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, a0, feat, nullptr, &dl, st, n_dev));
     const int nb = grid_blocks(h, 1, (n + 15) / 16);
-    FFN_HIP(ffn::launch_mlp_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, mp->sh_multiplier, sigma, rgb, LF,
-                                h->cfg.nd, h->cfg.nc, nb, st, n_dev));
+    FFN_HIP(ffn::launch_mlp_fwd(h->dc, w, a0, feat, (const float4*)rays, ids, n, mp->sh_multiplier, sigma, rgb,
+                                false, LF, h->cfg.nd, h->cfg.nc, nb, st, n_dev));
     FFN_HIP(ffn::launch_render_composite(off, counts, num_rays, sigma, rgb, mp->dt, mp->T_stop, state, acc,
                                          n_samples, st, n_dev));
   }

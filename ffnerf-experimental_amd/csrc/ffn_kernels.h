@@ -331,11 +331,11 @@ hipError_t launch_make_batch_weighted(const float* images, uint32_t n_images, ui
                                       float4* targets, uint32_t* pixel_ids, hipStream_t st);
 
 // forward-only MLP over n samples: encodings a0 (layout feat), view directions from rays[ray_ids[b]];
-// sigma[n], rgb[n][3]
+// sigma[n], rgb[n][3].  train: the sums of the training kernel's own forward, bit for bit (launch_mlp_marched follows)
 // (n_dev may be NULL: the count is then n; else min(n, *n_dev), read on the device)
 hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
                           const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
-                          float* rgb, int LF, int nd, int nc, int n_blocks, hipStream_t st,
+                          float* rgb, bool train, int LF, int nd, int nc, int n_blocks, hipStream_t st,
                           const uint32_t* n_dev = nullptr);
 
 // fused MLP forward + compositing + loss + backward + proposals, per 64-sample tile

@@ -4,24 +4,24 @@
 // Reference: ffnerf_OG.cl:1373-1466 (MLP fwd), 1505-1591 (compositing).
 //
 // MI355X design
-//   * The layers' products are fp32 products on bfloat16 matrix instructions, three planes a value and eight terms a
-//     product (ffn_mlp_split.h): half the matrix cycles of the fp32 instruction, beside vector instructions, and sums
-//     no further from 64 bits.
+//   * Where no training follows, the layers' products are fp32 products on bfloat16 matrix instructions, three planes
+//     a value and eight terms a product (ffn_mlp_split.h): half the matrix cycles of the fp32 instruction, beside
+//     vector instructions, and sums no further from 64 bits.  The marched step's forward has the training kernel's
+//     own sums (k_mlp_fwd).
 //   * A block of 16 wavefronts, one per CU, shares the weights in LDS (three bfloat16 planes, K-ordered rows); a
 //     wavefront works alone (no barrier after the staging): 16 samples through all layers, activations in registers
 //     in the D layout of one layer = the B operand of the next (K slot j of lane group g in block kb is neuron
 //     32 kb + 16 (j / 4) + 4 g + j % 4).  A forward-only step's wavefront takes a tile of 64 samples as four such
 //     groups and composites it on its 64 lanes.
 //   * What bounds it: matrix instructions and the vector instructions of the splits (5.5 per value) about alike.
-//     Measured against the fp32-MFMA forward (three blocks of four wavefronts per CU, 16-byte weight staging):
-//     880,000 marched samples of the 32-feature model 167 -> 108 us, a frame's first round of 3.0M samples 542 ->
-//     347; a preview of 590,000 samples of the 64-feature model with two density layers 166 -> 97 us.
+//     Measured against the fp32-MFMA forward (three blocks of four wavefronts per CU, 16-byte weight staging): a
+//     frame's first round of 3.0M samples 542 -> 418 us; a preview of 590,000 samples of the 64-feature model with two
+//     density layers 166 -> 102 us.
 //   * The split does not hold infinities (their m is not a number), and loses the lower planes of operands near the
 //     smallest numbers.  A wavefront sees infinities in its sums (every sum of a sample with such a value is not a
 //     number) and does those samples again on the fp32 instruction, with the weights from memory; a block whose staged
-//     weights are not all in the split's range takes the fp32 instruction alone
-//     (a preview of 2^20 samples of a diverged model: 0.58 ms, in the split's range 0.32; a sample and a lane per neuron
-//     at a time it took 15.8).
+//     weights are not all in the split's range takes the fp32 instruction alone (a preview of 2^20 samples of a
+//     diverged model: 0.58 ms, in the split's range 0.32; a sample and a lane per neuron at a time it took 15.8).
 #include "ffn_device.h"
 #include "ffn_kernels.h"
 #include "ffn_mlp_common.h"
@@ -31,30 +31,40 @@ namespace ffn {
 
 constexpr int VIEW_NT = 64 * MLP_VIEW_WAVES;
 
+// LDS: the colour output layer, the biases, then the other layers' weights (three planes or fp32 rows)
 template <int LF_, int ND_, int NC_>
 struct ArchF {
   static constexpr int LF = LF_, ND = ND_, NC = NC_;
+  static constexpr int OUT_P = FFN_M + 4;  // the colour output layer: four fp32 rows (the last one zero)
+  static constexpr int b_off(int k) {
+    int o = 4 * OUT_P;
+    for (int j = 0; j < k; ++j) o += layer_active(j, ND, NC) ? (j == FFN_WC_OUT ? 4 : layer_out(j)) : 0;
+    return o;
+  }
+  static constexpr int w_base() { return b_off(FFN_N_LAYERS); }
+  static_assert(w_base() % 4 == 0, "16-byte aligned weights");
   // layers on the split products (the colour output layer's three rows stay on fp32 4x4x1 MFMAs)
   static constexpr bool split(int k) { return layer_active(k, ND, NC) && k != FFN_WC_OUT; }
   static constexpr int cols(int k) { return layer_in(k, LF) < 32 ? 32 : layer_in(k, LF); }
   // row pitch in halves: the 8-half pad keeps the 16-byte reads aligned and spreads a tile's rows over the banks
   static constexpr int pitch(int k) { return cols(k) + 8; }
   static constexpr int sz(int k) { return split(k) ? layer_out(k) * pitch(k) : 0; }
-  static constexpr int w_off(int k) {  // of plane 0, in halves; plane p follows at p * plane()
+  static constexpr int w_off(int k) {  // of plane 0, in halves after w_base; plane p follows at p * plane()
     int o = 0;
     for (int j = 0; j < k; ++j) o += sz(j);
     return o;
   }
   static constexpr int plane() { return w_off(FFN_N_LAYERS); }
-  static constexpr int OUT_P = FFN_M + 4;  // the colour output layer: four fp32 rows (the last one zero)
-  static constexpr int out_off() { return 3 * plane() / 2; }  // in floats
-  static constexpr int b_off(int k) {
-    int o = out_off() + 4 * OUT_P;
-    for (int j = 0; j < k; ++j) o += layer_active(j, ND, NC) ? (j == FFN_WC_OUT ? 4 : layer_out(j)) : 0;
+  static constexpr int w_floats() { return w_base() + 3 * plane() / 2; }
+  static_assert(plane() % 8 == 0, "16-byte aligned planes");
+  // the same as fp32 rows (pitch in + 4, as in the training kernel)
+  static constexpr int pitch32(int k) { return layer_in(k, LF) + 4; }
+  static constexpr int off32(int k) {
+    int o = w_base();
+    for (int j = 0; j < k; ++j) o += split(j) ? layer_out(j) * pitch32(j) : 0;
     return o;
   }
-  static constexpr int w_floats() { return b_off(FFN_N_LAYERS); }
-  static_assert(plane() % 8 == 0, "16-byte aligned planes");
+  static constexpr int floats32() { return off32(FFN_N_LAYERS); }
 };
 
 // position of input neuron n in a layer's K-ordered row: for the first layer lane group g holds neurons (LF / 4) g
@@ -82,14 +92,14 @@ __device__ __forceinline__ bool split_holds(float w) {
 template <int LF, int ND, int NC>
 __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtrs& wp, int tid) {
   using A = ArchF<LF, ND, NC>;
-  __bf16* sW = reinterpret_cast<__bf16*>(sm);
+  __bf16* sW = reinterpret_cast<__bf16*>(sm + A::w_base());
   bool holds = true;
   read_weights<LF, ND, NC, VIEW_NT>(
       wp, tid,
       [&](auto K, int o, int i, const float4& v) {
         constexpr int k = K;
         if constexpr (k == FFN_WC_OUT) {
-          *reinterpret_cast<float4*>(sm + A::out_off() + o * A::OUT_P + i) = v;
+          *reinterpret_cast<float4*>(sm + o * A::OUT_P + i) = v;
         } else {
           const float x[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -98,7 +108,7 @@ __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtr
         }
       },
       [&](auto K, int o, float v) { sm[A::b_off(K) + o] = v; });
-  if (tid < A::OUT_P) sm[A::out_off() + 3 * A::OUT_P + tid] = 0.0f;
+  if (tid < A::OUT_P) sm[3 * A::OUT_P + tid] = 0.0f;
   if constexpr (LF == 16) {  // the first layer's rows have 16 neurons in 32 positions
     constexpr int P = A::pitch(FFN_WD_IN);
     for (int e = tid; e < 3 * FFN_M * 4; e += VIEW_NT) {
@@ -107,6 +117,21 @@ __device__ __forceinline__ bool stage_split(float* __restrict__ sm, const MlpPtr
     }
   }
   return holds;
+}
+
+// the same with fp32 rows
+template <int LF, int ND, int NC>
+__device__ __forceinline__ void stage_fp32(float* __restrict__ sm, const MlpPtrs& wp, int tid) {
+  using A = ArchF<LF, ND, NC>;
+  read_weights<LF, ND, NC, VIEW_NT>(
+      wp, tid,
+      [&](auto K, int o, int i, const float4& v) {
+        constexpr int k = K;
+        constexpr int at = k == FFN_WC_OUT ? 0 : A::off32(k), P = k == FFN_WC_OUT ? A::OUT_P : A::pitch32(k);
+        *reinterpret_cast<float4*>(sm + at + o * P + i) = v;
+      },
+      [&](auto K, int o, float v) { sm[A::b_off(K) + o] = v; });
+  if (tid < A::OUT_P) sm[3 * A::OUT_P + tid] = 0.0f;
 }
 
 // out tiles (D layout) = act(W . in + b) on the fp32 instruction, with the sums' order of the training kernels; W: the
@@ -134,28 +159,18 @@ __device__ __forceinline__ void fwd_fp32(const float* __restrict__ W, bool align
   }
 }
 
-// The forward of the wavefront's 16 samples with fp32 products, for samples and weights that the split cannot hold: the
-// weights straight from memory (the caches hold them), the biases and the colour output layer from LDS.  Not inlined:
-// its registers would be spilled on the split's path.  b: the lane's sample (< 0: none); relu: its record of the
-// ReLU tap (NULL: not written).  Returns the colours and the density network's first output.
-template <int LF, int ND, int NC, int FEAT, bool TAPS>
-__device__ __noinline__ float4 fwd_samples_fp32(const MlpPtrs* __restrict__ wp, const float* __restrict__ sm,
-                                                const float* __restrict__ a0, const FeatLayout* __restrict__ feat,
-                                                int64_t b, float dx, float dy, float dz, float sh_mult,
-                                                uint32_t* __restrict__ relu) {
+// forward of the wavefront's 16 samples through both networks with fp32 products, the training kernel's sums bit for
+// bit; W(k): layer k's weights, rows of in + PAD floats.  Returns the colours and the density network's first output.
+template <int LF, int ND, int NC, int PAD, class Wt, class Tap>
+__device__ __forceinline__ float4 fwd_nets_fp32(Wt W, bool al, const float* __restrict__ sm,
+                                                const float (&a0r)[LF / 4], const float (&dir)[3], float sh_mult,
+                                                int g, int s, Tap tap) {
   using A = ArchF<LF, ND, NC>;
-  const int lane = threadIdx.x & 63, g = lane >> 4, s = lane & 15;
-  const bool al = wp->aligned16;
   auto d_col = [&](int tp) { return 16 * tp + 4 * g; };
-  float a0r[LF / 4];
-  load_enc<LF, FEAT>(a0, *feat, b, b >= 0, g, a0r);
   floatx4 x[4], h[4];
 #pragma unroll
   for (int q = 0; q < LF / 16; ++q) x[q] = floatx4{a0r[4 * q], a0r[4 * q + 1], a0r[4 * q + 2], a0r[4 * q + 3]};
-  auto tap = [&](int layer, const floatx4 (&v)[4]) {
-    if constexpr (TAPS) tap_relu(relu, layer, v, g);
-  };
-  fwd_fp32<4, LF / 16>(wp->W[FFN_WD_IN], al, LF, sm + A::b_off(FFN_WD_IN), x, h, g, s, true,
+  fwd_fp32<4, LF / 16>(W(FFN_WD_IN), al, LF + PAD, sm + A::b_off(FFN_WD_IN), x, h, g, s, true,
                        [&](int q) { return LF / 4 * g + 4 * q; });
   tap(0, h);
 #pragma unroll
@@ -163,27 +178,44 @@ __device__ __noinline__ float4 fwd_samples_fp32(const MlpPtrs* __restrict__ wp, 
     const int k = i == 1 ? FFN_WD_01 : FFN_WD_12;
 #pragma unroll
     for (int t = 0; t < 4; ++t) x[t] = h[t];
-    fwd_fp32<4, 4>(wp->W[k], al, FFN_M, sm + A::b_off(k), x, h, g, s, true, d_col);
+    fwd_fp32<4, 4>(W(k), al, FFN_M + PAD, sm + A::b_off(k), x, h, g, s, true, d_col);
     tap(i, h);
   }
   floatx4 o1[4];
-  fwd_fp32<1, 4>(wp->W[FFN_WD_OUT], al, FFN_M, sm + A::b_off(FFN_WD_OUT), h, o1, g, s, false, d_col);
-  const float dir[3] = {dx, dy, dz};
+  fwd_fp32<1, 4>(W(FFN_WD_OUT), al, FFN_M + PAD, sm + A::b_off(FFN_WD_OUT), h, o1, g, s, false, d_col);
 #pragma unroll
   for (int r = 0; r < 4; ++r) o1[1][r] = sh_component(dir, 4 * g + r) * sh_mult;
-  fwd_fp32<4, 2>(wp->W[FFN_WC_IN], al, FFN_C_IN, sm + A::b_off(FFN_WC_IN), o1, h, g, s, true, d_col);
+  fwd_fp32<4, 2>(W(FFN_WC_IN), al, FFN_C_IN + PAD, sm + A::b_off(FFN_WC_IN), o1, h, g, s, true, d_col);
   tap(3, h);
 #pragma unroll
   for (int i = 1; i < NC; ++i) {
     const int k = i == 1 ? FFN_WC_01 : (i == 2 ? FFN_WC_12 : FFN_WC_23);
 #pragma unroll
     for (int t = 0; t < 4; ++t) x[t] = h[t];
-    fwd_fp32<4, 4>(wp->W[k], al, FFN_M, sm + A::b_off(k), x, h, g, s, true, d_col);
+    fwd_fp32<4, 4>(W(k), al, FFN_M + PAD, sm + A::b_off(k), x, h, g, s, true, d_col);
     tap(3 + i, h);
   }
   float rgb[3];
-  fwd_color_out(sm + A::out_off(), sm + A::b_off(FFN_WC_OUT), A::OUT_P, h, g, s, rgb);
+  fwd_color_out(sm, sm + A::b_off(FFN_WC_OUT), A::OUT_P, h, g, s, rgb);
   return make_float4(rgb[0], rgb[1], rgb[2], o1[0][0]);
+}
+
+// the same for samples and weights that the split cannot hold: the weights straight from memory (the caches hold
+// them), the biases and the colour output layer from LDS.  Not inlined: its registers would be spilled on the split's
+// path.  b: the lane's sample (< 0: none); relu: its record of the ReLU tap (NULL: not written).
+template <int LF, int ND, int NC, int FEAT, bool TAPS>
+__device__ __noinline__ float4 fwd_samples_fp32(const MlpPtrs* __restrict__ wp, const float* __restrict__ sm,
+                                                const float* __restrict__ a0, const FeatLayout* __restrict__ feat,
+                                                int64_t b, float dx, float dy, float dz, float sh_mult,
+                                                uint32_t* __restrict__ relu) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, s = lane & 15;
+  float a0r[LF / 4];
+  load_enc<LF, FEAT>(a0, *feat, b, b >= 0, g, a0r);
+  const float dir[3] = {dx, dy, dz};
+  return fwd_nets_fp32<LF, ND, NC, 0>([&](int k) { return wp->W[k]; }, wp->aligned16, sm, a0r, dir, sh_mult, g, s,
+                                      [&](int layer, const floatx4 (&v)[4]) {
+                                        if constexpr (TAPS) tap_relu(relu, layer, v, g);
+                                      });
 }
 
 // forward of the wavefront's 16 samples through both networks on the split products; hd, hc: the hidden activations (for
@@ -199,7 +231,7 @@ __device__ __forceinline__ uint32_t fwd_samples_split(const float* __restrict__ 
   int zero = 0;
   __asm__ volatile("" : "+s"(zero));
   sm += zero;
-  const __bf16* sW = reinterpret_cast<const __bf16*>(sm);
+  const __bf16* sW = reinterpret_cast<const __bf16*>(sm + A::w_base());
   float bad = 0.0f;
   Split8 x0[KB0];
 #pragma unroll
@@ -209,7 +241,8 @@ __device__ __forceinline__ uint32_t fwd_samples_split(const float* __restrict__ 
     for (int j = 0; j < 8; ++j) v[j] = 8 * kb + j < LF / 4 ? a0r[8 * kb + j] : 0.0f;
     x0[kb] = split8(v);
   }
-  fwd_split<4, KB0>(sW + A::w_off(FFN_WD_IN), PL, A::pitch(FFN_WD_IN), sm + A::b_off(FFN_WD_IN), x0, hd[0], g, s, true, bad);
+  fwd_split<4, KB0>(sW + A::w_off(FFN_WD_IN), PL, A::pitch(FFN_WD_IN), sm + A::b_off(FFN_WD_IN), x0, hd[0], g, s, true,
+                    bad);
   Split8 x[2];
 #pragma unroll
   for (int i = 1; i < ND; ++i) {
@@ -228,18 +261,23 @@ __device__ __forceinline__ uint32_t fwd_samples_split(const float* __restrict__ 
   for (int r = 0; r < 4; ++r) cin[1][r] = sh_component(dirv, 4 * g + r) * sh_mult;
   Split8 xc[1];
   split_tiles(cin, xc);
-  fwd_split<4, 1>(sW + A::w_off(FFN_WC_IN), PL, A::pitch(FFN_WC_IN), sm + A::b_off(FFN_WC_IN), xc, hc[0], g, s, true, bad);
+  fwd_split<4, 1>(sW + A::w_off(FFN_WC_IN), PL, A::pitch(FFN_WC_IN), sm + A::b_off(FFN_WC_IN), xc, hc[0], g, s, true,
+                  bad);
 #pragma unroll
   for (int i = 1; i < NC; ++i) {
     const int k = i == 1 ? FFN_WC_01 : (i == 2 ? FFN_WC_12 : FFN_WC_23);
     split_tiles(hc[i - 1], x);
     fwd_split<4, 2>(sW + A::w_off(k), PL, A::pitch(k), sm + A::b_off(k), x, hc[i], g, s, true, bad);
   }
-  fwd_color_out(sm + A::out_off(), sm + A::b_off(FFN_WC_OUT), A::OUT_P, hc[NC - 1], g, s, rgb);
+  fwd_color_out(sm, sm + A::b_off(FFN_WC_OUT), A::OUT_P, hc[NC - 1], g, s, rgb);
   return (uint32_t)__ballot(bad != 0.0f) & 0xFFFFu;  // not a number in all four lanes of a sample alike
 }
 
-template <int LF, int ND, int NC, int FEAT>
+// The forward over indexed samples.  SPLIT: the render's.  Without it the marched training step's, whose backward
+// recomputes the activations in fp32 (k_mlp): the forward's sums are the same bit for bit, so the loss gradients belong
+// to the activations and ReLU branches that the backward uses (880,000 samples of the 32-feature model: 160 us; with the
+// split's sums the step, 1.45 ms, was not 1 % faster).
+template <int LF, int ND, int NC, int FEAT, bool SPLIT>
 __global__ __launch_bounds__(VIEW_NT) void k_mlp_fwd(MlpPtrs wp, const float* __restrict__ a0, FeatLayout feat,
                                                      const float4* __restrict__ rays,
                                                      const uint32_t* __restrict__ ray_ids, int64_t n, float sh_mult,
@@ -252,7 +290,13 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_fwd(MlpPtrs wp, const float* __
   }
   if ((int64_t)blockIdx.x * 16 >= n) return;  // no samples for this block: skip staging the weights
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
-  const bool split_ok = __syncthreads_and(stage_split<LF, ND, NC>(smv, wp, tid));
+  bool split_ok = false;
+  if constexpr (SPLIT) {
+    split_ok = __syncthreads_and(stage_split<LF, ND, NC>(smv, wp, tid));
+  } else {
+    stage_fp32<LF, ND, NC>(smv, wp, tid);
+    __syncthreads();
+  }
   // groups of 16 samples: a block's first, then its second ..., so that few groups spread over the blocks
   for (int64_t grp = (int64_t)blockIdx.x + (int64_t)gridDim.x * wave; grp * 16 < n;
        grp += (int64_t)gridDim.x * MLP_VIEW_WAVES) {
@@ -267,14 +311,27 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_fwd(MlpPtrs wp, const float* __
     }
     float dout0, c[3];
     uint32_t redo = 0xFFFFu;
-    if (split_ok) {
+    if constexpr (!SPLIT) {
+      float a0r[LF / 4];
+      load_enc<LF, FEAT>(a0, feat, b, valid, g, a0r);
+      int zero = 0;  // as in fwd_samples_split
+      __asm__ volatile("" : "+s"(zero));
+      const float* sm = smv + zero;
+      const float4 f = fwd_nets_fp32<LF, ND, NC, 4>([&](int k) { return sm + ArchF<LF, ND, NC>::off32(k); }, true, sm,
+                                                    a0r, dirv, sh_mult, g, s, [](int, const floatx4 (&)[4]) {});
+      c[0] = f.x;
+      c[1] = f.y;
+      c[2] = f.z;
+      dout0 = f.w;
+      redo = 0u;
+    } else if (split_ok) {
       float a0r[LF / 4];
       load_enc<LF, FEAT>(a0, feat, b, valid, g, a0r);
       floatx4 hd[ND][4], hc[NC][4];
       redo = fwd_samples_split<LF, ND, NC>(smv, a0r, dirv, sh_mult, g, s, hd, hc, dout0, c);
     }
-    if (redo) {  // the other samples keep their results, which so do not depend on their neighbours
-      const MlpPtrs w = wp;  // (a copy of its own: a kernel argument whose address is taken is read from memory everywhere)
+    if (SPLIT && redo) {  // the other samples keep their results, which so do not depend on their neighbours
+      const MlpPtrs w = wp;  // (a copy: a kernel argument whose address is taken is read from memory everywhere)
       const FeatLayout lay = feat;
       const float4 f = fwd_samples_fp32<LF, ND, NC, FEAT, false>(&w, smv, a0, &lay, valid ? b : -1, dirv[0],
                                                                  dirv[1], dirv[2], sh_mult, nullptr);
@@ -378,33 +435,38 @@ __global__ __launch_bounds__(VIEW_NT) void k_mlp_view(MlpArgs a) {
 
 // ---------------------------------------------------------------------------
 
-template <int LF, int ND, int NC, int FEAT>
+template <int LF, int ND, int NC, int FEAT, bool SPLIT>
 static hipError_t launch_fwd_f(const MlpPtrs& w, const float* a0, const FeatLayout& feat, const float4* rays,
                                const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma, float* rgb,
                                int n_blocks, hipStream_t st, const uint32_t* n_dev) {
-  const size_t lds = sizeof(float) * (size_t)ArchF<LF, ND, NC>::w_floats();
+  using A = ArchF<LF, ND, NC>;
+  const size_t lds = sizeof(float) * (size_t)(SPLIT ? A::w_floats() : A::floats32());
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_fwd<LF, ND, NC, FEAT>,
+    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_fwd<LF, ND, NC, FEAT, SPLIT>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
-  hipLaunchKernelGGL((k_mlp_fwd<LF, ND, NC, FEAT>), dim3(n_blocks), dim3(VIEW_NT), lds, st, w, a0, feat, rays, ray_ids,
-                     n, sh_mult, sigma, rgb, n_dev);
+  hipLaunchKernelGGL((k_mlp_fwd<LF, ND, NC, FEAT, SPLIT>), dim3(n_blocks), dim3(VIEW_NT), lds, st, w, a0, feat, rays,
+                     ray_ids, n, sh_mult, sigma, rgb, n_dev);
   return hipGetLastError();
 }
 
 template <int LF, int ND, int NC>
 static hipError_t launch_fwd_t(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
                                const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
-                               float* rgb, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
+                               float* rgb, bool train, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
+#define FFN_FWD(F)                                                                                                  \
+  train ? launch_fwd_f<LF, ND, NC, F, false>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev) \
+        : launch_fwd_f<LF, ND, NC, F, true>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev)
   switch (c.F) {
-    case 1: return launch_fwd_f<LF, ND, NC, 1>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
-    case 2: return launch_fwd_f<LF, ND, NC, 2>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
-    case 4: return launch_fwd_f<LF, ND, NC, 4>(w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
+    case 1: return FFN_FWD(1);
+    case 2: return FFN_FWD(2);
+    case 4: return FFN_FWD(4);
     default: return hipErrorInvalidValue;
   }
+#undef FFN_FWD
 }
 
 template <int LF, int ND, int NC, int FEAT, bool TAPS, int SC>
@@ -448,11 +510,12 @@ static hipError_t launch_view_t(const MlpArgs& a, int n_blocks, hipStream_t st) 
 
 hipError_t launch_mlp_fwd(const DevCfg& c, const MlpPtrs& w, const float* a0, const FeatLayout& feat,
                           const float4* rays, const uint32_t* ray_ids, int64_t n, float sh_mult, float* sigma,
-                          float* rgb, int LF, int nd, int nc, int n_blocks, hipStream_t st, const uint32_t* n_dev) {
+                          float* rgb, bool train, int LF, int nd, int nc, int n_blocks, hipStream_t st,
+                          const uint32_t* n_dev) {
   if (n <= 0) return hipSuccess;
 #define X(l, d, nn)                   \
   if (LF == l && nd == d && nc == nn) \
-    return launch_fwd_t<l, d, nn>(c, w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, n_blocks, st, n_dev);
+    return launch_fwd_t<l, d, nn>(c, w, a0, feat, rays, ray_ids, n, sh_mult, sigma, rgb, train, n_blocks, st, n_dev);
   FFN_MLP_FWD_CONFIGS(X)
 #undef X
   return hipErrorInvalidValue;

@@ -61,7 +61,8 @@ def test_a_lost_term_shows(term):
 
 # The split sums may be no further from float64 than the fp32 instruction's (2-norm: of 262,144 sums, so steady to a
 # per cent), nor, for their largest error, than that or one and a half roundings of the sum's terms.  With six of the
-# eight terms a single product is off by up to 4.7e-7 and by 7e-8 in the 2-norm; the fp32 instruction by 6.0e-8 and 2.5e-8.
+# eight terms a single product is off by up to 4.7e-7 and by 7e-8 in the 2-norm; with the fp32 instruction by 6.0e-8 and
+# 2.5e-8.
 @pytest.mark.gpu
 @pytest.mark.parametrize("K", [32, 64])
 @pytest.mark.parametrize("kind", ["dense", "bias", "relu", "positive", "large", "one", "three", "full one",
