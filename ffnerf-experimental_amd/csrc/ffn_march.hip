@@ -485,12 +485,13 @@ __global__ __launch_bounds__(256) void k_march_lattice(MarchArgs a, uint32_t ray
           const float p = L.o[i] + L.t0 * L.d[i];
           L.p0[i] = (p - a.bmin[i]) * inv;
           L.slope[i] = L.d[i] * inv;
-          // With u = 2^-24, A the larger |bound| of the box, D = t1 |d| and s its extent, the coordinate
-          // p0 + tau slope is off by at most u (2 D + A + 9 s) inv cells from the real one at t_k and a face's
-          // exit time by u (3 D + A + 3 s) inv; eps doubles the sum (second-order terms, points a rounding
-          // outside the box).
+          // With u = 2^-24, A the larger |bound| of the box, s its extent and D = max(|t0|, |t1|) |d| (with a negative
+          // t_near the box can lie behind the origin), the coordinate p0 + tau slope is off by at most
+          // u (2 D + A + 9 s) inv cells from the real one at t_k and a face's exit time by u (3 D + A + 3 s) inv; eps
+          // doubles the sum (second-order terms, points a rounding outside the box).
           const float A = fmaxf(fabsf(a.bmin[i]), fabsf(a.bmax[i]));
-          const float e = (5.0f * L.t1 * fabsf(L.d[i]) + 2.0f * A + 12.0f * size) * inv * (2.0f / 16777216.0f);
+          const float far = fmaxf(fabsf(L.t0), fabsf(L.t1));
+          const float e = (5.0f * far * fabsf(L.d[i]) + 2.0f * A + 12.0f * size) * inv * (2.0f / 16777216.0f);
           L.eps = fmaxf(L.eps, e);
           if (!(e < 0.5f)) L.eps = 1.0f;  // (NaN included) every point takes the exact path
         }

@@ -57,3 +57,26 @@ def test_walks_agree(monkeypatch, R, K, max_steps, n):
         t = ora.march_ray(cfg, m, bits, rays[r])
         assert counts[r] == len(t)
         np.testing.assert_array_equal(samples[int(offsets[r]):int(offsets[r]) + len(t), 3], t)
+
+
+# A negative t_near reaches a box behind the ray's origin, where the largest |t| is the entry's: the points that lie
+# within rounding of a cell's face are found from that, and the lattice is as many roundings coarser as it lies away.
+@pytest.mark.parametrize("away", [3.0, 60.0, 1000.0])
+def test_box_behind_the_origin(monkeypatch, away):
+    import ffn_lib as fl
+    from gpu_helpers import GpuModel
+    spec = dict(SPEC, t_near=-1e4)
+    g = GpuModel(spec, random_params(spec, seed=5))
+    R, n = 256, 1500
+    bits = shell_bits(R, seed=R, frac=0.3, half_width=0.1)
+    rays = look_at_rays(n, spec, seed=6, radius=away, miss_frac=0.0)
+    rays[::2, 4:7] *= -1.0  # every other one looks away from the box
+    mp = fl.march_params(R, np.float32(np.sqrt(3.0) / 1024), 1024)
+    res = []
+    for env in ("1", "0"):
+        monkeypatch.setenv("FFN_MARCH_LATTICE", env)
+        print(f"[walks behind] away={away} walk={env}", flush=True)
+        res.append(g.march(rays, bits, mp))
+    assert res[1][0][::2].sum() > 10000
+    for a, b in zip(res[0], res[1]):
+        np.testing.assert_array_equal(a, b)
