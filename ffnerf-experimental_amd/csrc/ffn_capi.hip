@@ -940,6 +940,7 @@ ffn::MarchArgs march_args(Handle* h, const void* rays, uint32_t num_rays, const 
   a.dt = mp->dt;
   a.max_steps = mp->max_steps;
   a.chunk = mp->max_steps;
+  a.lattice = ffn::march_takes_lattice(a);
   return a;
 }
 
@@ -949,7 +950,7 @@ ffn::MarchArgs march_args(Handle* h, const void* rays, uint32_t num_rays, const 
 hipError_t set_march_blocks(Handle* h, ffn::MarchArgs& a, hipStream_t st) {
   const char* env = getenv("FFN_MARCH_BLOCKS");
   a.blocks = a.blocks_use = nullptr;
-  if ((env && env[0] == '0') || ffn::march_takes_lattice(a)) return hipSuccess;
+  if ((env && env[0] == '0') || a.lattice) return hipSuccess;
   const size_t NB = ((size_t)a.res + 7) / 8;
   const size_t words = (NB * NB * NB + 31) / 32;
   hipError_t e = h->m_blocks.ensure(sizeof(uint32_t) * (words + 1));

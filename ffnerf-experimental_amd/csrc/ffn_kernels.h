@@ -230,9 +230,10 @@ hipError_t launch_occ_decay(uint32_t* occ_in, uint32_t* occ_st, uint32_t n_words
                             uint32_t seed, hipStream_t st);
 
 // occupancy bitfield and DDA marcher (no counterpart in the reference; see ffn_march.hip)
+// a ray's walk between the calls of a chunked march, all of which take the same walk (MarchArgs::lattice)
 struct MarchState {
   uint32_t k;      // next lattice index
-  uint32_t cell;   // current cell, 10 bits per axis
+  uint32_t cell;   // current cell, 10 bits per axis (the cell walk's; the lattice walk finds it from k)
   uint32_t n;      // samples emitted so far
   uint32_t flags;  // MARCH_FRESH, MARCH_DONE
 };
@@ -245,6 +246,7 @@ struct MarchArgs {
   const uint32_t* bits;
   int res;
   float dt;
+  bool lattice;              // which walk: march_takes_lattice, decided once for all calls that share `state`
   uint32_t max_steps;        // per ray in total
   uint32_t chunk;            // per call
   MarchState* state;         // NULL: every ray starts fresh and no state is kept
@@ -267,7 +269,7 @@ hipError_t launch_occ_bitfield(const uint32_t* occ, int G, uint32_t q_min, uint3
 // occupied; *use = 1 when at least half the blocks are empty, else 0
 hipError_t launch_occ_blocks(const uint32_t* bits, int R, uint32_t* blocks, uint32_t* use, hipStream_t st);
 hipError_t launch_march(const MarchArgs& a, bool emit, hipStream_t st);
-// whether launch_march takes the lattice walk (which does not use the block summary) for these arguments
+// whether these arguments (but `lattice`) are better taken by the lattice walk, which does not use the block summary
 bool march_takes_lattice(const MarchArgs& a);
 // per-ray slots (ray r's counts[r] samples at slots + r * stride) -> the compacted order (offsets), with ray ids
 // (gate: as MarchArgs::gate)

@@ -944,7 +944,7 @@ bool march_takes_lattice(const MarchArgs& a) {
 
 hipError_t launch_march(const MarchArgs& a, bool emit, hipStream_t st) {
   if (a.num_rays == 0) return hipSuccess;
-  if (march_takes_lattice(a)) {
+  if (a.lattice) {
     // rays a wavefront sets up at once: as many as leave 8192 wavefronts (8 per SIMD), at least 4
     uint32_t rpw = 64;
     while (rpw > 4 && (a.num_rays + rpw - 1) / rpw < 8192u) rpw >>= 1;
