@@ -158,8 +158,26 @@ bool march_slots_fit(const Scratch& held, size_t need) {
 // encode: 2^16 points 138 without, 129 up to 58^3, 151 up to 111^3; 2^18 475, 423, 401).  Below 2^16 samples none:
 // the fill's launch costs more (512 rays x 64: step 219 us with all, 201 without).  FFN_DENSE_MAX_CELLS sets the
 // number of vertices alone.
+size_t level_bytes(const ffn::DevCfg& c, int l) {
+  return ((size_t)c.mask[l] + 1) * (size_t)c.F * (c.table_f16 ? 2 : 4);
+}
+
+constexpr size_t XCD_L2_BYTES = (size_t)4 << 20;
+
+bool level_is_dense(const ffn::DevCfg& c, int l, int64_t n) {
+  const long long R = c.res[l], T = (long long)c.mask[l] + 1;
+  long long max_cells = 1ll << 21;
+  if (const char* env = getenv("FFN_DENSE_MAX_CELLS")) {
+    max_cells = atoll(env);
+  } else {
+    const double worth = n < (1 << 16) ? 0.0 : (level_bytes(c, l) <= XCD_L2_BYTES ? 0.6 : 4.0) * (double)n;
+    if (worth < (double)max_cells) max_cells = (long long)worth;
+    if (16 * T < max_cells) max_cells = 16 * T;
+  }
+  return R >= 2 && R * R * R <= max_cells;
+}
+
 hipError_t build_dense_levels(Handle* h, const void* table, int64_t n, ffn::DenseLevels* dl, hipStream_t st) {
-  const char* env = getenv("FFN_DENSE_MAX_CELLS");
   const ffn::DevCfg& c = h->dc;
   const size_t elem = c.table_f16 ? 2 : 4;
   uint64_t total = 0;
@@ -168,17 +186,8 @@ hipError_t build_dense_levels(Handle* h, const void* table, int64_t n, ffn::Dens
   dl->bricked = 0u;
   bool leading = true;
   for (int l = 0; l < c.L; ++l) {
-    const long long R = c.res[l], T = (long long)c.mask[l] + 1;
-    long long max_cells = 1ll << 21;
-    if (env) {
-      max_cells = atoll(env);
-    } else {
-      const bool in_l2 = (size_t)T * (size_t)c.F * elem <= ((size_t)4 << 20);
-      const double worth = n < (1 << 16) ? 0.0 : (in_l2 ? 0.6 : 4.0) * (double)n;
-      if (worth < (double)max_cells) max_cells = (long long)worth;
-      if (16 * T < max_cells) max_cells = 16 * T;
-    }
-    if (R >= 2 && R * R * R <= max_cells) {
+    const long long R = c.res[l];
+    if (level_is_dense(c, l, n)) {
       // copies of at most 2 MiB are row-major and the leading ones share one gather pass
       // (FFN_DENSE_MULTI=0: none); larger copies are bricked (4x4x4 vertices, the grid padded to whole bricks)
       const bool small = (size_t)(R * R * R) * (size_t)c.F * elem <= ((size_t)2 << 20);
@@ -238,22 +247,40 @@ bool capturing(hipStream_t st) {
   return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
-// Whether ffn_hash_encode_fwd gathers in a spatial order of its points: the sort and the rows written through its
-// permutation cost about 65 us and 0.07 ns a point, and the gather wins the more, the further the tables lie from
-// the L2 and the closer the points.  us, plain / ordered, uniform points; points on a shell:
-//   16 x 2^22 entries (32 MiB a level): 2^18 417 / 457; 375 / 352    2^20 1475 / 1363; 1355 / 907
-//                                       2^22 5711 / 4440; 5208 / 2580  2^24 22020 / 14395; 20858 / 7685
-//   16 x 2^19 entries (4 MiB): 2^20 579 / 597; 552 / 479    2^22 2172 / 1892; 2015 / 1440
-//    8 x 2^14 entries: 2^20 216 / 255; 201 / 206    2^22 794 / 715; 742 / 593
+// Whether ffn_hash_encode_fwd gathers in a spatial order of its points: where that gains more, summed over the levels,
+// than the sort and the rows written through its permutation cost (40 us and 0.083 ns a point).  What a level gains is
+// measured on uniform points, the case where it gains least, with q = points per cell of the level:
+//   * per point 0.16 ns times the share of its table beyond an XCD's 4 MiB L2, at least 0.02, times q / (q + 0.3) (one
+//     level of 2^22 entries, 32 MiB, 2^22 points: q 1.15 0.104 ns, 0.43 0.086, 0.063 0.024, 0.009 0.005);
+//   * 0.013 ns a point for a level with a dense copy (16^3 .. 111^3 vertices: 0.003 to 0.03).
+// us, plain / ordered, uniform points; points on a shell (F = 2; the finest L of 16 levels from 16 to 2048):
+//   entries          L = 1              L = 2              L = 4              L = 8                 L = 16
+//   2^22, 2^20 pts   149/276; 147/259   288/411; 283/389   554/682; 554/605   1092/1162; 1057/774   1434/1323; 1318/888
+//   2^22, 2^22       559/902; 559/810   1097/1444; ..      2173/2493; ..      4315/3944; 4189/2223  5547/4311; 5090/2565
+//   2^22, 2^24       2200/3620; ..      4342/5649; ..      8624/9841; ..      17201/13146; ..       21977/14385; ..
+//   2^20, 2^22       328/675; 328/606   635/981; 635/859   1255/1581; ..      2487/2474; 2415/1546  3476/2797; 3152/1833
+//   2^19, 2^20       52/180; 52/165     95/223; 94/208     178/306; 177/285   344/466; 343/384      572/591; 546/477
+//   2^19, 2^22       180/536; 184/474   344/688; ..        668/1006; ..       1330/1582; 1328/1161  2166/1885; 2009/1430
+//   2^14, 2^22       134/488; 139/429   253/594; ..        475/810; ..        941/1190; 946/913     1664/1460; 1610/1160
+// The rule orders all of these where uniform points gain and none where they lose; points that lie closer gain more.
+// Below 2^20 points none is ordered (16 x 2^22 entries, 2^18: 417/457; 375/352).
 // The scatter gains nothing reliable (2^22 points, 16 x 2^22: 3837 / 3882; 4187 / 3749; 16 x 2^19 2713 / 2925): the
 // merged pairs leave runs of one or two pairs a bucket, which are padded to eight.  FFN_ORDER=0: never, 1: always.
 bool order_pays(const Handle* h, int64_t n, hipStream_t st) {
   if (n >= ((int64_t)1 << 31)) return false;
   if (const char* e = getenv("FFN_ORDER")) return atoi(e) != 0;
-  uint32_t T = 0;
-  for (int l = 0; l < h->dc.L; ++l) T = h->dc.mask[l] + 1 > T ? h->dc.mask[l] + 1 : T;
-  const bool in_l2 = (size_t)T * (size_t)h->dc.F * (h->dc.table_f16 ? 2 : 4) <= ((size_t)4 << 20);
-  if (n < ((int64_t)1 << (in_l2 ? 22 : 20))) return false;
+  if (n < ((int64_t)1 << 20)) return false;
+  double gain = 0.0;  // ns a point
+  for (int l = 0; l < h->dc.L; ++l) {
+    if (level_is_dense(h->dc, l, n)) {
+      gain += 0.013;
+      continue;
+    }
+    const double R = h->dc.res[l], q = (double)n / (R * R * R);
+    const double far = 0.16 * (1.0 - (double)XCD_L2_BYTES / (double)level_bytes(h->dc, l));
+    gain += (far > 0.02 ? far : 0.02) * q / (q + 0.3);
+  }
+  if (gain * (double)n <= 40e3 + 0.083 * (double)n) return false;
   // 36 bytes a point of scratch: the plain order where the device is short of memory
   const size_t need = (size_t)n * (2 * sizeof(uint2) + sizeof(float4) + sizeof(uint32_t));
   const bool held = h->order_pairs.bytes >= 2 * sizeof(uint2) * (size_t)n &&

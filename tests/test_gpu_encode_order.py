@@ -92,3 +92,33 @@ def test_graph_outlives_larger_calls(monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), encode(m, x, 4).view(np.uint32))
+
+
+# The rule weighs what the levels gain: few large levels among none, or large levels so fine that no cell holds two
+# points, keep the plain order; all 16 do not.  Seen by the order's scratch (36 bytes a point).
+@pytest.mark.parametrize("log2_T,first,n,ordered", [([20, 20], 14, 1 << 20, False), ([22], 15, 1 << 20, False),
+                                                    ([22] * 4, 12, 1 << 20, False), ([14] * 15 + [22], 0, 1 << 20, False),
+                                                    ([22] * 16, 0, (1 << 20) - 1, False), ([22] * 16, 0, 1 << 20, True),
+                                                    ([19] * 8, 8, 1 << 22, False), ([19] * 16, 0, 1 << 22, True)])
+def test_rule_weighs_the_levels(monkeypatch, log2_T, first, n, ordered):
+    import torch
+    from gpu_helpers import GpuModel
+    res = [float(np.rint(16.0 * 128.0 ** (l / 15))) for l in range(16)][first:first + len(log2_T)]
+    spec = spec_cfg0(n_levels=len(log2_T), f_per_level=2, log2_T=log2_T, res=res)
+    p = random_params(spec_cfg0(n_levels=len(log2_T), log2_T=[4] * len(log2_T), res=res), seed=4)
+    for k in ("table", "m_table", "v_table"):
+        p[k] = np.zeros(2 * sum(1 << t for t in log2_T), np.float32)
+    x = torch.rand((n, 3), device="cuda")
+    out = torch.empty((n, 2 * len(log2_T)), device="cuda")
+    held = []
+    for env in ("0", None):
+        monkeypatch.setenv("FFN_ORDER", env) if env else monkeypatch.delenv("FFN_ORDER")
+        m = GpuModel(spec, p)
+        import ffn_lib as fl
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        print(f"[encode order] rule levels={len(log2_T)} n={n} order={env}", flush=True)
+        fl.check(m.lib.ffn_hash_encode_fwd(m.h.h, fl.ptr(x), n, fl.ptr(out), None, fl.stream_ptr()), "encode")
+        torch.cuda.synchronize()
+        held.append(before - torch.cuda.mem_get_info()[0])
+    assert (held[1] - held[0] > 30 * n) == ordered
