@@ -947,9 +947,15 @@ int check_march(Handle* h, const void* rays, const uint32_t* bits, const ffn_mar
   return 0;
 }
 
-// samples per ray a marched step's or render's scatter and dense copies are planned for (the ball scene of the
-// benchmark marches 22, its shell field 10)
-constexpr int64_t MARCH_TYPICAL_SAMPLES = 16;
+// Samples per ray that a render's dense copies are made for (the ball scene of the benchmark marches 22, its shell
+// field 10; the count is known only round by round, after the copies).
+constexpr int64_t RENDER_TYPICAL_SAMPLES = 16;
+// Samples per ray that a marched step's bucket sizes are chosen for.  They have to follow from the rays alone (a step
+// sized for a capacity must take those of the exactly sized one, see plan_bins), and the two mistakes differ: large
+// buckets for a small batch cost at most 7 us of a step, small ones for a large batch 10 to 17 % of the scatter (43 us
+// for 4000 rays of 200 samples).  At 128 the line lies at 1536 rays: rays of 16 samples above it lose 3 to 6 us, rays
+// of 256 below it at most 20.
+constexpr int64_t SCATTER_TYPICAL_SAMPLES = 128;
 
 ffn::MarchArgs march_args(Handle* h, const void* rays, uint32_t num_rays, const uint32_t* bits,
                           const ffn_march_params* mp) {
@@ -1161,7 +1167,7 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
   {
     StageTimer tm(h, 1, st);
     ffn::DenseLevels dl;
-    FFN_HIP(build_dense_levels(h, P.table, MARCH_TYPICAL_SAMPLES * num_rays, &dl, st));
+    FFN_HIP(build_dense_levels(h, P.table, n, &dl, st));
     FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, P.table, a0, feat, nullptr, &dl, st, n_dev));
   }
   // 3-5. forward MLP, compositing with early termination and the loss, MLP backward.  (With a capacity the
@@ -1251,7 +1257,7 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
     StageTimer tm(h, 3, st);
     ffn::BinPlan plan{};
     ffn::BinScratch bs{};
-    FFN_HIP(ensure_bins(h, n > 0 ? n : 1, MARCH_TYPICAL_SAMPLES * num_rays, &plan, &bs));
+    FFN_HIP(ensure_bins(h, n > 0 ? n : 1, SCATTER_TYPICAL_SAMPLES * num_rays, &plan, &bs));
     ffn::BinApply ap{};
     ap.dst = P.table;
     ap.dst_f16 = h->dc.table_f16;
@@ -1363,7 +1369,7 @@ int ffn_render(void* handle, const void* rays, uint32_t num_rays, const uint32_t
   a1.ray_ids = nullptr;
   const uint32_t rounds = (mp->max_steps + mp->chunk - 1) / mp->chunk;
   ffn::DenseLevels dl;  // the table does not change during the render: one copy serves every round
-  FFN_HIP(build_dense_levels(h, h->params.table, MARCH_TYPICAL_SAMPLES * num_rays, &dl, st));
+  FFN_HIP(build_dense_levels(h, h->params.table, RENDER_TYPICAL_SAMPLES * num_rays, &dl, st));
   // (without waits: the round's count is *total, read on the device; n the capacity)
   const uint32_t* n_dev = no_wait ? total : nullptr;
   for (uint32_t round = 0; round < rounds; ++round) {

@@ -1074,15 +1074,16 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_bud
   // more than 64 buckets.  An emit round's pairs spread over the buckets, and every run costs its two edge
   // sectors twice (the neighbouring buckets' blocks read them too) plus its padding: at the benchmark shape
   // 64 buckets per level measured emit 4.95 and reduce 2.81 ms against 5.12 and 3.19 ms with 128.
-  // Small batches (fewer than 512 rounds; at 625 the large buckets measured emit 257 and reduce 204 us against 283
-  // and 227): the table's update, not the pairs, is most of the reduce's work, so
-  // a level gets up to 256 buckets, of at most 2048 entries (4096 at F = 1) where that many suffice, and several
-  // blocks share a CU.
+  // Small batches: the table's update, not the pairs, is most of the reduce's work, so a level gets up to 256 buckets,
+  // of at most 2048 entries (4096 at F = 1) where that many suffice, and several blocks share a CU.  Scatter in us,
+  // small / large buckets, samples (16 x 2^19 entries at F = 2 with Adam; the reference's tables, F = 4 with SGD):
+  //   32k 93/95; 30/36   64k 110/113; 36/41   128k 142/144; 48/50   256k 211/207; 74/71   400k 311/292; 123/121
+  //   800k 485/442; 216/196   2M 1122/993; 525/466   8M 3790/3234; 2050/1766  (2^14 or 2^21 entries: alike)
   int max_be = c.F == 4 ? 11 : (c.F == 2 ? 12 : 13);
   uint32_t max_T = 0;
   for (int l = 0; l < c.L; ++l) max_T = c.mask[l] + 1 > max_T ? c.mask[l] + 1 : max_T;
   if ((max_T >> max_be) > 64u) ++max_be;
-  const bool small = (n_typical + rs - 1) / rs < 512;
+  const bool small = n_typical < 3 * (1 << 16);
   for (int l = 0; l < c.L; ++l) {
     int lg = max_be;
     if (small) lg = c.F == 1 ? 12 : (c.F == 2 ? 11 : 10);  // 32 KiB

@@ -24,11 +24,13 @@ def scatter(m, x, g, n_tab, shift):
 
 
 # levels from two entries up to more than 256 (512 at F = 4) of the smallest buckets; n around one emit round
-# (1024 samples, 512 at F = 4), around the 512 rounds from which the run table is transposed and large buckets
-# are used, and one point
+# (1024 samples, 512 at F = 4), around the 512 rounds from which the run table is transposed, around the 3 2^16 samples
+# from which large buckets are used, and one point
 @pytest.mark.parametrize("F,log2_T,n", [(1, [1, 5, 13, 21], 1), (1, [1, 5, 13, 21], 1025), (2, [2, 9, 14, 20], 1023),
                                         (2, [2, 9, 14, 20], 33000), (2, [12, 19], 512 * 1024),
-                                        (2, [12, 19], 512 * 1024 + 1), (4, [3, 13, 17, 20], 513),
+                                        (2, [12, 19], 512 * 1024 + 1), (2, [12, 19], 3 * 65536 - 1),
+                                        (2, [12, 19], 3 * 65536), (4, [3, 13, 17, 19], 3 * 65536 - 1),
+                                        (4, [3, 13, 17, 19], 3 * 65536), (4, [3, 13, 17, 20], 513),
                                         (4, [3, 13, 17, 20], 512 * 512 + 7)])
 @pytest.mark.parametrize("table", [0, 1])
 def test_scatter_plans(F, log2_T, n, table):
