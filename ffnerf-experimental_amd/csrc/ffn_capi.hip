@@ -34,31 +34,42 @@ int fail(int code, const char* fmt, ...) {
     if (e_ != hipSuccess) return fail(-3, "%s: %s", #call, hipGetErrorString(e_));        \
   } while (0)
 
-// A buffer that grows with its calls.  Its size is not a function of the call's size alone (the bucket sizes and the
-// dense copies follow the samples a call is planned for), so a smaller call may grow it: once a call of the handle
-// has been captured into a graph, outgrown buffers are kept for the graph's launches until ffn_destroy.
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// whether this thread's running entry point is being captured into a graph (set by UseMark)
+thread_local bool call_captured = false;
+
+// A buffer that grows with its calls.  A captured call's graph keeps using the buffer it was captured with, so growing
+// it retires that buffer (to `outgrown`, freed by ffn_destroy) instead of freeing it: once per capture, the buffers of
+// later eager calls are in no graph.
 struct Scratch {
   void* p = nullptr;
   size_t bytes = 0;
-  std::vector<void*>* outgrown = nullptr;  // set by the handle's first captured call
+  bool in_graph = false;  // a captured call uses p
+  std::vector<void*>* outgrown = nullptr;  // the handle's
   hipError_t ensure(size_t need) {
-    if (need <= bytes) return hipSuccess;
-    if (p && outgrown) {
-      outgrown->push_back(p);
+    if (need > bytes) {
+      if (p && in_graph) {
+        outgrown->push_back(p);
+      } else if (p) {
+        hipError_t e = hipFree(p);
+        if (e != hipSuccess) return e;
+      }
       p = nullptr;
       bytes = 0;
-    }
-    if (p) {
-      hipError_t e = hipFree(p);
+      in_graph = false;
+      hipError_t e = hipMalloc(&p, need);
       if (e != hipSuccess) return e;
-      p = nullptr;
-      bytes = 0;
+      bytes = need;
     }
-    hipError_t e = hipMalloc(&p, need);
-    if (e != hipSuccess) return e;
-    bytes = need;
+    in_graph = in_graph || call_captured;
     return hipSuccess;
   }
+  // what growing the buffer gives back to the device
+  size_t freed() const { return in_graph ? 0 : bytes; }
   void release() {
     if (p) (void)hipFree(p);
     p = nullptr;
@@ -105,7 +116,12 @@ struct Handle {
   Scratch order_counts, order_pairs, order_perm, order_pts;  // the encode entry points' spatial order
   Scratch tile_sched;  // the MLP's tile order: busy flags (bytes), order, busy count
   uint32_t* host_total = nullptr;  // pinned
-  std::vector<void*> outgrown;     // buffers that captured calls may use, replaced by larger ones since
+  std::vector<void*> outgrown;     // buffers that captured calls use, replaced by larger ones since
+
+  Handle() {
+    each_scratch([this](Scratch& sc) { sc.outgrown = &outgrown; });
+  }
+  Handle(const Handle&) = delete;
 
   template <class Fn>
   void each_scratch(Fn&& fn) {
@@ -117,13 +133,13 @@ struct Handle {
   }
 };
 
-// A scratch buffer may grow to `need` bytes when it is no larger than what it already holds plus half of the
+// A scratch buffer may grow to `need` bytes when it is no larger than what its growth frees plus half of the
 // device memory free now, so that other allocations of the process (a second handle, torch's cache) keep room
 bool growth_fits_free(const Scratch& held, size_t need) {
   if (need <= held.bytes) return true;
   size_t fr = 0, tot = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) return true;  // unknown: let the allocation itself decide
-  return need <= held.bytes + fr / 2;
+  return need <= held.freed() + fr / 2;
 }
 
 // Pair-buffer budget of the scatter: FFN_BIN_BUDGET_MB (MiB, clamped to [64, 2^22]) when set, else 32 GiB
@@ -225,7 +241,8 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* pl
   if (!from_env && !growth_fits_free(h->bin_pairs, pair_bytes * (size_t)plan->max_pairs)) {
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) == hipSuccess) {
-      const size_t cap = h->bin_pairs.bytes + fr / 2;
+      size_t cap = h->bin_pairs.freed() + fr / 2;
+      if (cap < h->bin_pairs.bytes) cap = h->bin_pairs.bytes;
       *plan = ffn::plan_bins(h->dc, n, n_typical, cap < ((size_t)64 << 20) ? ((size_t)64 << 20) : cap, h->n_cu);
     }
   }
@@ -240,11 +257,6 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* pl
   s->pairs = (uint4*)h->bin_pairs.p;
   s->cmax = (float*)h->bin_max.p;
   return hipSuccess;
-}
-
-bool capturing(hipStream_t st) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
 // Whether ffn_hash_encode_fwd gathers in a spatial order of its points: where that gains more, summed over the levels,
@@ -266,7 +278,7 @@ bool capturing(hipStream_t st) {
 // Below 2^20 points none is ordered (16 x 2^22 entries, 2^18: 417/457; 375/352).
 // The scatter gains nothing reliable (2^22 points, 16 x 2^22: 3837 / 3882; 4187 / 3749; 16 x 2^19 2713 / 2925): the
 // merged pairs leave runs of one or two pairs a bucket, which are padded to eight.  FFN_ORDER=0: never, 1: always.
-bool order_pays(const Handle* h, int64_t n, hipStream_t st) {
+bool order_pays(const Handle* h, int64_t n) {
   if (n >= ((int64_t)1 << 31)) return false;
   if (const char* e = getenv("FFN_ORDER")) return atoi(e) != 0;
   if (n < ((int64_t)1 << 20)) return false;
@@ -287,7 +299,7 @@ bool order_pays(const Handle* h, int64_t n, hipStream_t st) {
                     h->order_pts.bytes >= sizeof(float4) * (size_t)n &&
                     h->order_perm.bytes >= sizeof(uint32_t) * (size_t)n;
   // (a captured call cannot allocate it either)
-  return held || (!capturing(st) && growth_fits_free(Scratch{}, need));
+  return held || (!call_captured && growth_fits_free(Scratch{}, need));
 }
 
 // the points' Morton order in the handle's scratch: src becomes the ordered points, *perm their indices
@@ -532,10 +544,7 @@ struct StageTimer {
 void note_use(Handle* h, hipStream_t st) {
   // a call captured into a graph runs when the graph is launched, not here: the caller orders those launches
   // before ffn_destroy (no event is recorded into the capture)
-  if (capturing(st)) {
-    h->each_scratch([&](Scratch& sc) { sc.outgrown = &h->outgrown; });
-    return;
-  }
+  if (call_captured) return;
   for (StreamUse& u : h->uses) {
     if (u.st == st) {
       if (hipEventRecord(u.ev, st) != hipSuccess) h->uses_lost = true;
@@ -551,10 +560,12 @@ void note_use(Handle* h, hipStream_t st) {
   if (hipEventRecord(ev, st) != hipSuccess) h->uses_lost = true;
 }
 
-// note_use at the end of an entry point's scope (every return path), after everything it enqueued
+// An entry point's scope, from before its first use of scratch: whether it is captured, and note_use at its end (every
+// return path), after everything it enqueued
 struct UseMark {
   Handle* h;
   hipStream_t st;
+  UseMark(Handle* h_, hipStream_t st_) : h(h_), st(st_) { call_captured = capturing(st); }
   ~UseMark() {
     if (h) note_use(h, st);
   }
@@ -689,7 +700,7 @@ int ffn_hash_encode_fwd(void* handle, const float* x, int64_t n, float* a0, uint
   const ffn::FeatLayout lm = ffn::level_major(n, h->dc.F);
   ffn::PosSrc src{x, nullptr, nullptr, 0};
   const uint32_t* perm = nullptr;  // (corner indices are written in the points' own order)
-  if (!idx_out && order_pays(h, n, st)) FFN_HIP(order_points(h, n, &src, &perm, st));
+  if (!idx_out && order_pays(h, n)) FFN_HIP(order_points(h, n, &src, &perm, st));
   ffn::DenseLevels dl;
   FFN_HIP(build_dense_levels(h, h->params.table, n, &dl, st));
   FFN_HIP(ffn::launch_hash_fwd(h->dc, src, n, h->params.table, (float*)h->a0.p, lm, idx_out, &dl, st));
@@ -731,6 +742,7 @@ static int step_by_march(Handle* h, const void* rays, const void* targets, void*
                          const ffn_step_scalars* sc, const ffn_taps* taps, void* stream) {
   const int G = h->cfg.occ_G, R = 2 * G;
   const size_t words = ((size_t)R * R * R + 31) / 32;
+  call_captured = capturing((hipStream_t)stream);
   FFN_HIP(h->m_bits.ensure(sizeof(uint32_t) * words));
   uint32_t* bits = (uint32_t*)h->m_bits.p;
   FFN_HIP(ffn::launch_occ_bitfield(h->params.occ_in, G, (uint32_t)h->cfg.march_q_min, bits, (hipStream_t)stream));
