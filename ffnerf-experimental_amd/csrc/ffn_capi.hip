@@ -232,26 +232,37 @@ hipError_t build_dense_levels(Handle* h, const void* table, int64_t n, ffn::Dens
   return ffn::launch_hash_densify(c, table, *dl, st);
 }
 
-// size the bucketed-scatter scratch for n samples (n_typical: see plan_bins) and fill the views
-hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, ffn::BinPlan* plan, ffn::BinScratch* s) {
+// Size the bucketed-scatter scratch for n samples (n_typical: see plan_bins) and fill the views.  Small batches' buckets
+// need more of it a sample, so it is sized for a small batch of n_small samples as well, the largest that a later call
+// no larger than this one may be: that call can then be captured into a graph, where nothing can be allocated.
+hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, int64_t n_small, ffn::BinPlan* plan,
+                       ffn::BinScratch* s) {
   bool from_env = false;
-  const size_t budget = bin_budget_bytes(&from_env);
+  size_t budget = bin_budget_bytes(&from_env);
   const size_t pair_bytes = 2 + 4 * (size_t)h->dc.F;
   *plan = ffn::plan_bins(h->dc, n, n_typical, budget, h->n_cu);
   if (!from_env && !growth_fits_free(h->bin_pairs, pair_bytes * (size_t)plan->max_pairs)) {
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) == hipSuccess) {
-      size_t cap = h->bin_pairs.freed() + fr / 2;
-      if (cap < h->bin_pairs.bytes) cap = h->bin_pairs.bytes;
-      *plan = ffn::plan_bins(h->dc, n, n_typical, cap < ((size_t)64 << 20) ? ((size_t)64 << 20) : cap, h->n_cu);
+      budget = h->bin_pairs.freed() + fr / 2;
+      if (budget < h->bin_pairs.bytes) budget = h->bin_pairs.bytes;
+      if (budget < ((size_t)64 << 20)) budget = (size_t)64 << 20;
+      *plan = ffn::plan_bins(h->dc, n, n_typical, budget, h->n_cu);
     }
   }
+  int64_t pairs = plan->max_pairs, meta = plan->meta_elems, meta_t = plan->transpose ? plan->meta_elems : 0;
+  const ffn::BinPlan sm = ffn::plan_bins(h->dc, n_small, 0, budget, h->n_cu);
+  if (growth_fits_free(h->bin_pairs, pair_bytes * (size_t)sm.max_pairs)) {
+    pairs = sm.max_pairs > pairs ? sm.max_pairs : pairs;
+    meta = sm.meta_elems > meta ? sm.meta_elems : meta;
+    if (sm.transpose && sm.meta_elems > meta_t) meta_t = sm.meta_elems;
+  }
   hipError_t e;
-  if ((e = h->bin_meta.ensure(sizeof(uint32_t) * (size_t)plan->meta_elems)) != hipSuccess) return e;
-  if (plan->transpose && (e = h->bin_meta_t.ensure(sizeof(uint32_t) * (size_t)plan->meta_elems)) != hipSuccess)
-    return e;
-  if ((e = h->bin_pairs.ensure((2 + 4 * (size_t)h->dc.F) * (size_t)plan->max_pairs)) != hipSuccess) return e;
-  if ((e = h->bin_max.ensure(sizeof(float) * (size_t)plan->levels_per_group * plan->nblk)) != hipSuccess) return e;
+  if ((e = h->bin_meta.ensure(sizeof(uint32_t) * (size_t)meta)) != hipSuccess) return e;
+  if ((e = h->bin_meta_t.ensure(sizeof(uint32_t) * (size_t)meta_t)) != hipSuccess) return e;
+  if ((e = h->bin_pairs.ensure(pair_bytes * (size_t)pairs)) != hipSuccess) return e;
+  // (a round per block at most, whatever the plan)
+  if ((e = h->bin_max.ensure(sizeof(float) * (size_t)h->dc.L * plan->n_rounds)) != hipSuccess) return e;
   s->meta = (uint32_t*)h->bin_meta.p;
   s->meta_t = (uint32_t*)h->bin_meta_t.p;
   s->pairs = (uint4*)h->bin_pairs.p;
@@ -721,7 +732,7 @@ int ffn_hash_encode_bwd(void* handle, const float* x, const float* g, int64_t n,
   UseMark um{h, (hipStream_t)stream};
   ffn::BinPlan plan;
   ffn::BinScratch bs;
-  FFN_HIP(ensure_bins(h, n, n, &plan, &bs));
+  FFN_HIP(ensure_bins(h, n, n, ffn::small_batch(n), &plan, &bs));
   // the scatter reads one level per pass: the caller's sample-major rows are transposed to level-major
   // first (the passes would otherwise fetch every row once per level for F floats of it)
   const hipStream_t st = (hipStream_t)stream;
@@ -798,7 +809,7 @@ int ffn_train_step(void* handle, const void* rays, const void* targets, void* ou
   }
   ffn::BinPlan plan{};
   ffn::BinScratch bs{};
-  if (train) FFN_HIP(ensure_bins(h, N, N, &plan, &bs));
+  if (train) FFN_HIP(ensure_bins(h, N, N, ffn::small_batch(N), &plan, &bs));
   const ffn::FeatLayout feat = ffn::level_major(N, h->dc.F);
   const ffn::PosSrc src{nullptr, (const float4*)rays, nullptr, log2S};
   float* Ts = (float*)h->Ts.p;
@@ -1269,7 +1280,8 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
     StageTimer tm(h, 3, st);
     ffn::BinPlan plan{};
     ffn::BinScratch bs{};
-    FFN_HIP(ensure_bins(h, n > 0 ? n : 1, SCATTER_TYPICAL_SAMPLES * num_rays, &plan, &bs));
+    const int64_t n1s = n > 0 ? n : 1;  // (fewer rays of the same capacity may be a small batch)
+    FFN_HIP(ensure_bins(h, n1s, SCATTER_TYPICAL_SAMPLES * num_rays, n1s, &plan, &bs));
     ffn::BinApply ap{};
     ap.dst = P.table;
     ap.dst_f16 = h->dc.table_f16;

@@ -1083,7 +1083,7 @@ BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_bud
   uint32_t max_T = 0;
   for (int l = 0; l < c.L; ++l) max_T = c.mask[l] + 1 > max_T ? c.mask[l] + 1 : max_T;
   if ((max_T >> max_be) > 64u) ++max_be;
-  const bool small = n_typical < 3 * (1 << 16);
+  const bool small = n_typical < SCATTER_SMALL_BATCH;
   for (int l = 0; l < c.L; ++l) {
     int lg = max_be;
     if (small) lg = c.F == 1 ? 12 : (c.F == 2 ? 11 : 10);  // 32 KiB

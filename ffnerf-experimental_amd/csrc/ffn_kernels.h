@@ -183,6 +183,9 @@ struct BinApply {
 // enter the fixed-point scale's pair counts, so a step sized for a capacity passes what the exactly sized step
 // would, and both give the same table bit for bit); n_cu: the GPU's compute units
 BinPlan plan_bins(const DevCfg& c, int64_t n, int64_t n_typical, size_t pair_budget_bytes, int n_cu);
+// samples from which large buckets are chosen (plan_bins), and the largest small batch of at most n samples
+constexpr int64_t SCATTER_SMALL_BATCH = 3 * (1 << 16);
+inline int64_t small_batch(int64_t n) { return n < SCATTER_SMALL_BATCH ? n : SCATTER_SMALL_BATCH - 1; }
 // whether the scatter is built for this table shape: a round's stage must fit in a CU's LDS and its run
 // offsets in 16 bits (F = 4 with 2^22-entry levels does not)
 bool scatter_supported(const DevCfg& c);

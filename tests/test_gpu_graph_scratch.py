@@ -77,3 +77,51 @@ def test_later_buffers_are_freed(monkeypatch, captured):
         torch.cuda.synchronize()
         if captured == "encode":
             assert torch.equal(out[:n0], ref)
+
+
+# A step of fewer samples takes the small batches' buckets, which need more scratch a sample than the large ones of the
+# eager step before it; under capture nothing can be allocated.
+@pytest.mark.parametrize("marched", [False, True])
+def test_smaller_step_is_captured(marched):
+    import ctypes as C
+    import ffn_lib as fl
+    import torch
+    from gpu_helpers import GpuModel
+    spec = spec_cfg0(n_levels=8, f_per_level=2, log2_T=[19] * 8, res=[16.0 * 1.6 ** i for i in range(8)])
+    p = random_params(spec, seed=2)
+    n_large, n_small = (3000, 1000) if marched else (4800, 2900)
+    rays = torch.from_numpy(look_at_rays(n_large, spec, seed=3)).cuda()
+    tg, out = torch.rand((n_large, 4), device="cuda"), torch.zeros((n_large, 4), device="cuda")
+    bits = torch.full((32 ** 3 // 32,), -1, dtype=torch.int32, device="cuda")
+    mp = fl.march_params(32, np.float32(1.0 / 100), 200, T_stop=1e-3, sample_capacity=200000)
+    d = default_scalars()
+    sc = fl.FfnStepScalars()
+    for k in ("lr", "lr_t", "color_rel_lr", "sh_multiplier", "occ_strength", "beta1", "beta2", "eps"):
+        setattr(sc, k, float(d[k]))
+    sc.rng_seed, sc.do_train = 5, 1
+
+    def step(m, n):
+        if marched:
+            rc = m.lib.ffn_train_step_marched(m.h.h, fl.ptr(rays), fl.ptr(tg), fl.ptr(out), n, fl.ptr(bits),
+                                              C.byref(mp), C.byref(sc), None, None, fl.stream_ptr())
+        else:
+            rc = m.lib.ffn_train_step(m.h.h, fl.ptr(rays), fl.ptr(tg), fl.ptr(out), n, 64, C.byref(sc), None,
+                                      fl.stream_ptr())
+        fl.check(rc, "step")
+
+    print(f"[graph scratch] smaller step marched={marched}", flush=True)
+    m, ref = GpuModel(spec, p), GpuModel(spec, p)
+    step(m, n_large)
+    step(ref, n_large)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        step(m, n_small)
+    for _ in range(3):
+        graph.replay()
+        step(ref, n_small)
+        torch.cuda.synchronize()
+        a, b = m.state(), ref.state()
+        for k in a:
+            np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32), err_msg=k)
