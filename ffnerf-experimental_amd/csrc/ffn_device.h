@@ -19,6 +19,22 @@
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// K-ordered rows of the K = 32 matrix instructions: position p = 32 kb + 8 g + j (slot j of lane group g in block kb)
+// holds the neuron that the lanes' results of the layer before put there, and back; four consecutive neurons from a
+// multiple of four on have consecutive positions
+__host__ __device__ constexpr int kpos_neuron(int p) {
+  return (p & ~31) + 16 * ((p >> 2) & 1) + 4 * ((p >> 3) & 3) + (p & 3);
+}
+__host__ __device__ constexpr int neuron_kpos(int n) {
+  return (n & ~31) + 8 * ((n >> 2) & 3) + 4 * ((n >> 4) & 1) + (n & 3);
+}
+constexpr bool kpos_inverse() {
+  for (int n = 0; n < 64; ++n)
+    if (kpos_neuron(neuron_kpos(n)) != n || neuron_kpos(n & ~3) + (n & 3) != neuron_kpos(n)) return false;
+  return true;
+}
+static_assert(kpos_inverse());
+
 namespace ffn {
 
 // Everything a kernel needs from ffn_config, flattened into a kernel argument.

@@ -59,19 +59,6 @@ __device__ __forceinline__ floatx4 mfma_k32b(const bf16x8& a, const bf16x8& b, c
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// neuron of K slot j of lane group g in K block kb (see the file comment)
-__host__ __device__ constexpr int kslot_neuron(int kb, int g, int j) {
-  return 32 * kb + 16 * (j >> 2) + 4 * g + (j & 3);
-}
-// the same for the position p = 32 kb + 8 g + j of a K-ordered row
-__host__ __device__ constexpr int kpos_neuron(int p) { return kslot_neuron(p >> 5, (p >> 3) & 3, p & 7); }
-
-// the position of neuron n in a K-ordered row (kpos_neuron's inverse); four consecutive neurons from a multiple of
-// four on have consecutive positions
-__host__ __device__ constexpr int neuron_kpos(int n) {
-  return (n & ~31) + 8 * ((n >> 2) & 3) + 4 * ((n >> 4) & 1) + (n & 3);
-}
-
 __device__ __forceinline__ half4 to_half4(const floatx4& v) {
   half4 h;
 #pragma unroll

@@ -76,7 +76,7 @@ __device__ __forceinline__ constexpr int row_pos(int n) {
     const int g = n / KA, kk = n % KA;
     return 32 * (kk / 8) + 8 * g + kk % 8;
   } else {
-    return (n & ~31) + 8 * ((n >> 2) & 3) + 4 * ((n >> 4) & 1) + (n & 3);
+    return neuron_kpos(n);
   }
 }
 

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(64) void k_probe_layer(const float* __restrict__ x,
   for (int e = lane; e < 64 * K / 4; e += 64) {
     const int o = e / (K / 4), i = 4 * (e % (K / 4));
     const float w[4] = {W[o * K + i], W[o * K + i + 1], W[o * K + i + 2], W[o * K + i + 3]};
-    put_split4(sW + o * P + (i & ~31) + 8 * ((i >> 2) & 3) + 4 * ((i >> 4) & 1), PLANE, w);
+    put_split4(sW + o * P + neuron_kpos(i), PLANE, w);
   }
   sB[lane] = B[lane];
   __syncthreads();
@@ -52,7 +52,8 @@ __global__ __launch_bounds__(64) void k_probe_layer(const float* __restrict__ x,
   }
 }
 
-// x [n][32 kb], W [64][32 kb], B [64] -> out [n][64], device arrays.  Returns 0, or 1 for bad arguments or a launch error.
+// x [n][32 kb], W [64][32 kb], B [64] -> out [n][64], device arrays.  Returns 0, or 1 for bad arguments or a launch
+// error.
 extern "C" int ffn_probe_layer(int kb, int split, const float* x, const float* W, const float* B, float* out, int n) {
   if (kb < 1 || kb > 2 || n < 1) return 1;
   const dim3 grid((n + 15) / 16), block(64);
