@@ -288,22 +288,26 @@ hipError_t ensure_bins(Handle* h, int64_t n, int64_t n_typical, int64_t n_small,
 // The rule orders all of these where uniform points gain and none where they lose; points that lie closer gain more.
 // Below 2^20 points none is ordered (16 x 2^22 entries, 2^18: 417/457; 375/352).
 // The scatter gains nothing reliable (2^22 points, 16 x 2^22: 3837 / 3882; 4187 / 3749; 16 x 2^19 2713 / 2925): the
-// merged pairs leave runs of one or two pairs a bucket, which are padded to eight.  FFN_ORDER=0: never, 1: always.
+// merged pairs leave runs of one or two pairs a bucket, which are padded to eight.  FFN_ORDER=0: never, 1: wherever
+// there is room for it.
 bool order_pays(const Handle* h, int64_t n) {
   if (n >= ((int64_t)1 << 31)) return false;
-  if (const char* e = getenv("FFN_ORDER")) return atoi(e) != 0;
-  if (n < ((int64_t)1 << 20)) return false;
-  double gain = 0.0;  // ns a point
-  for (int l = 0; l < h->dc.L; ++l) {
-    if (level_is_dense(h->dc, l, n)) {
-      gain += 0.013;
-      continue;
+  if (const char* e = getenv("FFN_ORDER")) {
+    if (atoi(e) == 0) return false;
+  } else {
+    if (n < ((int64_t)1 << 20)) return false;
+    double gain = 0.0;  // ns a point
+    for (int l = 0; l < h->dc.L; ++l) {
+      if (level_is_dense(h->dc, l, n)) {
+        gain += 0.013;
+        continue;
+      }
+      const double R = h->dc.res[l], q = (double)n / (R * R * R);
+      const double far = 0.16 * (1.0 - (double)XCD_L2_BYTES / (double)level_bytes(h->dc, l));
+      gain += (far > 0.02 ? far : 0.02) * q / (q + 0.3);
     }
-    const double R = h->dc.res[l], q = (double)n / (R * R * R);
-    const double far = 0.16 * (1.0 - (double)XCD_L2_BYTES / (double)level_bytes(h->dc, l));
-    gain += (far > 0.02 ? far : 0.02) * q / (q + 0.3);
+    if (gain * (double)n <= 40e3 + 0.083 * (double)n) return false;
   }
-  if (gain * (double)n <= 40e3 + 0.083 * (double)n) return false;
   // 36 bytes a point of scratch: the plain order where the device is short of memory
   const size_t need = (size_t)n * (2 * sizeof(uint2) + sizeof(float4) + sizeof(uint32_t));
   const bool held = h->order_pairs.bytes >= 2 * sizeof(uint2) * (size_t)n &&

@@ -125,3 +125,24 @@ def test_smaller_step_is_captured(marched):
         a, b = m.state(), ref.state()
         for k in a:
             np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32), err_msg=k)
+
+
+# asked for the spatial order, a captured encode takes the plain one if no eager call has sized the order's scratch
+def test_order_is_not_allocated_under_capture(monkeypatch):
+    import torch
+    m = model()
+    n = 70000
+    x, out, ref = torch.rand((n, 3), device="cuda"), torch.zeros((n, 32), device="cuda"), torch.zeros((n, 32), device="cuda")
+    print("[graph scratch] order under capture", flush=True)
+    monkeypatch.setenv("FFN_ORDER", "0")
+    encode(m, x, ref, n)
+    torch.cuda.synchronize()
+    monkeypatch.setenv("FFN_ORDER", "1")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        encode(m, x, out, n)
+    for _ in range(2):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
