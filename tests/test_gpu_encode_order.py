@@ -108,17 +108,20 @@ def test_rule_weighs_the_levels(monkeypatch, log2_T, first, n, ordered):
     p = random_params(spec_cfg0(n_levels=len(log2_T), log2_T=[4] * len(log2_T), res=res), seed=4)
     for k in ("table", "m_table", "v_table"):
         p[k] = np.zeros(2 * sum(1 << t for t in log2_T), np.float32)
+    p["table"] = np.resize(np.random.default_rng(n).random(999983, dtype=np.float32), p["table"].size)
     x = torch.rand((n, 3), device="cuda")
-    out = torch.empty((n, 2 * len(log2_T)), device="cuda")
-    held = []
+    held, outs = [], []
     for env in ("0", None):
         monkeypatch.setenv("FFN_ORDER", env) if env else monkeypatch.delenv("FFN_ORDER")
         m = GpuModel(spec, p)
         import ffn_lib as fl
         torch.cuda.synchronize()
+        out = torch.zeros((n, 2 * len(log2_T)), device="cuda")
         before = torch.cuda.mem_get_info()[0]
         print(f"[encode order] rule levels={len(log2_T)} n={n} order={env}", flush=True)
         fl.check(m.lib.ffn_hash_encode_fwd(m.h.h, fl.ptr(x), n, fl.ptr(out), None, fl.stream_ptr()), "encode")
         torch.cuda.synchronize()
         held.append(before - torch.cuda.mem_get_info()[0])
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
     assert (held[1] - held[0] > 30 * n) == ordered
