@@ -1284,8 +1284,9 @@ int ffn_train_step_marched(void* handle, const void* rays, const void* targets, 
     StageTimer tm(h, 3, st);
     ffn::BinPlan plan{};
     ffn::BinScratch bs{};
-    const int64_t n1s = n > 0 ? n : 1;  // (fewer rays of the same capacity may be a small batch)
-    FFN_HIP(ensure_bins(h, n1s, SCATTER_TYPICAL_SAMPLES * num_rays, n1s, &plan, &bs));
+    // (fewer rays of the same capacity may be a small batch; a step that waits cannot be captured)
+    const int64_t nb = n > 0 ? n : 1;
+    FFN_HIP(ensure_bins(h, nb, SCATTER_TYPICAL_SAMPLES * num_rays, cap > 0 ? nb : 1, &plan, &bs));
     ffn::BinApply ap{};
     ap.dst = P.table;
     ap.dst_f16 = h->dc.table_f16;
