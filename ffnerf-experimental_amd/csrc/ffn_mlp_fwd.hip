@@ -222,8 +222,9 @@ __device__ __noinline__ float4 fwd_samples_fp32(const MlpPtrs* __restrict__ wp, 
 // the ReLU tap).  Returns the samples (bit per sample) whose sums are not finite, to be done again by fwd_samples_fp32.
 template <int LF, int ND, int NC>
 __device__ __forceinline__ uint32_t fwd_samples_split(const float* __restrict__ sm, const float (&a0r)[LF / 4],
-                                            const float (&dirv)[3], float sh_mult, int g, int s, floatx4 (&hd)[ND][4],
-                                            floatx4 (&hc)[NC][4], float& dout0, float (&rgb)[3]) {
+                                                      const float (&dirv)[3], float sh_mult, int g, int s,
+                                                      floatx4 (&hd)[ND][4], floatx4 (&hc)[NC][4], float& dout0,
+                                                      float (&rgb)[3]) {
   using A = ArchF<LF, ND, NC>;
   constexpr int PL = A::plane(), KB0 = A::cols(FFN_WD_IN) / 32;
   // an offset of zero that the compiler cannot see through: it would read the weights before the caller's loop and
